@@ -415,16 +415,18 @@ int lekf_event_sync(void *ev);
 #define LEKF_TUNE_GRAM_WAVES 0 /* waves per point of the k > 32 Gram kernel: 2, 4 or 8 */
 #define LEKF_TUNE_GRAM_WS_MB 1 /* Gram workspace per launch, MiB, 16 .. 65536 (16384) */
 #define LEKF_TUNE_SEL_PER_CU 2 /* capped-selection workgroups per CU: 1 .. 4 */
-#define LEKF_TUNE_EIG_SPLIT 3  /* 32 < k <= 64: 1 = tridiagonalisation, QL (one lane per point)
-                                  and apply kernels (the apply pushes the state rows through
-                                  Q and the recorded rotations instead of forming the
-                                  eigenvectors, unless trans or pao is asked for), 0 = one
-                                  fused eigen kernel; the two agree to rounding */
-#define LEKF_TUNE_SPLIT_RCAP 4 /* rotations a point's QL stream may hold in the three-kernel
-                                  eigensolver; a point whose stream is longer is solved by
-                                  the fused kernel's steps instead; 0: the default 2k^2 + 8k
-                                  (smaller values test that fallback) */
-#define LEKF_TUNE_MIXED_KAPPA 5 /* split-BF16x3 and FP32 forms on the three-kernel eigensolver
+#define LEKF_TUNE_EIG_SPLIT 3  /* 32 < k <= 95: 1 = jobs without trans and pao by a tridiagonal
+                                  form and a rational function of it (no eigenvalues), jobs
+                                  with them, up to k = 64, by tridiagonalisation, QL (one lane
+                                  per point) and replay kernels; 0 = one fused eigen kernel;
+                                  all agree to rounding */
+#define LEKF_TUNE_SPLIT_RCAP 4 /* rotations a point's QL stream may hold in the solve with
+                                  recorded rotations; a point whose stream is longer is solved
+                                  by the fused kernel's steps instead.  0: the default
+                                  2k^2 + 8k; a value above 0 (k <= 64) also sends the jobs
+                                  without trans and pao through the recorded rotations (smaller
+                                  values test that fallback) */
+#define LEKF_TUNE_MIXED_KAPPA 5 /* split-BF16x3 and FP32 forms under LEKF_TUNE_EIG_SPLIT = 1
                                    (32 < k <= 64): a point whose C + (k-1)/alpha I has condition
                                    number above this value (16 times it for FP32) is solved
                                    again from an FP64 Gram (status bit LEKF_PT_FP64);

@@ -195,18 +195,21 @@ void* scratch_ptr()
 }
 
 // One solve launch; ws is grown to the Gram workspace the class needs.
-int run_solve(const lekf_job* djobs, int njobs, long npt, int kmax, int nvmax, int mode,
+int run_solve(const lekf_job* djobs, int njobs, long npt, int kmax, int nvmax, int mode, int outs,
               DevBuf& ws, hipStream_t st)
 {
-    const size_t need = lekf_solve_ws_bytes(npt, kmax);
+    const size_t need = lekf_solve_ws_bytes(npt, kmax, outs);
     if (need) HIPCHK(ws.ensure(need));
-    HIPCHK(lekf_solve_launch(djobs, njobs, npt, kmax, nvmax, mode, need ? ws.p : nullptr,
+    HIPCHK(lekf_solve_launch(djobs, njobs, npt, kmax, nvmax, mode, outs, need ? ws.p : nullptr,
                              need ? ws.n : 0, st));
     return 0;
 }
 
 // state rows a job's points apply their transform to (0 without the apply)
 int job_rows(const lekf_job& j) { return (j.flags & LEKF_F_APPLY) ? j.nv3d + j.nv2d : 0; }
+
+// whether a job asks for the k x k outputs
+int job_outs(const lekf_job& j) { return j.trans || j.pao ? LEKF_OUT_TRANS : LEKF_OUT_PLAIN; }
 
 // The grouped launches of launch_grouped over caller-provided device memory:
 // descriptors at dj (room for J.size()), workspace ws of ws_bytes.  Nothing is
@@ -222,25 +225,27 @@ int launch_grouped_fixed(std::vector<lekf_job> J, int mode, lekf_job* dj, void* 
         if (i == 0 || lekf_solve_class(J[i].k) != lekf_solve_class(J[i - 1].k)) starts.push_back(i);
     starts.push_back(J.size());
     std::vector<long> tot(starts.size(), 0);
-    std::vector<int> kmax(starts.size(), 0), nvmax(starts.size(), 0);
+    std::vector<int> kmax(starts.size(), 0), nvmax(starts.size(), 0), outs(starts.size(), 0);
     for (size_t g = 0; g + 1 < starts.size(); ++g)
         for (size_t i = starts[g]; i < starts[g + 1]; ++i) {
             J[i].pt_begin = tot[g];
             tot[g] += J[i].npt;
             kmax[g] = std::max(kmax[g], J[i].k);
             nvmax[g] = std::max(nvmax[g], job_rows(J[i]));
+            outs[g] |= job_outs(J[i]);
         }
     for (size_t g = 0; g + 1 < starts.size(); ++g)
-        if (tot[g] > 0 && lekf_solve_ws_bytes(1, kmax[g]) > ws_bytes) {
+        if (tot[g] > 0 && lekf_solve_ws_bytes(1, kmax[g], outs[g]) > ws_bytes) {
             snprintf(g_errmsg, sizeof(g_errmsg),
                      "lekf_core_batch_noalloc: a point record of k = %d needs %zu bytes, the "
-                     "workspace holds %zu", kmax[g], lekf_solve_ws_bytes(1, kmax[g]), ws_bytes);
+                     "workspace holds %zu",
+                     kmax[g], lekf_solve_ws_bytes(1, kmax[g], outs[g]), ws_bytes);
             return LEKF_ERR_SIZE;
         }
     HIPCHK(hipMemcpyAsync(dj, J.data(), sizeof(lekf_job) * J.size(), hipMemcpyHostToDevice, st));
     for (size_t g = 0; g + 1 < starts.size(); ++g)
         HIPCHK(lekf_solve_launch(dj + starts[g], (int)(starts[g + 1] - starts[g]), tot[g], kmax[g],
-                                 nvmax[g], mode, kmax[g] > 32 ? ws : nullptr,
+                                 nvmax[g], mode, outs[g], kmax[g] > 32 ? ws : nullptr,
                                  kmax[g] > 32 ? ws_bytes : 0, st));
     return 0;
 }
@@ -259,18 +264,19 @@ int launch_grouped(std::vector<lekf_job> J, int mode, DevBuf& db, DevBuf& ws, hi
         if (i == 0 || lekf_solve_class(J[i].k) != lekf_solve_class(J[i - 1].k)) starts.push_back(i);
     starts.push_back(J.size());
     std::vector<long> tot(starts.size(), 0);
-    std::vector<int> kmax(starts.size(), 0), nvmax(starts.size(), 0);
+    std::vector<int> kmax(starts.size(), 0), nvmax(starts.size(), 0), outs(starts.size(), 0);
     for (size_t g = 0; g + 1 < starts.size(); ++g)
         for (size_t i = starts[g]; i < starts[g + 1]; ++i) {
             J[i].pt_begin = tot[g];
             tot[g] += J[i].npt;
             kmax[g] = std::max(kmax[g], J[i].k);
             nvmax[g] = std::max(nvmax[g], job_rows(J[i]));
+            outs[g] |= job_outs(J[i]);
         }
     HIPCHK(hipMemcpyAsync(db.p, J.data(), sizeof(lekf_job) * J.size(), hipMemcpyHostToDevice, st));
     for (size_t g = 0; g + 1 < starts.size(); ++g) {
         const int rc = run_solve(db.as<lekf_job>() + starts[g], (int)(starts[g + 1] - starts[g]),
-                                 tot[g], kmax[g], nvmax[g], mode, ws, st);
+                                 tot[g], kmax[g], nvmax[g], mode, outs[g], ws, st);
         if (rc) return rc;
     }
     return 0;
@@ -552,7 +558,7 @@ int lekf_mem_info(size_t* free_bytes, size_t* total_bytes)
 long lekf_solve_workspace_bytes(long npt, int k)
 {
     if (npt <= 0 || k < 2 || k > LEKF_KMAX) return 0;
-    return (long)lekf_solve_ws_bytes(npt, k);
+    return (long)lekf_solve_ws_bytes(npt, k, LEKF_OUT_PLAIN);
 }
 
 int lekf_core_f64(int ne, int nobs, int nobsl, const double* hdxb, const double* rdiag,
@@ -613,7 +619,7 @@ int lekf_core_f64(int ne, int nobs, int nobsl, const double* hdxb, const double*
     J.pao = pao ? c.pa.as<double>() : nullptr;
     J.status = c.stat.as<int>();
     HIPCHK(hipMemcpyAsync(c.job.p, &J, sizeof(J), hipMemcpyHostToDevice, st));
-    rc = run_solve(c.job.as<lekf_job>(), 1, 1, ne, 0, 0, c.gws, st);
+    rc = run_solve(c.job.as<lekf_job>(), 1, 1, ne, 0, 0, LEKF_OUT_TRANS, c.gws, st);
     if (rc) return rc;
     int pst = 0;
     HIPCHK(hipMemcpyAsync(trans, c.tr.p, sizeof(double) * k * k, hipMemcpyDeviceToHost, st));
@@ -1760,7 +1766,7 @@ int lekf_das_solve(lekf_handle* h)
         npt = h->chunk_pts[1];
     }
     const int rc = run_solve(h->djob.as<lekf_job>(), 1, npt, h->ne, job_rows(h->job),
-                             mode_of_prec(h->prec), h->gws, h->st);
+                             mode_of_prec(h->prec), job_outs(h->job), h->gws, h->st);
     if (rc) return rc;
     return run_relax(h);
 }
@@ -1773,7 +1779,8 @@ int das_run_eager(lekf_handle* h)
             int rc = reg_select_chunk(h, (int)c);
             if (rc) return rc;
             rc = run_solve(h->djob.as<lekf_job>() + c, 1, h->chunk_pts[c + 1] - h->chunk_pts[c],
-                           h->ne, job_rows(h->job), mode_of_prec(h->prec), h->gws, h->st);
+                           h->ne, job_rows(h->job), mode_of_prec(h->prec), job_outs(h->job), h->gws,
+                           h->st);
             if (rc) return rc;
         }
         return run_relax(h);

@@ -59,6 +59,30 @@ __device__ __forceinline__ double rn_div(double a, double b)
     return a / b;
 }
 
+// what the jobs of a solve launch ask for: any without trans and pao, any with
+#define LEKF_OUT_PLAIN 1
+#define LEKF_OUT_TRANS 2
+
+// Reciprocal and reciprocal square root: hardware estimate refined by Newton
+// steps to full FP64 accuracy (a Jacobi rotation only needs c^2 + s^2 = 1 to
+// rounding, which an accurate c = (1+t^2)^-1/2 and s = t c give).
+__device__ __forceinline__ double rcp_nr(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return r;
+}
+
+__device__ __forceinline__ double rsq_nr(double x)
+{
+    double r = __builtin_amdgcn_rsq(x);
+    const double h = 0.5 * x;
+    r = r * fma(-h * r, r, 1.5);
+    r = r * fma(-h * r, r, 1.5);
+    return r;
+}
+
 // Jacobi: rotate a pair while |a_pq| > tol * sqrt(a_pp a_qq); stop after a
 // sweep with no rotation.
 #define LEKF_JACOBI_TOL 1.0e-15

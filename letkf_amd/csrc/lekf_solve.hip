@@ -19,29 +19,25 @@
 //   * k <= 32: one fused kernel, one wave per point; the eigendecomposition is
 //     a one-sided Jacobi with the matrix in registers.
 //   * 32 < k <= LEKF_KSPLIT: a Gram kernel (2-8 waves per point, MFMA) writes
-//     C, b and the sums to a workspace; a second kernel (one wave per point)
-//     reduces C to tridiagonal form by Householder reflections, diagonalises
-//     it by implicit QL with shifts (the method of EISPACK tred2/tql2, the
-//     reference's own eigensolver), and assembles W and the apply, with the
-//     matrix in registers (k <= 64) or LDS.
+//     C, b and the sums to a workspace.  Jobs without trans and pao are then
+//     solved without eigenvalues (lekf_trf.hip).  The others: reduction to
+//     tridiagonal form by Householder reflections, implicit QL with shifts (the
+//     method of EISPACK tred2/tql2, the reference's own eigensolver), assembly
+//     of W and the apply, with the matrix in registers (k <= 64) or LDS.
 //   * LEKF_KSPLIT < k <= LEKF_KMAX: a block Gram kernel (one wave per 64 x 64
 //     block of a point) writes the same workspace record, and the eigen
 //     kernel runs the same steps with the matrix left in that record in
 //     global memory (a k = 256 FP64 matrix is 512 KB, beyond the LDS).
 // A point's arithmetic depends only on its own data, so its result is the
 // same whatever else shares the launch.
+#include <algorithm>
+
 #include "lekf_dev.hpp"
 #include "lekf_tune.hpp"
 #include "lekf_ktime.hpp"
+#include "lekf_split.hpp"
 
 namespace {
-
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 
 // value of x in lane src (src uniform across the wave)
 __device__ __forceinline__ double lane_bcast(double x, int src)
@@ -50,26 +46,6 @@ __device__ __forceinline__ double lane_bcast(double x, int src)
     const int lo = __builtin_amdgcn_readlane((int)b, src);
     const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// Reciprocal and reciprocal square root: hardware estimate refined by Newton
-// steps to full FP64 accuracy (a Jacobi rotation only needs c^2 + s^2 = 1 to
-// rounding, which an accurate c = (1+t^2)^-1/2 and s = t c give).
-__device__ __forceinline__ double rcp_nr(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    r = fma(r, fma(-x, r, 1.0), r);
-    return r;
-}
-
-__device__ __forceinline__ double rsq_nr(double x)
-{
-    double r = __builtin_amdgcn_rsq(x);
-    const double h = 0.5 * x;
-    r = r * fma(-h * r, r, 1.5);
-    r = r * fma(-h * r, r, 1.5);
-    return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -335,16 +311,6 @@ __device__ __forceinline__ void store_gram(const ACC* acc, int k, int lda, int l
             ++a;
         }
     }
-}
-
-// Adaptive inflation update (common_letkf.f90:218-239)
-__device__ __forceinline__ double adaptive_alpha(double alpha, double p1, double p2, double p3)
-{
-    const double p4 = (p1 - p3) / p2 - alpha;
-    const double qv = (alpha * p2 + p3) / p2;
-    const double so = 2.0 / p3 * (qv * qv);
-    const double sb2 = 0.04 * 0.04;
-    return alpha + sb2 / (so + sb2) * p4;
 }
 
 // ===========================================================================
@@ -810,17 +776,6 @@ void lekf_solve_kernel(const LekfJob* __restrict__ jobs, int njobs, long npt, in
 // 32 < k <= LEKF_KMAX: Gram kernel + eigen/assembly/apply kernel
 // ===========================================================================
 
-// workspace record of one point: C (k x k, row-major), b (k), sum w d^2, P3
-__host__ __device__ inline long gram_stride(int kmax)
-{
-    return ((long)kmax * kmax + kmax + 2 + 1) & ~1L;
-}
-
-// split-record flag: the mixed-precision pass found C ill-conditioned and put
-// the point on the redo list, whose points a second pass solves again from an
-// FP64 Gram after the launch's last sub-batch
-constexpr int kSplitRedo = 16;
-
 // Waves per SIMD asked of the Gram kernel: the FP64 and FP32 forms with
 // 4 x 4 tiles (49 <= k <= 64) take 214 and 188 registers, two waves per
 // SIMD, unless held to three's budget (which they fit without spilling)
@@ -835,10 +790,12 @@ template <int NT, int MODE, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(gram_waves_per_simd(NT, MODE))))
 void lekf_gram_kernel(
     const LekfJob* __restrict__ jobs, int njobs, long gp0, double* __restrict__ ws, long gstride,
-    const int* __restrict__ rlist)
+    const int* __restrict__ rlist, int* __restrict__ zlist)
 {
     extern __shared__ double smem[];
     const long slot = blockIdx.x;
+    // the launch's first sub-batch empties the redo list before any kernel adds to it
+    if (zlist && blockIdx.x == 0 && threadIdx.x == 0) zlist[0] = 0;
     long gp = gp0 + slot;
     if (rlist) {  // FP64 pass of a split launch: slot i holds the redo list's i-th point
         if (slot >= rlist[0]) return;
@@ -2722,35 +2679,17 @@ __device__ void big_dual_point(const LekfJob& J, int b, double* rec, double* rbu
 // the optional trans/transm/pao outputs and the fused apply
 // Xa = x-mean + X' T evaluated as x-mean + (X' V) diag(sqrt((k-1)/L)) V^T
 // + (X' w-bar) 1^T.
-// The split eigensolver (32 < k <= 64, three kernels per sub-batch): the
-// point's record carries, after the Gram, the Householder Q (transposed: Q_rt
+// The solve with recorded rotations (32 < k <= 64, three kernels per sub-batch,
+// for the jobs that output trans or pao): the point's record carries, after the Gram, the Householder Q (transposed: Q_rt
 // at qoff + t k + r), the tridiagonal d and e, then the eigenvalues, the
 // rotation-stream length and the QL status written by the QL kernel.  The
 // rotation stream of a point holds, per QL sweep, a header (m, count) and the
 // sweep's (c, s) pairs for i = m-1 down to m-count.
 struct SplitRec {
-    long qoff, doff, eoff, lamoff, cntoff, flagoff, qroff;
+    long qoff, doff, eoff, lamoff, cntoff, flagoff;
     const double* rot;  // this point's rotation stream
     long rcap;          // its capacity in (c, s) entries
 };
-constexpr int kSplitOverflow = 8;  // flag: the stream overflowed (the point is solved again in full)
-
-// Flat point of slot `slot` of a split kernel: pass 0 the sub-batch's own
-// (gp0 + slot, nb slots), pass 1 the redo list's (rlist[0] entries from
-// rlist[1], of which the first nb were written: the count goes on past the
-// list's capacity); false past the end.
-__device__ inline bool split_slot_point(long slot, long gp0, long nb, int pass,
-                                        const int* rlist, long& gp)
-{
-    if (pass) {
-        if (slot >= nb || slot >= rlist[0]) return false;
-        gp = rlist[1 + slot];
-        return true;
-    }
-    gp = gp0 + slot;
-    return slot < nb;
-}
-
 // Whether a split kernel of pass `pass` (0: the launch's own precision, 1: the
 // FP64 redo) leaves a point with local obs to the other pass.
 __device__ inline bool split_other_pass(const double* rec, long flagoff, int pass)
@@ -2758,10 +2697,11 @@ __device__ inline bool split_other_pass(const double* rec, long flagoff, int pas
     return ((((int)rec[flagoff]) & kSplitRedo) != 0) != (pass != 0);
 }
 
-__host__ __device__ inline long split_qoff(int kmax) { return gram_stride(kmax); }
+// the flag of both solves follows the Gram
+__host__ __device__ inline long split_qoff(int kmax) { return gram_stride(kmax) + 2; }
 __host__ __device__ inline long split_stride(int kmax)
 {
-    return (gram_stride(kmax) + 2L * kmax * kmax + 3L * kmax + 2 + 1) & ~1L;
+    return (gram_stride(kmax) + 2 + (long)kmax * kmax + 3L * kmax + 1 + 1) & ~1L;
 }
 __host__ __device__ inline long split_rcap(int kmax) { return 2L * kmax * kmax + 8L * kmax; }
 // per point: the column of each rotation-stream entry (-1: a sweep header),
@@ -2778,8 +2718,7 @@ __host__ __device__ inline SplitRec split_rec(int kmax, const double* rot)
     S.eoff = S.doff + kmax;
     S.lamoff = S.eoff + kmax;
     S.cntoff = S.lamoff + kmax;
-    S.flagoff = S.cntoff + 1;
-    S.qroff = S.flagoff + 1;  // Q again, row-major (Q[i][j] at qroff + i * kmax + j)
+    S.flagoff = gram_stride(kmax);
     S.rot = rot;
     S.rcap = split_rcap(kmax);
     return S;
@@ -3046,11 +2985,12 @@ constexpr int eig_waves_per_simd(int kr) { return (kr >= 40 && kr <= 48) ? 2 : 1
 template <int KR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(eig_waves_per_simd(KR))))
 void lekf_eig_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
-                     double* __restrict__ ws, long gstride, int nvmax)
+                     double* __restrict__ ws, long gstride, int nvmax, int all)
 {
     extern __shared__ double smem[];
     const long gp = gp0 + blockIdx.x;
     const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
+    if (!all && !J.trans && !J.pao) return;  // lekf_trd_kernel's
     eig_point<KR, 0>(J, (int)(gp - J.pt_begin + J.pt0), ws + (gp - gp0) * gstride, gstride, nvmax,
                      0L, smem, threadIdx.x);
 }
@@ -3062,14 +3002,13 @@ void lekf_eig_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
 __global__ __launch_bounds__(64) void lekf_tri_kernel(const LekfJob* __restrict__ jobs, int njobs,
                                                        long gp0, double* __restrict__ ws,
                                                        long gstride, int kmax, int pass,
-                                                       int* __restrict__ rlist, int zero)
+                                                       const int* __restrict__ rlist, int all)
 {
     extern __shared__ double smem[];
-    // the launch's first sub-batch empties the redo list (before its QL kernel)
-    if (zero && blockIdx.x == 0 && threadIdx.x == 0) rlist[0] = 0;
     long gp;
     if (!split_slot_point(blockIdx.x, gp0, (long)gridDim.x, pass, rlist, gp)) return;
     const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
+    if (!all && !J.trans && !J.pao) return;  // lekf_trd_kernel's
     const int b = (int)(gp - J.pt_begin + J.pt0);
     const int k = J.k, lane = threadIdx.x, lda = eig_lda(k);
     const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - J.loc_off[b]);
@@ -3089,11 +3028,8 @@ __global__ __launch_bounds__(64) void lekf_tri_kernel(const LekfJob* __restrict_
     __syncthreads();
     eig_tridiag64(L, k, lda, lane);
     if (lane < k) {
-        // Z[r * lda + c] = Q[r][c]; both copies are written a row at a time
-        for (int t = 0; t < k; ++t) {
-            rec[S.qoff + (long)t * k + lane] = L.Z[lane * lda + t];   // Q[lane][t], column-major
-            rec[S.qroff + (long)t * k + lane] = L.Z[t * lda + lane];  // Q[t][lane], row-major
-        }
+        // Z[r * lda + c] = Q[r][c], column-major in the record
+        for (int t = 0; t < k; ++t) rec[S.qoff + (long)t * k + lane] = L.Z[lane * lda + t];
         rec[S.doff + lane] = L.d[lane];
         rec[S.eoff + lane] = L.e[lane];
     }
@@ -3111,7 +3047,7 @@ __global__ __launch_bounds__(64) void lekf_ql_kernel(const LekfJob* __restrict__
                                                       long gstride, double* __restrict__ rot,
                                                       short* __restrict__ ridx, int kmax,
                                                       long rlim, int pass, double kthr,
-                                                      int* __restrict__ rlist, long lcap)
+                                                      int* __restrict__ rlist, long lcap, int all)
 {
     extern __shared__ double sm[];
     const int lane = threadIdx.x;
@@ -3119,6 +3055,7 @@ __global__ __launch_bounds__(64) void lekf_ql_kernel(const LekfJob* __restrict__
     long gp;
     if (!split_slot_point(pt, gp0, nb, pass, rlist, gp)) return;  // no barrier below
     const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
+    if (!all && !J.trans && !J.pao) return;
     const int b = (int)(gp - J.pt_begin + J.pt0);
     const int n = J.k;
     const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - J.loc_off[b]);
@@ -3226,14 +3163,15 @@ template <int KR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(eig_waves_per_simd(KR))))
 void lekf_eig3_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
                       double* __restrict__ ws, long gstride, int nvmax, int kmax,
-                      const double* __restrict__ rot, int pass, const int* __restrict__ rlist)
+                      const double* __restrict__ rot, int pass, const int* __restrict__ rlist,
+                      int all)
 {
     extern __shared__ double smem[];
     const long slot = blockIdx.x;
     long gp;
     if (!split_slot_point(slot, gp0, (long)gridDim.x, pass, rlist, gp)) return;
     const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
-    if (!J.trans && !J.pao) return;  // lekf_evf_kernel's
+    if (!all && !J.trans && !J.pao) return;
     const int b = (int)(gp - J.pt_begin + J.pt0);
     const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - J.loc_off[b]);
     double* rec = ws + slot * gstride;
@@ -3244,342 +3182,44 @@ void lekf_eig3_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
     if (pass && threadIdx.x == 0 && J.status) J.status[b] |= LEKF_PT_FP64;
 }
 
-// Kernel 3 for the other jobs (no trans or pao output): the analysis without
-// forming the eigenvectors.  With A = Q T Q^T (kernel 1) and T = R L R^T (the
-// recorded rotations, R = G_1 G_2 ...), V = Q R, and every quantity the apply
-// needs is a row vector pushed through Q, R, a diagonal, R^T and Q^T:
-//   u = L^-1 V^T b             : row b^T -> b^T Q -> (.) R -> / lambda
-//   X'V diag(U) V^T            : row x   -> x Q   -> (.) R -> * U -> (.) R^T -> (.) Q^T
-//   X' w-bar = (X'V) . u       : the row after R, dotted with u
-//   w-bar = V u                : u -> (.) R^T -> (.) Q^T
-// (U = sqrt((k-1)/lambda), common/common_letkf.f90:119-147).  A rotation costs
-// 6 flops per row instead of 6k for the whole of V, so G = nvmax + 1 lanes
-// serve one point (its state rows, then b) and a wave takes 64 / G points;
-// each lane keeps its row in LDS and follows its own point's rotation
-// stream (column of each entry from the QL kernel, -1 for a sweep header),
-// forward for R and backward with the transposed rotations for R^T.
-// Results agree with the explicit form to rounding.
-constexpr int kEvfChunk = 24;  // rotation-stream entries loaded at once per lane
-
-// Entries e0 .. e0 + kEvfChunk - 1 of a lane's rotation stream (e0 a multiple
-// of 4): (c, s) pairs as 16-byte loads, columns four at a time (the column
-// rows are 8-byte aligned and padded to a multiple of 4); entries from ntot on
-// have column -1.
-__device__ __forceinline__ void evf_chunk(double* cc, double* ss, int* ii, const double* rs,
-                                          const short* rx, long e0, long ntot)
-{
-#pragma unroll
-    for (int u = 0; u < kEvfChunk; u += 4) {
-        const long e = e0 + u;
-        short4 q = make_short4(-1, -1, -1, -1);
-        if (e < ntot) q = *reinterpret_cast<const short4*>(rx + e);
-        ii[u] = e < ntot ? q.x : -1;
-        ii[u + 1] = e + 1 < ntot ? q.y : -1;
-        ii[u + 2] = e + 2 < ntot ? q.z : -1;
-        ii[u + 3] = e + 3 < ntot ? q.w : -1;
-    }
-#pragma unroll
-    for (int u = 0; u < kEvfChunk; ++u) {
-        const long e = e0 + u;
-        double2 cs = make_double2(0.0, 0.0);
-        if (e < ntot) cs = *reinterpret_cast<const double2*>(rs + 2 * e);
-        cc[u] = cs.x;
-        ss[u] = cs.y;
-    }
-}
-
-// The rows of a point group times a k x k matrix M (row-major, global
-// memory), in place in the rows: row_r <- row_r M for the group's G <= RM rows
-// (LDS, stride ld).  Lane v of the group forms columns 8v .. 8v + 7 of every
-// row (G * 8 >= k), so each element of M is loaded by one lane of the group
-// and the loads are contiguous; each sum runs over l in order, as the
-// one-row-per-lane form does.  Uniform call (barriers inside).
-template <int RM>
-__device__ __forceinline__ void evf_coop_mv(double* rows, int ld, int G, int k, const double* M,
-                                            int v, bool solve)
-{
-    double acc[RM][8];
-#pragma unroll
-    for (int r = 0; r < RM; ++r)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[r][j] = 0.0;
-    const int c0 = v * 8;
-    const bool mine = solve && c0 < k;
-    if (mine) {
-        for (int l = 0; l < k; ++l) {
-            const double* ml = M + (size_t)l * k + c0;
-            double q[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) q[j] = (c0 + j < k) ? ml[j] : 0.0;
-#pragma unroll
-            for (int r = 0; r < RM; ++r)
-                if (r < G) {
-                    const double xr = rows[(size_t)r * ld + l];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) acc[r][j] = fma(xr, q[j], acc[r][j]);
-                }
-        }
-    }
-    __syncthreads();
-    if (mine)
-#pragma unroll
-        for (int r = 0; r < RM; ++r)
-            if (r < G)
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (c0 + j < k) rows[(size_t)r * ld + c0 + j] = acc[r][j];
-    __syncthreads();
-}
-
-template <int KR>
-__global__ __launch_bounds__(64) void lekf_evf_kernel(const LekfJob* __restrict__ jobs, int njobs,
-                                                       long gp0, long nb,
-                                                       const double* __restrict__ ws, long gstride,
-                                                       const double* __restrict__ rot,
-                                                       const short* __restrict__ ridx, int nvmax,
-                                                       int kmax, int pass,
-                                                       const int* __restrict__ rlist)
-{
-    extern __shared__ double sm[];
-    const int lane = threadIdx.x;
-    const int G = nvmax + 1, P = 64 / G;
-    const int grp = lane / G, v = lane - grp * G;
-    const long pt = (long)blockIdx.x * P + grp;  // the slot
-    const int ld = kmax | 1;
-    double* row = sm + (size_t)lane * ld;
-    const long rstride = split_rcap(kmax);
-    const SplitRec S = split_rec(kmax, nullptr);
-
-    // this lane's point and row
-    const LekfJob* Jp = nullptr;
-    int b = 0, k = 0, p = 0, nrow = 0, n3 = 0, lev = 0, ij = 0;
-    bool work = false;  // a point this kernel solves
-    long gp = 0;
-    if (grp < P && split_slot_point(pt, gp0, nb, pass, rlist, gp)) {
-        Jp = &jobs[lekf_job_of(jobs, njobs, gp)];
-        b = (int)(gp - Jp->pt_begin + Jp->pt0);
-        k = Jp->k;
-        p = Jp->loc_cnt ? Jp->loc_cnt[b] : (int)(Jp->loc_off[b + 1] - Jp->loc_off[b]);
-        work = !Jp->trans && !Jp->pao;
-        // no local obs: pass 0 writes the outputs; else the pass the flag names
-        if (work && (p <= 0 ? pass != 0 : split_other_pass(ws + pt * gstride, S.flagoff, pass)))
-            work = false;
-        if (work && p > 0 && (((int)ws[pt * gstride + S.flagoff]) & kSplitOverflow)) work = false;
-        if ((Jp->flags & LEKF_F_APPLY)) {
-            lev = b / Jp->nij;
-            ij = b - lev * Jp->nij;
-            n3 = Jp->nv3d;
-            nrow = n3 + (lev == 0 ? Jp->nv2d : 0);
-        }
-    }
-    const bool isb = work && v == nvmax;           // the lane of b
-    const bool isx = work && v < nrow;             // a state row
-    const double* rec = ws + pt * gstride;
-    const double* xsrc = nullptr;
-    double* xdst = nullptr;
-    bool upd = true;
-    if (isx) {
-        const LekfJob& J = *Jp;
-        xsrc = (v < n3) ? J.x3b + ((size_t)b * n3 + v) * k : J.x2b + ((size_t)ij * J.nv2d + (v - n3)) * k;
-        xdst = (v < n3) ? J.x3a + ((size_t)b * n3 + v) * k : J.x2a + ((size_t)ij * J.nv2d + (v - n3)) * k;
-        const uint32_t mask = J.upd_mask ? J.upd_mask[lev] : 0xffffffffu;
-        upd = (v >= n3) || ((mask >> v) & 1u);
-    }
-    double alpha = 1.0;
-    if (work) alpha = Jp->infl_in ? Jp->infl_in[b] : Jp->infl_fixed;
-    // the row's mean in member order (speedy/common/common_speedy.f90:335-370)
-    double mean = 0.0;
-    if (isx) {
-        double sx = xsrc[0];
-        for (int m = 1; m < k; ++m) sx += xsrc[m];
-        mean = sx / (double)k;
-    }
-    const bool solve = work && p > 0;
-    if (work && p <= 0) {
-        // no local obs (common_letkf.f90:82-96): T = sqrt(alpha) I
-        const double sa = sqrt(alpha);
-        if (isx)
-            for (int m = 0; m < k; ++m) {
-                const double xm = xsrc[m] - mean;
-                xdst[m] = upd ? mean + sa * xm : mean + xm;
-            }
-        if (isb) {
-            const LekfJob& J = *Jp;
-            if (J.transm)
-                for (int i = 0; i < k; ++i) J.transm[(size_t)b * k + i] = 0.0;
-            if (J.infl_out) J.infl_out[b] = (J.flags & LEKF_F_FIXED_INFL) ? J.infl_fixed : alpha;
-            if (J.status) J.status[b] = 0;
-        }
-    }
-    const bool act = solve && (isx || isb);
-    // the group's rows go through the matrix products together when they fit
-    // (G <= 8 rows, 8 columns per lane); else each lane its own row
-    const bool coop = G <= 8 && G * 8 >= kmax;
-    // row <- x Q (Q row-major at qroff)
-    if (act) {
-        if (isx)
-            for (int m = 0; m < k; ++m) row[m] = xsrc[m] - mean;
-        else
-            for (int i = 0; i < k; ++i) row[i] = rec[(size_t)k * k + i];
-    }
-    if (coop) {
-        __syncthreads();
-        evf_coop_mv<8>(sm + (size_t)grp * G * ld, ld, G, k, rec + S.qroff, v, solve);
-    } else if (act) {
-        double y[KR];
-#pragma unroll
-        for (int t = 0; t < KR; ++t) y[t] = 0.0;
-        const double* qr = rec + S.qroff;
-        for (int l = 0; l < k; ++l) {
-            const double xl = row[l];
-            const double* ql = qr + (size_t)l * k;
-#pragma unroll
-            for (int t = 0; t < KR; ++t)
-                if (t < k) y[t] = fma(xl, ql[t], y[t]);
-        }
-#pragma unroll
-        for (int t = 0; t < KR; ++t)
-            if (t < k) row[t] = y[t];
-    }
-    // forward through R: entry e rotates columns (i, i+1), (c, s) as the
-    // replay applies it
-    const long ntot = act ? (long)rec[S.cntoff] : 0;
-    const double* rs = rot + pt * 2 * rstride;
-    const short* rx = ridx + pt * split_ridx_stride(kmax);
-    long emax = ntot;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const long t = __shfl_xor(emax, o, 64);
-        emax = t > emax ? t : emax;
-    }
-    // the stream is read kEvfChunk entries at a time, all loads issued before
-    // the chunk's rotations run
-    for (long e0 = 0; e0 < emax; e0 += kEvfChunk) {
-        double cc[kEvfChunk], ss[kEvfChunk];
-        int ii[kEvfChunk];
-        evf_chunk(cc, ss, ii, rs, rx, e0, ntot);
-#pragma unroll
-        for (int u = 0; u < kEvfChunk; ++u) {
-            const int i = ii[u];
-            if (i >= 0) {
-                const double a0 = row[i], a1 = row[i + 1];
-                row[i] = fma(cc[u], a0, -ss[u] * a1);
-                row[i + 1] = fma(ss[u], a0, cc[u] * a1);
-            }
-        }
-    }
-    __syncthreads();
-    // u = (b^T V) / lambda in b's lane; truncation test on lambda
-    double lmax = 0.0, lmin = 1.0e308;
-    if (act)
-        for (int t = 0; t < k; ++t) {
-            const double lt = rec[S.lamoff + t];
-            lmax = lt > lmax ? lt : lmax;
-            lmin = lt < lmin ? lt : lmin;
-            if (isb) row[t] = row[t] / lt;
-        }
-    __syncthreads();
-    // X' w-bar = (x V) . u, then x V diag(U)
-    double cw = 0.0;
-    if (act && isx) {
-        const double* u = sm + (size_t)(grp * G + nvmax) * ld;
-        for (int t = 0; t < k; ++t) cw = fma(row[t], u[t], cw);
-        for (int t = 0; t < k; ++t) row[t] = row[t] * sqrt((double)(k - 1) / rec[S.lamoff + t]);
-    }
-    __syncthreads();
-    // backward through R^T: the entries in reverse, each rotation transposed
-    for (long e0 = emax > 0 ? ((emax - 1) / kEvfChunk) * kEvfChunk : -1; e0 >= 0;
-         e0 -= kEvfChunk) {
-        double cc[kEvfChunk], ss[kEvfChunk];
-        int ii[kEvfChunk];
-        evf_chunk(cc, ss, ii, rs, rx, e0, ntot);
-#pragma unroll
-        for (int u = kEvfChunk - 1; u >= 0; --u) {
-            const int i = ii[u];
-            if (i >= 0) {
-                const double a0 = row[i], a1 = row[i + 1];
-                row[i] = fma(cc[u], a0, ss[u] * a1);
-                row[i + 1] = fma(-ss[u], a0, cc[u] * a1);
-            }
-        }
-    }
-    // out = row Q^T (Q column-major at qoff: Q[m][t] at qoff + t * k + m, i.e.
-    // Q^T row-major)
-    if (coop) {
-        __syncthreads();
-        evf_coop_mv<8>(sm + (size_t)grp * G * ld, ld, G, k, rec + S.qoff, v, solve);
-    }
-    if (act) {
-        double out[KR];
-#pragma unroll
-        for (int m = 0; m < KR; ++m) out[m] = 0.0;
-        if (coop) {
-#pragma unroll
-            for (int m = 0; m < KR; ++m)
-                if (m < k) out[m] = row[m];
-        } else {
-            const double* qc = rec + S.qoff;
-            for (int t = 0; t < k; ++t) {
-                const double zt = row[t];
-                const double* qt = qc + (size_t)t * k;
-#pragma unroll
-                for (int m = 0; m < KR; ++m)
-                    if (m < k) out[m] = fma(zt, qt[m], out[m]);
-            }
-        }
-        const LekfJob& J = *Jp;
-        if (isx) {
-#pragma unroll
-            for (int m = 0; m < KR; ++m)
-                if (m < k) xdst[m] = upd ? mean + (cw + out[m]) : mean + (xsrc[m] - mean);
-        } else {
-            // w-bar, inflation, status
-            if (J.transm)
-#pragma unroll
-                for (int i = 0; i < KR; ++i)
-                    if (i < k) J.transm[(size_t)b * k + i] = out[i];
-            if ((J.flags & LEKF_F_MINFL) && J.minfl > 0.0 && alpha < J.minfl) alpha = J.minfl;
-            if (J.infl_out) {
-                double tr = 0.0;
-                for (int i = 0; i < k; ++i) tr += rec[(size_t)i * k + i];
-                const double p1 = rec[(size_t)k * k + k], p3 = rec[(size_t)k * k + k + 1];
-                J.infl_out[b] = (J.flags & LEKF_F_FIXED_INFL)
-                                    ? J.infl_fixed
-                                    : adaptive_alpha(alpha, p1, tr / (double)(k - 1), p3);
-            }
-            if (J.status) {
-                int status = (((int)rec[S.flagoff]) & 1) ? LEKF_PT_NOCONV : 0;
-                if (!(lmax > 0.0) || lmin < fabs(lmax) * 1.4901161193847656e-08)
-                    status |= LEKF_PT_RANKDEF;
-                J.status[b] = status | (pass ? LEKF_PT_FP64 : 0);
-            }
-        }
-    }
-}
-
-// The points of a split launch whose rotation stream overflowed: the fused
-// eigen kernel's work (from the Gram still at the start of the record), the
-// others return at once.
+// The points of a launch that the other kernels flagged kSplitOverflow (a rotation
+// stream that overflowed, a condition number past the rational form's tables): the
+// fused eigen kernel's work, from the Gram still at the start of the record.  A
+// workgroup looks through 64 slots' flags and solves the flagged ones in turn.
 template <int KR>
 __global__ __launch_bounds__(64) void lekf_eig_fix_kernel(const LekfJob* __restrict__ jobs,
-                                                           int njobs, long gp0,
+                                                           int njobs, long gp0, long nb,
                                                            double* __restrict__ ws, long gstride,
-                                                           int nvmax, int kmax, int pass,
+                                                           int nvmax, int kmax, int pass, int all,
                                                            const int* __restrict__ rlist)
 {
     extern __shared__ double smem[];
-    long gp;
-    if (!split_slot_point(blockIdx.x, gp0, (long)gridDim.x, pass, rlist, gp)) return;
-    const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
-    const int b = (int)(gp - J.pt_begin + J.pt0);
-    const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - J.loc_off[b]);
-    double* rec = ws + (long)blockIdx.x * gstride;
-    const SplitRec S = split_rec(kmax, nullptr);
-    if (p <= 0 || split_other_pass(rec, S.flagoff, pass) ||
-        !(((int)rec[S.flagoff]) & kSplitOverflow))
-        return;
-    eig_point<KR, 0>(J, b, rec, gstride, nvmax, 0L, smem, threadIdx.x);
-    if (pass && threadIdx.x == 0 && J.status) J.status[b] |= LEKF_PT_FP64;
+    const long slot0 = (long)blockIdx.x * 64;
+    bool mine = false;
+    {
+        const long slot = slot0 + threadIdx.x;
+        long gp;
+        if (slot < nb && split_slot_point(slot, gp0, nb, pass, rlist, gp)) {
+            const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
+            const int b = (int)(gp - J.pt_begin + J.pt0);
+            const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - J.loc_off[b]);
+            // (points that no kernel of this launch flags have no flag to read)
+            if (p > 0 && (all || (!J.trans && !J.pao))) {
+                const int flag = (int)ws[slot * gstride + gram_stride(kmax)];
+                mine = (flag & kSplitOverflow) && ((flag & kSplitRedo) != 0) == (pass != 0);
+            }
+        }
+    }
+    for (unsigned long long left = __ballot(mine); left; left &= left - 1) {
+        const long slot = slot0 + (__ffsll(left) - 1);
+        long gp;
+        (void)split_slot_point(slot, gp0, nb, pass, rlist, gp);
+        const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
+        const int b = (int)(gp - J.pt_begin + J.pt0);
+        __syncthreads();
+        eig_point<KR, 0>(J, b, ws + slot * gstride, gstride, nvmax, 0L, smem, threadIdx.x);
+        if (pass && threadIdx.x == 0 && J.status) J.status[b] |= LEKF_PT_FP64;
+    }
 }
 
 // LEKF_KSPLIT < k: one persistent wave per workgroup slot strides over the
@@ -3645,32 +3285,60 @@ size_t lekf_solve_lds_bytes(int k, int nvmax)
 // of 4 for k <= 64, 0 (LDS eigensolver) above
 static int eig_kr(int kmax) { return kmax <= 64 ? (kmax + 3) & ~3 : 0; }
 
-static bool split_path(int kmax)
+// the solves that read the Gram from the workspace (32 < k <= LEKF_KSPLIT), by
+// what the launch's jobs ask for (outs: LEKF_OUT_PLAIN, LEKF_OUT_TRANS)
+struct SplitPlan {
+    bool plain;    // lekf_trd_kernel + lekf_trf_kernel for the jobs without trans and pao
+    bool streams;  // Householder, QL with recorded rotations, replay (k <= 64)
+    bool fused;    // lekf_eig_kernel
+    int all;       // the streams or the fused kernel take every job
+};
+static SplitPlan split_plan(int kmax, int outs)
 {
-    return kmax > 32 && kmax <= LEKF_KSPLIT && g_lekf_tune.eig_split && eig_kr(kmax) > 0;
+    const bool reg = eig_kr(kmax) > 0;
+    SplitPlan P{};
+    if (!g_lekf_tune.eig_split) {
+        P.fused = true;
+        P.all = 1;
+        return P;
+    }
+    // a stream capacity that was set explicitly asks for the recorded rotations
+    P.all = reg && g_lekf_tune.split_rcap > 0;
+    P.plain = (outs & LEKF_OUT_PLAIN) && !P.all;
+    P.streams = reg && ((outs & LEKF_OUT_TRANS) || P.all);
+    P.fused = !reg && (outs & LEKF_OUT_TRANS);
+    return P;
 }
 
-// bytes per point of a sub-batch: the record, plus the rotation stream on the
-// split path
-static size_t ws_rec_bytes(int kmax)
+static long split_rec_stride(int kmax, const SplitPlan& P)
+{
+    long n = gram_stride(kmax);
+    if (P.plain) n = std::max(n, trf_stride(kmax));
+    if (P.streams) n = std::max(n, split_stride(kmax));
+    return n;
+}
+
+// bytes per point of a sub-batch: the record, the rotation stream where one is
+// recorded, a redo-list entry
+static size_t ws_rec_bytes(int kmax, int outs)
 {
     if (kmax > LEKF_KSPLIT) return (size_t)big_stride(kmax) * sizeof(double);
-    if (split_path(kmax))  // record, rotation stream, its columns, a redo-list entry
-        return (size_t)(split_stride(kmax) + 2 * split_rcap(kmax) + split_ridx_doubles(kmax) + 1) *
-               sizeof(double);
-    return (size_t)gram_stride(kmax) * sizeof(double);
+    const SplitPlan P = split_plan(kmax, outs);
+    long n = split_rec_stride(kmax, P) + 1;
+    if (P.streams) n += 2 * split_rcap(kmax) + split_ridx_doubles(kmax);
+    return (size_t)n * sizeof(double);
 }
 
-size_t lekf_solve_ws_bytes(long npt, int kmax)
+size_t lekf_solve_ws_bytes(long npt, int kmax, int outs)
 {
     if (kmax <= 32 || npt <= 0) return 0;
     const bool big = kmax > LEKF_KSPLIT;
-    const size_t rec = ws_rec_bytes(kmax);
+    const size_t rec = ws_rec_bytes(kmax, outs);
     size_t per = g_lekf_tune.gram_ws_bytes / rec;
     if (per < 1) per = 1;
-    // large-k records are MBs each, and the split path's QL kernel takes 64
-    // points per wave: keep at least 1024 points per launch
-    if ((big || split_path(kmax)) && per < 1024) per = 1024;
+    // large-k records are MBs each, and the QL kernel takes 64 points per wave:
+    // keep at least 1024 points per launch
+    if ((big || g_lekf_tune.eig_split) && per < 1024) per = 1024;
     if ((size_t)npt < per) per = (size_t)npt;
     return per * rec;
 }
@@ -3690,14 +3358,14 @@ static hipError_t launch_fused(const LekfJob* djobs, int njobs, long npt, int km
 }
 
 static hipError_t launch_eig(int kr, long nb, size_t elds, hipStream_t st, const LekfJob* djobs,
-                             int njobs, long g0, double* ws, long gs, int nvmax)
+                             int njobs, long g0, double* ws, long gs, int nvmax, int all)
 {
     KTime kt("eig", st);
     switch (kr) {
 #define LEKF_EIG_CASE(K)                                                                       \
     case K:                                                                                    \
         hipLaunchKernelGGL(lekf_eig_kernel<K>, dim3((unsigned)nb), dim3(LEKF_WAVE), elds, st, \
-                           djobs, njobs, g0, ws, gs, nvmax);                                  \
+                           djobs, njobs, g0, ws, gs, nvmax, all);                             \
         break;
         LEKF_EIG_CASE(36)
         LEKF_EIG_CASE(40)
@@ -3714,15 +3382,13 @@ static hipError_t launch_eig(int kr, long nb, size_t elds, hipStream_t st, const
     return hipGetLastError();
 }
 
-static hipError_t launch_eig_split(int kr, long nb, size_t elds, hipStream_t st,
-                                   const LekfJob* djobs, int njobs, long g0, double* ws, long gs,
-                                   int nvmax, int kmax, double* rot, short* ridx, int pass,
-                                   double kthr, int* rlist, int zero, long lcap)
+// the recorded-rotation solve of a sub-batch (32 < k <= 64)
+static hipError_t launch_streams(int kr, long nb, size_t elds, hipStream_t st,
+                                 const LekfJob* djobs, int njobs, long g0, double* ws, long gs,
+                                 int nvmax, int kmax, double* rot, short* ridx, int pass,
+                                 double kthr, int* rlist, long lcap, int all)
 {
     const unsigned nwq = (unsigned)((nb + 63) / 64);
-    const int evp = 64 / (nvmax + 1);  // points per wave of the eigenvector-free kernel
-    const unsigned nwe = (unsigned)((nb + evp - 1) / evp);
-    const size_t flds = 64 * (size_t)(kmax | 1) * sizeof(double);
     const size_t qlds = 2 * (size_t)kr * 64 * sizeof(double);
     const size_t tlds = tri_lds_doubles(kmax) * sizeof(double);
     switch (kr) {
@@ -3731,21 +3397,17 @@ static hipError_t launch_eig_split(int kr, long nb, size_t elds, hipStream_t st,
         {                                                                                        \
             KTime kt(pass ? "redo_tri" : "eig_tri", st);                                         \
             hipLaunchKernelGGL(lekf_tri_kernel, dim3((unsigned)nb), dim3(LEKF_WAVE), tlds, st,    \
-                               djobs, njobs, g0, ws, gs, kmax, pass, rlist, zero);              \
+                               djobs, njobs, g0, ws, gs, kmax, pass, rlist, all);               \
         }                                                                                        \
         {                                                                                        \
             KTime kt(pass ? "redo_ql" : "eig_ql", st);                                           \
             hipLaunchKernelGGL(lekf_ql_kernel<K>, dim3(nwq), dim3(LEKF_WAVE), qlds, st, djobs,    \
                                njobs, g0, nb, ws, gs, rot, ridx, kmax,                           \
-                               g_lekf_tune.split_rcap, pass, kthr, rlist, lcap);                \
+                               g_lekf_tune.split_rcap, pass, kthr, rlist, lcap, all);           \
         }                                                                                        \
         KTime kt(pass ? "redo_apply" : "eig_apply", st);                                         \
         hipLaunchKernelGGL(lekf_eig3_kernel<K>, dim3((unsigned)nb), dim3(LEKF_WAVE), elds, st,    \
-                           djobs, njobs, g0, ws, gs, nvmax, kmax, rot, pass, rlist);            \
-        hipLaunchKernelGGL(lekf_evf_kernel<K>, dim3(nwe), dim3(LEKF_WAVE), flds, st, djobs,      \
-                           njobs, g0, nb, ws, gs, rot, ridx, nvmax, kmax, pass, rlist);         \
-        hipLaunchKernelGGL(lekf_eig_fix_kernel<K>, dim3((unsigned)nb), dim3(LEKF_WAVE), elds, st, \
-                           djobs, njobs, g0, ws, gs, nvmax, kmax, pass, rlist);                 \
+                           djobs, njobs, g0, ws, gs, nvmax, kmax, rot, pass, rlist, all);       \
         break;                                                                                   \
     }
         LEKF_SPLIT_CASE(36)
@@ -3762,65 +3424,104 @@ static hipError_t launch_eig_split(int kr, long nb, size_t elds, hipStream_t st,
     return hipGetLastError();
 }
 
+static hipError_t launch_fix(int kr, long nb, size_t elds, hipStream_t st, const LekfJob* djobs,
+                             int njobs, long g0, double* ws, long gs, int nvmax, int kmax, int pass,
+                             int all, const int* rlist)
+{
+    const unsigned nwg = (unsigned)((nb + 63) / 64);
+    switch (kr) {
+#define LEKF_FIX_CASE(K)                                                                          \
+    case K:                                                                                       \
+        hipLaunchKernelGGL(lekf_eig_fix_kernel<K>, dim3(nwg), dim3(LEKF_WAVE), elds, st, djobs,   \
+                           njobs, g0, nb, ws, gs, nvmax, kmax, pass, all, rlist);                 \
+        break;
+        LEKF_FIX_CASE(36)
+        LEKF_FIX_CASE(40)
+        LEKF_FIX_CASE(44)
+        LEKF_FIX_CASE(48)
+        LEKF_FIX_CASE(52)
+        LEKF_FIX_CASE(56)
+        LEKF_FIX_CASE(60)
+        LEKF_FIX_CASE(64)
+        LEKF_FIX_CASE(0)
+#undef LEKF_FIX_CASE
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 template <int NT, int MODE>
 static hipError_t launch_gram(int W, long nb, size_t glds, hipStream_t st, const LekfJob* djobs,
-                              int njobs, long g0, double* ws, long gs, const int* rlist)
+                              int njobs, long g0, double* ws, long gs, const int* rlist,
+                              int* zlist)
 {
     KTime kt(rlist ? "redo_gram" : "gram", st);
     if (W == 2)
         hipLaunchKernelGGL((lekf_gram_kernel<NT, MODE, 2>), dim3((unsigned)nb), dim3(128), glds, st,
-                           djobs, njobs, g0, ws, gs, rlist);
+                           djobs, njobs, g0, ws, gs, rlist, zlist);
     else if (W == 8)
         hipLaunchKernelGGL((lekf_gram_kernel<NT, MODE, 8>), dim3((unsigned)nb), dim3(512), glds, st,
-                           djobs, njobs, g0, ws, gs, rlist);
+                           djobs, njobs, g0, ws, gs, rlist, zlist);
     else
         hipLaunchKernelGGL((lekf_gram_kernel<NT, MODE, 4>), dim3((unsigned)nb), dim3(256), glds, st,
-                           djobs, njobs, g0, ws, gs, rlist);
+                           djobs, njobs, g0, ws, gs, rlist, zlist);
     return hipGetLastError();
 }
 
 template <int NT, int MODE>
 static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int kmax, int nvmax,
-                               void* ws, size_t ws_bytes, hipStream_t st)
+                               int outs, void* ws, size_t ws_bytes, hipStream_t st)
 {
-    const bool s3 = split_path(kmax);
-    const long gs = s3 ? split_stride(kmax) : gram_stride(kmax);
-    const long per = (long)(ws_bytes / ws_rec_bytes(kmax));
+    const SplitPlan plan = split_plan(kmax, outs);
+    const long gs = split_rec_stride(kmax, plan);
+    const long per = (long)(ws_bytes / ws_rec_bytes(kmax, outs));
     if (per < 1 || !ws) return hipErrorInvalidValue;
     double* rot = (double*)ws + (size_t)per * gs;  // the rotation streams after the records
-    short* ridx = (short*)(rot + (size_t)per * 2 * split_rcap(kmax));  // then their columns
-    int* rlist = (int*)(ridx + (size_t)per * split_ridx_stride(kmax));  // then the redo list
+    short* ridx = (short*)(rot + (plan.streams ? (size_t)per * 2 * split_rcap(kmax) : 0));
+    // then their columns, then the redo list
+    int* rlist = (int*)(ridx + (plan.streams ? (size_t)per * split_ridx_stride(kmax) : 0));
     const int W = g_lekf_tune.gram_waves;
+    const int kr = eig_kr(kmax);
     const size_t glds = ((size_t)kmax * (kmax + 1) + kmax + 4 + W) * sizeof(double);
     const size_t elds = eig_lds_doubles(kmax, nvmax) * sizeof(double);
-    // mixed forms on the split eigensolver: the QL kernel lists the points whose
-    // C is worse conditioned than kthr (up to one sub-batch of them per launch),
-    // and after the last sub-batch one FP64 pass solves the listed points again
-    // (one set of kernel latencies per launch, whatever the sub-batch count).
-    // The FP32 Gram rounds about 16 times finer than split-BF16x3, so its
-    // threshold is 16 times the value set.
-    const double kthr = (MODE != 0 && s3 && npt <= 0x7fffffffL)
+    // mixed forms on the split eigensolver: the points whose C is worse conditioned
+    // than kthr are listed (up to one sub-batch of them per launch), and after the
+    // last sub-batch one FP64 pass solves the listed points again (one set of
+    // kernel latencies per launch, whatever the sub-batch count).  The FP32 Gram
+    // rounds about 16 times finer than split-BF16x3, so its threshold is 16 times
+    // the value set.
+    const double kthr = (MODE != 0 && kr > 0 && g_lekf_tune.eig_split && npt <= 0x7fffffffL)
                             ? (MODE == 1 ? 16.0 : 1.0) * (double)g_lekf_tune.mixed_kappa
                             : 0.0;
+    auto solve = [&](long g0, long nb, int pass, double thr) {
+        hipError_t e = hipSuccess;
+        if (plan.streams)
+            e = launch_streams(kr, nb, elds, st, djobs, njobs, g0, (double*)ws, gs, nvmax, kmax,
+                               rot, ridx, pass, thr, rlist, per, plan.all);
+        if (e == hipSuccess && plan.plain)
+            e = lekf_trf_launch(nb, st, djobs, njobs, g0, (double*)ws, gs, nvmax, kmax, pass,
+                                pass ? 0 : MODE, thr, rlist, per);
+        if (e == hipSuccess && (plan.streams || plan.plain))
+            e = launch_fix(kr, nb, elds, st, djobs, njobs, g0, (double*)ws, gs, nvmax, kmax, pass,
+                           plan.streams, rlist);
+        if (e == hipSuccess && plan.fused)
+            e = launch_eig(plan.all ? kr : 0, nb, elds, st, djobs, njobs, g0, (double*)ws, gs,
+                           nvmax, plan.all);
+        return e;
+    };
     for (long g0 = 0; g0 < npt; g0 += per) {
         const long nb = per < npt - g0 ? per : npt - g0;
-        hipError_t e =
-            launch_gram<NT, MODE>(W, nb, glds, st, djobs, njobs, g0, (double*)ws, gs, nullptr);
-        if (e != hipSuccess) return e;
-        if (s3)
-            e = launch_eig_split(eig_kr(kmax), nb, elds, st, djobs, njobs, g0, (double*)ws, gs,
-                                 nvmax, kmax, rot, ridx, 0, kthr, rlist, g0 == 0, per);
-        else
-            e = launch_eig(eig_kr(kmax), nb, elds, st, djobs, njobs, g0, (double*)ws, gs, nvmax);
+        hipError_t e = launch_gram<NT, MODE>(W, nb, glds, st, djobs, njobs, g0, (double*)ws, gs,
+                                             nullptr, g0 == 0 ? rlist : nullptr);
+        if (e == hipSuccess) e = solve(g0, nb, 0, kthr);
         if (e != hipSuccess) return e;
     }
     if (kthr > 0.0) {
         // grids of one sub-batch; the slots past the list's length return at once
         const long nl = per < npt ? per : npt;
-        hipError_t e = launch_gram<NT, 0>(W, nl, glds, st, djobs, njobs, 0, (double*)ws, gs, rlist);
-        if (e == hipSuccess)
-            e = launch_eig_split(eig_kr(kmax), nl, elds, st, djobs, njobs, 0, (double*)ws, gs, nvmax,
-                                 kmax, rot, ridx, 1, 0.0, rlist, 0, per);
+        hipError_t e = launch_gram<NT, 0>(W, nl, glds, st, djobs, njobs, 0, (double*)ws, gs, rlist,
+                                          nullptr);
+        if (e == hipSuccess) e = solve(0, nl, 1, 0.0);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -3853,7 +3554,7 @@ static hipError_t launch_big(const LekfJob* djobs, int njobs, long npt, int kmax
 
 template <int MODE>
 static hipError_t launch_mode(int cls, const LekfJob* djobs, int njobs, long npt, int kmax,
-                              int nvmax, void* ws, size_t ws_bytes, hipStream_t st)
+                              int nvmax, int outs, void* ws, size_t ws_bytes, hipStream_t st)
 {
     switch (cls) {
     case 4 * 8 + 1: return launch_fused<1, 4, MODE>(djobs, njobs, npt, kmax, nvmax, st);
@@ -3864,10 +3565,10 @@ static hipError_t launch_mode(int cls, const LekfJob* djobs, int njobs, long npt
     case 24 * 8 + 2: return launch_fused<2, 24, MODE>(djobs, njobs, npt, kmax, nvmax, st);
     case 28 * 8 + 2: return launch_fused<2, 28, MODE>(djobs, njobs, npt, kmax, nvmax, st);
     case 32 * 8 + 3: return launch_fused<3, 32, MODE>(djobs, njobs, npt, kmax, nvmax, st);
-    case 3: return launch_split<3, MODE>(djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
-    case 4: return launch_split<4, MODE>(djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
-    case 5: return launch_split<5, MODE>(djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
-    case 6: return launch_split<6, MODE>(djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
+    case 3: return launch_split<3, MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
+    case 4: return launch_split<4, MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
+    case 5: return launch_split<5, MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
+    case 6: return launch_split<6, MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
     case kClassBig: return launch_big<MODE>(djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
     default: return hipErrorInvalidValue;
     }
@@ -3875,15 +3576,16 @@ static hipError_t launch_mode(int cls, const LekfJob* djobs, int njobs, long npt
 
 // Launch the solve over npt flat points of njobs jobs (device array djobs).
 // Every job of a launch has the same kernel class; kmax (the largest k) and
-// nvmax (the most state rows a point applies to) size the LDS; ws is the
-// Gram workspace of lekf_solve_ws_bytes(npt, kmax) bytes (k > 32).
+// nvmax (the most state rows a point applies to) size the LDS; outs: whether any
+// of them outputs trans or pao, and whether any does not; ws is the Gram workspace
+// of lekf_solve_ws_bytes(npt, kmax, outs) bytes (k > 32).
 hipError_t lekf_solve_launch(const LekfJob* djobs, int njobs, long npt, int kmax, int nvmax,
-                             int mode, void* ws, size_t ws_bytes, hipStream_t st)
+                             int mode, int outs, void* ws, size_t ws_bytes, hipStream_t st)
 {
     if (npt <= 0) return hipSuccess;
     if (nvmax > LEKF_NVMAX) return hipErrorInvalidValue;
     const int cls = lekf_solve_class(kmax);
-    if (mode == 0) return launch_mode<0>(cls, djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
-    if (mode == 1) return launch_mode<1>(cls, djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
-    return launch_mode<2>(cls, djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
+    if (mode == 0) return launch_mode<0>(cls, djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
+    if (mode == 1) return launch_mode<1>(cls, djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
+    return launch_mode<2>(cls, djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
 }

@@ -31,6 +31,8 @@
 // candidates, the new set and the block's evictions come from ranks in the
 // union, and a candidate evicted within its own block passes its slot on
 // (pointer jumping).
+#include <algorithm>
+
 #include "lekf_dev.hpp"
 #include "lekf_regional.hpp"
 #include "lekf_tune.hpp"
@@ -485,29 +487,37 @@ __device__ int cap_stream(SelLds& S, const CapGlobal& G, KeyAt keyat, Emit emit,
 }
 
 // ---------------------------------------------------------------------------
-// The cap by one wave (caps up to LEKF_CAP_LDS), fed chunk by chunk with the
-// candidates of one bucket stream in scan order.
+// The cap by one wave (caps up to LEKF_CAP_LDS), fed with the candidates of one
+// bucket stream in scan order.
 //
-// The kept set S (the cap smallest (key, scan position) of the stream so
-// far) is held ascending in key[], with each entry's storage slot in slot[];
-// so[s] (caller's memory) is the candidate in storage slot s (an obs or list
-// position, which increases in scan order).  The first cap candidates fill
-// slots 0..cap-1; each 64 of them are sorted across the lanes and merged
-// into the sorted prefix as they arrive.  A later candidate can enter only if
-// its key is below the key tau of S's last entry (an earlier candidate with
-// an equal key precedes it), and tau only falls, so candidates are filtered
-// against tau into a queue and each block of 64 queued candidates is merged
-// at once:
+// The kept set S (the cap smallest (key, scan position) of the stream so far) is
+// held ascending in key[], with each entry's storage slot in slot[]; so[s]
+// (caller's memory) is the candidate in storage slot s.  The first cap candidates
+// fill slots 0..cap-1: only their positions are kept until the cap-th arrives, then
+// they are sorted in by batches.  A later candidate can enter only if its key is
+// below the key tau of S's last entry (an earlier candidate with an equal key
+// precedes it), and tau only falls, so the caller filters candidates by any bound
+// that keeps every key below tau, into a queue, and up to kWcB = 224 queued
+// candidates are evaluated exactly (four per lane, their long chains overlapping)
+// and merged at once:
 // * a candidate enters iff fewer than cap of S and of the earlier queued
-//   candidates precede it; all of S precedes it in scan order, so its count
-//   in S is the number of keys <= its key, and the earlier queued candidates
-//   before it come from a 64-lane sort by (key, lane);
-// * the entries of S move up by the entrants before them, and the top e of
-//   S and the entrants leave;
-// * the i-th entrant in scan order takes the slot of the i-th largest entry
-//   that left: the reference evicts the current last entry each time, and
-//   the last key only falls; an entrant that leaves in its own block hands
-//   its slot on (pointer jumping).
+//   candidates precede it.  All of S precedes it in scan order, so its count there
+//   candidates precede it.  All of S precedes it in scan order, so its count there
+//   is c1, the number of keys <= its key; the block's candidates are ranked by key
+//   (a counting sort over the leading bits of the keys' range), and where c1 and the
+//   rank together reach cap the earlier ones among those ranked before are counted
+//   as a set of scan positions;
+// * the entrants are counted per c1: a scan of the counts over S from the top gives
+//   every entry's move;
+// * of S and the entrants the top e leave; the i-th entrant in scan order takes the
+//   slot of the i-th largest entry that left: the reference evicts the current last
+//   entry each time, and the last key only falls; an entrant that leaves in its own
+//   block hands its slot on (pointer jumping).
+// Bound by VALU issue, 62% of it at three waves per SIMD.  Against blocks of 64 sorted
+// across the lanes with every candidate evaluated exactly as it was scanned, a stream
+// takes 46 k vector and 17 k scalar instructions instead of 69 k and 42 k, and the
+// radar 128 x 128 x 60 selection (two streams of 12.5 k candidates per point) 251
+// instead of 401 ms per cycle; the GFS-sized grid's list_cap_wave 22 instead of 33 ms.
 // ---------------------------------------------------------------------------
 
 // order of the lanes' LDS traffic within the wave (no cross-wave sharing)
@@ -517,262 +527,462 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
-struct WaveCap {
-    unsigned long long key[LEKF_CAP_LDS];
+// Candidates per block, at most kWcU per lane.  The LDS decides how many waves hide
+// each other's latencies: 13,440 bytes a wave are 21 granules (1280 bytes) for two,
+// six such workgroups per CU, three waves per SIMD.
+constexpr int kWcU = 4;
+constexpr int kWcB = 224;
+
+struct __align__(16) WaveCap {
+    unsigned long long key[LEKF_CAP_LDS];  // while S fills: the positions, in the upper half
+    unsigned cnt[LEKF_CAP_LDS / 2];        // 16-bit counts, and what comes after them in a block
     unsigned short slot[LEKF_CAP_LDS];
-    unsigned long long qkey[128];  // queued candidates, scan order
-    int qo[128];
-    int ev[64];                    // entries that left a block, ascending: slot, or -(entrant + 1)
-    int slotn[64];
-    int link[64];
+    int qp[kWcB + 64];                     // queued candidates, scan order
 };
+static_assert(sizeof(WaveCap) == 13440, "LDS per wave of the cap");
+constexpr unsigned short kWcOwn = 0x8000, kWcNone = 0xffff;
+
+// Positions of the first cap candidates.  When the fill has sorted the first lim of
+// them their keys end at byte 8 lim and the positions still to come begin at byte
+// 4 LEKF_CAP_LDS + 4 lim, so none is overwritten before it is read.
+__device__ __forceinline__ int* wc_fill_pos(WaveCap& L)
+{
+    return (int*)(L.key + LEKF_CAP_LDS / 2);
+}
 
 struct WcState {
-    int n;                   // stream candidates so far
+    int n;                   // stream candidates so far (exact up to cap)
     int m;                   // sorted prefix of S while it fills
     int q;                   // queued candidates
-    unsigned long long tau;  // key of S's last entry (once n >= cap)
+    unsigned long long tau;  // key of S's last entry (once m = cap)
 };
 
-// ascending bitonic sort of the 64 lanes' (key, id) pairs (ids distinct)
-__device__ __forceinline__ void wave_sort64(unsigned long long& k, int& id, int lane)
+__device__ __forceinline__ int wave_scan(int v)  // inclusive sum over the lanes up to this one
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+
+__device__ __forceinline__ unsigned wave_scan_or(unsigned v)  // the same, by or
+{
+    v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);
+    v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+    v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);
+    v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned dpp_max(unsigned v)
+{
+    const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+    return o > v ? o : v;
+}
+__device__ __forceinline__ unsigned wave_max(unsigned v)
+{
+    v = dpp_max<0x111, 0xf>(v);
+    v = dpp_max<0x112, 0xf>(v);
+    v = dpp_max<0x114, 0xf>(v);
+    v = dpp_max<0x118, 0xf>(v);
+    v = dpp_max<0x142, 0xa>(v);
+    v = dpp_max<0x143, 0xc>(v);
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ unsigned wave_min(unsigned v) { return ~wave_max(~v); }
+
+// The counts: LEKF_CAP_LDS of 16 bits (no count passes kWcB), added to in pairs.
+__device__ __forceinline__ void wc_zero(WaveCap& L, int lane)
 {
 #pragma unroll
-    for (int sz = 2; sz <= 64; sz <<= 1) {
+    for (int j = 0; j < LEKF_CAP_LDS / 512; ++j)
+        reinterpret_cast<uint4*>(L.cnt)[j * 64 + lane] = make_uint4(0, 0, 0, 0);
+}
+__device__ __forceinline__ int wc_count(WaveCap& L, int i)  // returns the count before
+{
+    const int sh = (i & 1) * 16;
+    return (int)((atomicAdd(&L.cnt[i >> 1], 1u << sh) >> sh) & 0xffffu);
+}
+
+// One block: np <= kWcB candidates (positions src[0 .. np), scan order) join S.
+// fill < 0: S is full, queued candidates against tau; else S's first fill entries are
+// sorted and the candidates are its entries fill .. fill + np - 1, in slots of that
+// number.  eval(p, ok): the key of the candidate at position p, ok: it is a stream
+// candidate (the fill's are).  Returns S's new last key.
+template <class Eval>
+__device__ __forceinline__ unsigned long long wc_block(WaveCap& L, int* so, const int* src, int np,
+                                                       int fill, int cap, int lane,
+                                                       unsigned long long tau, Eval eval)
+{
+    const bool full = fill < 0;
+    const int n = full ? cap : fill;         // entries of S
+    const int lim = full ? cap : fill + np;  // and after the block
+    int p[kWcU], c1[kWcU], t[kWcU], rank[kWcU];
+    unsigned long long y[kWcU];
+    bool ent[kWcU];
 #pragma unroll
-        for (int j = sz >> 1; j > 0; j >>= 1) {
-            const unsigned lo = (unsigned)lane_xor((int)(unsigned)k, j, lane);
-            const unsigned hi = (unsigned)lane_xor((int)(unsigned)(k >> 32), j, lane);
-            const unsigned long long ok = ((unsigned long long)hi << 32) | lo;
-            const int oid = lane_xor(id, j, lane);
-            const bool up = (lane & sz) == 0;
-            const bool lower = (lane & j) == 0;
-            const bool oless = ok < k || (ok == k && oid < id);
-            if (lower == up ? oless : !oless) {
-                k = ok;
-                id = oid;
-            }
-        }
-    }
-}
-
-// number of the first n keys (ascending) that are <= y
-__device__ __forceinline__ int wc_count_le(const WaveCap& L, int n, unsigned long long y)
-{
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (L.key[mid] <= y)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
-// Entries 0..n-1 of key[]/slot[] move up by the new entries placed before
-// them (lanes with ent, at count c1 of the old entries: before old entry i
-// iff c1 <= i); an entry that lands at lim or above goes to ev[] instead
-// (its slot).  Windows of 64 go top down, so a window's writes only reach
-// entries that already moved, and each lane holds one entry at a time.
-__device__ __forceinline__ void wc_shift(WaveCap& L, int n, int lim, bool ent, int c1, int lane)
-{
-    const unsigned long long em = __ballot(ent);
-    if (!em || n <= 0) return;
-    const int c1min = __builtin_amdgcn_readlane(c1, __builtin_ctzll(em));
-    for (int lo = ((n - 1) >> 6) << 6; lo >= 0 && lo + 64 > c1min; lo -= 64) {
-        const int i = lo + lane;
-        unsigned long long k = 0;
-        int s = 0;
-        if (i < n) {
-            k = L.key[i];
-            s = L.slot[i];
-        }
-        int ptr = __popcll(__ballot(ent && c1 < lo));
-        unsigned long long wm = __ballot(ent && c1 >= lo && c1 < lo + 64);
-        while (wm) {
-            const int bl = __builtin_ctzll(wm);
-            wm &= wm - 1;
-            const int d = __builtin_amdgcn_readlane(c1, bl) - lo;
-            ptr += lane >= d ? 1 : 0;
-        }
-        if (i < n && ptr > 0) {
-            const int ni = i + ptr;
-            if (ni < lim) {
-                L.key[ni] = k;
-                L.slot[ni] = (unsigned short)s;
-            } else {
-                L.ev[ni - lim] = s;
-            }
-        }
-    }
-}
-
-// While S fills: the nt (<= 64) entries at m.. (slots m.., unsorted) join
-// the sorted prefix 0..m-1.
-__device__ void wc_fill_merge(WaveCap& L, int m, int nt, int lane)
-{
-    unsigned long long sk = lane < nt ? L.key[m + lane] : ~0ull;
-    int sid = lane;
-    wave_sort64(sk, sid, lane);  // the nt entries take lanes 0..nt-1 (ties: slot order)
-    const bool v = lane < nt;
-    const int c1 = v ? wc_count_le(L, m, sk) : m;
+    for (int u = 0; u < kWcU; ++u) p[u] = u * 64 + lane < np ? src[u * 64 + lane] : -1;
     wave_sync();
-    wc_shift(L, m, m + nt, v, c1, lane);
-    wave_sync();
-    if (v) {
-        L.key[c1 + lane] = sk;
-        L.slot[c1 + lane] = (unsigned short)(m + sid);
-    }
-    wave_sync();
-}
-
-// One block: queued candidates 0..np-1 (np <= 64) against the full set S.
-__device__ void wc_block(WaveCap& L, int* so, int np, int cap, int lane, unsigned long long& tau)
-{
-    const bool valid = lane < np;
-    const unsigned long long y = valid ? L.qkey[lane] : ~0ull;
-    const bool live = valid && y < tau;  // tau has fallen below it since it was queued: out
-    const int c1 = live ? wc_count_le(L, cap, y) : cap;
-    // sort the live candidates by (key, lane): lane L holds the L-th
-    unsigned long long sk = live ? y : ~0ull;
-    int sid = lane;
-    wave_sort64(sk, sid, lane);
-    const bool slive = sk != ~0ull;
-    unsigned long long pm = slive ? (1ull << sid) : 0ull;
+    wc_zero(L, lane);
+    int nlive = 0;
+    unsigned hmin = ~0u, hmax = 0u;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const unsigned long long t = __shfl_up(pm, d, 64);
-        if (lane >= d) pm |= t;
+    for (int u = 0; u < kWcU; ++u) {
+        bool ok = false;
+        y[u] = ~0ull;
+        if (p[u] >= 0) y[u] = eval(p[u], ok);
+        ent[u] = p[u] >= 0 && (full ? ok && y[u] < tau : true);
+        nlive += __popcll(__ballot(ent[u]));
+        const unsigned h = (unsigned)(y[u] >> 32);
+        if (ent[u]) {
+            hmin = h < hmin ? h : hmin;
+            hmax = h > hmax ? h : hmax;
+        }
     }
-    // earlier (in scan order) live candidates sorted before this one
-    const unsigned long long before = pm & ~(slive ? (1ull << sid) : 0ull);
-    const int c2 = __popcll(before & (sid == 0 ? 0ull : (~0ull >> (64 - sid))));
-    const int c1s = __shfl(c1, sid, 64);
-    const bool ents = slive && c1s + c2 < cap;
-    const unsigned long long emS = __ballot(ents);
-    const int e = __popcll(emS);
-    if (e == 0) return;
-    const int r = __popcll(emS & lane_lt(lane));  // rank among the entrants
-    const int U = c1s + r;                        // position in S + entrants
-    // scan-order index of each entrant: its flag back to the candidate's lane
-    const int ento = __builtin_amdgcn_ds_permute(sid << 2, ents ? 1 : 0);
-    const unsigned long long emO = __ballot(ento != 0);
-    const int t = __shfl((int)__popcll(emO & lane_lt(lane)), sid, 64);
-    wave_sync();
-    wc_shift(L, cap, cap, ents, c1s, lane);
-    wave_sync();
-    if (ents) {
-        if (U < cap)
-            L.key[U] = sk;
-        else
-            L.ev[U - cap] = -(t + 1);
-    }
-    wave_sync();
-    int sl = -1, ln = -1;
-    if (ents) {
-        const int v = L.ev[e - 1 - t];
-        if (v >= 0)
-            sl = v;
-        else
-            ln = -v - 1;
-        L.slotn[t] = sl;
-        L.link[t] = ln;
-    }
-    wave_sync();
-    for (int round = 0; round < 8 && __ballot(ents && sl < 0); ++round) {
-        int s2 = -1, l2 = -1;
-        if (ents && sl < 0) {
-            s2 = L.slotn[ln];
-            l2 = L.link[ln];
+    if (nlive == 0) return tau;
+    // rank by key: counting sort over the leading bits of the keys' range, then a look
+    // at the candidates of the same count
+    {
+        const unsigned long long k0 = (unsigned long long)wave_min(hmin) << 32;
+        const unsigned span = wave_max(hmax) - (unsigned)(k0 >> 32);
+        const int sh = span ? 54 - __builtin_clz(span) : 22;  // (span + 1) 2^32 - 1 >> sh < 1024
+        int g[kWcU], tick[kWcU], base[kWcU], mem[kWcU], big = 1;
+        wave_sync();
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u) {
+            g[u] = ent[u] ? (int)((y[u] - k0) >> sh) : 0;
+            tick[u] = ent[u] ? wc_count(L, g[u]) : 0;
         }
         wave_sync();
-        if (ents && sl < 0) {
-            if (s2 >= 0)
-                sl = s2;
+        unsigned short* cnt = (unsigned short*)L.cnt;  // counts to the ranks they start at
+        int run = 0;
+        for (int lo = 0; lo < LEKF_CAP_LDS; lo += 256) {
+            int cn[4], pin[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) cn[j] = cnt[lo + 64 * j + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) pin[j] = wave_scan(cn[j]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                cnt[lo + 64 * j + lane] = (unsigned short)(run + pin[j] - cn[j]);
+                run += __builtin_amdgcn_readlane(pin[j], 63);
+            }
+        }
+        wave_sync();
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u) {
+            base[u] = cnt[g[u]];
+            mem[u] = ent[u] ? (g[u] + 1 < LEKF_CAP_LDS ? (int)cnt[g[u] + 1] : nlive) - base[u] : 0;
+            big = mem[u] > big ? mem[u] : big;
+            rank[u] = base[u];
+        }
+        wave_sync();
+        unsigned long long* ekey = (unsigned long long*)L.cnt;  // the counts are spent
+        unsigned char* eidx = (unsigned char*)(ekey + kWcB);
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u)
+            if (mem[u] > 1) {
+                ekey[base[u] + tick[u]] = y[u];
+                eidx[base[u] + tick[u]] = (unsigned char)(u * 64 + lane);
+            }
+        wave_sync();
+        for (int j = 0; __ballot(big > 1 && j < big); ++j)
+#pragma unroll
+            for (int u = 0; u < kWcU; ++u)
+                if (j < mem[u] && mem[u] > 1) {
+                    const unsigned long long x = ekey[base[u] + j];
+                    rank[u] += x < y[u] || (x == y[u] && (int)eidx[base[u] + j] < u * 64 + lane);
+                }
+        wave_sync();
+    }
+    // entries of S before each candidate
+    {
+        int lo[kWcU], hi[kWcU];
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u) {
+            lo[u] = 0;
+            hi[u] = ent[u] ? n : 0;
+        }
+        for (int w = n; w > 0; w >>= 1)
+#pragma unroll
+            for (int u = 0; u < kWcU; ++u) {
+                const int mid = (lo[u] + hi[u]) >> 1;
+                const bool le = L.key[mid < n ? mid : 0] <= y[u];
+                if (lo[u] < hi[u]) {
+                    lo[u] = le ? mid + 1 : lo[u];
+                    hi[u] = le ? hi[u] : mid;
+                }
+            }
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u) c1[u] = lo[u];
+    }
+    int e = nlive;
+    if (full) {
+        // a live candidate enters if fewer than cap of S and of the live candidates
+        // before it precede it; rank bounds the latter
+        bool amb = false;
+        int lt[kWcU], before = 0;
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u) {
+            const unsigned long long m = __ballot(ent[u]);
+            const int r = before + __popcll(m & lane_lt(lane));
+            lt[u] = r < rank[u] ? r : rank[u];
+            amb |= ent[u] && c1[u] + lt[u] >= cap;
+            before += __popcll(m);
+        }
+        if (__ballot(amb)) {
+            // in rank order, four candidates per lane: the set of scan positions
+            // ranked before each (their bits are distinct), and of it those earlier
+            unsigned char* sidx = (unsigned char*)L.cnt;
+            unsigned short* c2 = (unsigned short*)(L.cnt + 64);
+#pragma unroll
+            for (int u = 0; u < kWcU; ++u)
+                if (ent[u]) sidx[rank[u]] = (unsigned char)(u * 64 + lane);
+            wave_sync();
+            const unsigned ids = L.cnt[lane];
+            unsigned own[8], ex[8];
+#pragma unroll
+            for (int d = 0; d < 8; ++d) {
+                own[d] = 0;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int i = (ids >> (8 * v)) & 255;
+                    if (4 * lane + v < nlive && (i >> 5) == d) own[d] |= 1u << (i & 31);
+                }
+                ex[d] = wave_scan_or(own[d]) & ~own[d];
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int i = (ids >> (8 * v)) & 255;
+                int c = 0;
+#pragma unroll
+                for (int d = 0; d < 8; ++d) {
+                    const unsigned lower = (i >> 5) > d ? ~0u : (i >> 5) == d ? (1u << (i & 31)) - 1 : 0u;
+                    c += __popc(ex[d] & lower);
+                    if ((i >> 5) == d) ex[d] |= 1u << (i & 31);
+                }
+                if (4 * lane + v < nlive) c2[4 * lane + v] = (unsigned short)c;
+            }
+            wave_sync();
+            // the entrants, and their ranks among themselves
+            bool in[kWcU];
+            e = 0;
+#pragma unroll
+            for (int u = 0; u < kWcU; ++u) {
+                in[u] = ent[u] && c1[u] + (int)c2[ent[u] ? rank[u] : 0] < cap;
+                e += __popcll(__ballot(in[u]));
+            }
+            if (e == 0) return tau;
+            wave_sync();
+            if (e < nlive) {
+                L.cnt[lane] = 0;
+                wave_sync();
+#pragma unroll
+                for (int u = 0; u < kWcU; ++u)
+                    if (in[u]) sidx[rank[u]] = 1;
+                wave_sync();
+                const unsigned fl = L.cnt[lane];
+                const int own4 = __popc(fl);
+                int r = wave_scan(own4) - own4;
+                unsigned short* re = c2;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    re[4 * lane + v] = (unsigned short)r;
+                    r += (fl >> (8 * v)) & 1;
+                }
+                wave_sync();
+#pragma unroll
+                for (int u = 0; u < kWcU; ++u) {
+                    ent[u] = in[u];
+                    if (in[u]) rank[u] = re[rank[u]];
+                }
+                wave_sync();
+            }
+        }
+    }
+    {
+        int before = 0;
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u) {
+            const unsigned long long m = __ballot(ent[u]);
+            t[u] = before + __popcll(m & lane_lt(lane));  // rank among the entrants, scan order
+            before += __popcll(m);
+        }
+    }
+    // entrants per c1; then, from the top down, 256 entries of S at a time: entry i
+    // moves up by the entrants with c1 <= i (writes only reach entries that have been
+    // read)
+    wc_zero(L, lane);
+    wave_sync();
+#pragma unroll
+    for (int u = 0; u < kWcU; ++u)
+        if (ent[u]) (void)wc_count(L, c1[u]);
+    wave_sync();
+    const unsigned short* at = (const unsigned short*)L.cnt;
+    unsigned short* ev = (unsigned short*)L.qp;  // entries that left, ascending: slot, or
+                                                 // kWcOwn + entrant (these candidates are read)
+    for (int lo = (full ? n - 1 : n) & ~255, left = e; lo >= 0 && left > 0; lo -= 256) {
+        int cn[4], shift[4];
+        unsigned long long k[4];
+        unsigned short s[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = lo + 64 * j + lane;
+            cn[j] = at[i];
+            k[j] = L.key[i];
+            s[j] = L.slot[i];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) shift[j] = wave_scan(cn[j]);
+        int tot = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int w = __builtin_amdgcn_readlane(shift[j], 63);
+            shift[j] += tot;
+            tot += w;
+        }
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = lo + 64 * j + lane;
+            const int ni = i + left - tot + shift[j];
+            if (i < n && ni > i) {
+                if (ni < lim) {
+                    L.key[ni] = k[j];
+                    L.slot[ni] = s[j];
+                } else {
+                    ev[ni - lim] = s[j];
+                }
+            }
+        }
+        left -= tot;
+        wave_sync();
+    }
+    if (!full) {
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u)
+            if (ent[u]) {
+                const int q = c1[u] + rank[u];
+                L.key[q] = y[u];
+                L.slot[q] = (unsigned short)(fill + t[u]);
+                so[fill + t[u]] = p[u];
+            }
+        wave_sync();
+        return L.key[lim - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < kWcU; ++u)
+        if (ent[u]) {
+            const int q = c1[u] + rank[u];
+            if (q < cap)
+                L.key[q] = y[u];
             else
-                ln = l2;
-            L.slotn[t] = sl;
-            L.link[t] = ln;
+                ev[q - cap] = (unsigned short)(kWcOwn | t[u]);
         }
-        wave_sync();
-    }
-    if (ents && U < cap && sl >= 0) {
-        L.slot[U] = (unsigned short)sl;
-        so[sl] = L.qo[sid];
+    wave_sync();
+    unsigned short* slotn = (unsigned short*)L.cnt;  // the counts are spent
+    unsigned short* link = slotn + kWcB;
+    int sl[kWcU], ln[kWcU];
+    bool open = false;
+#pragma unroll
+    for (int u = 0; u < kWcU; ++u) {
+        sl[u] = 0;
+        ln[u] = 0;
+        if (ent[u]) {
+            const int v = ev[e - 1 - t[u]];
+            const bool own = (v & kWcOwn) != 0;
+            sl[u] = own ? -1 : v;
+            ln[u] = v & ~kWcOwn;
+            open |= own;
+            slotn[t[u]] = own ? kWcNone : (unsigned short)v;
+            link[t[u]] = (unsigned short)ln[u];
+        }
     }
     wave_sync();
-    tau = L.key[cap - 1];
+    // chains of at most kWcB entrants: 8 doublings
+    for (int round = 0; round < 8 && __ballot(open); ++round) {
+        int s2[kWcU], l2[kWcU];
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u) {
+            s2[u] = slotn[sl[u] < 0 ? ln[u] : 0];
+            l2[u] = link[sl[u] < 0 ? ln[u] : 0];
+        }
+        wave_sync();
+        open = false;
+#pragma unroll
+        for (int u = 0; u < kWcU; ++u)
+            if (sl[u] < 0) {
+                if (s2[u] != kWcNone)
+                    sl[u] = s2[u];
+                else
+                    ln[u] = l2[u];
+                open |= sl[u] < 0;
+                slotn[t[u]] = sl[u] < 0 ? kWcNone : (unsigned short)sl[u];
+                link[t[u]] = (unsigned short)ln[u];
+            }
+        wave_sync();
+    }
+#pragma unroll
+    for (int u = 0; u < kWcU; ++u)
+        if (ent[u] && c1[u] + rank[u] < cap && sl[u] >= 0) {
+            L.slot[c1[u] + rank[u]] = (unsigned short)sl[u];
+            so[sl[u]] = p[u];
+        }
+    wave_sync();
+    return L.key[cap - 1];
 }
 
-// One chunk of the stream: lane l's position is a stream candidate iff ok
-// (key k, candidate o); positions are in scan order across the lanes.
-__device__ void wc_push(WaveCap& L, int* so, WcState& S, bool ok, unsigned long long k, int o,
-                        int cap, int lane)
+// A chunk of the stream: lane l's candidate p enters the fill or the queue iff in
+// (while S fills every stream candidate; then at least those with a key below tau).
+__device__ __forceinline__ void wc_push(WaveCap& L, WcState& S, bool in, int p, int cap, int lane)
 {
-    const unsigned long long am = __ballot(ok);
-    if (!am) return;
-    const int rank = __popcll(am & lane_lt(lane));
-    const int n0 = S.n;
-    S.n += __popcll(am);
-    bool pend = ok;
-    if (n0 < cap) {
-        if (ok && n0 + rank < cap) {
-            const int f = n0 + rank;
-            L.key[f] = k;
-            so[f] = o;
-            pend = false;
-        }
-        wave_sync();
-        const int nf = S.n < cap ? S.n : cap;
-        while (nf - S.m >= 64 || (S.n >= cap && S.m < cap)) {
-            const int nt = nf - S.m < 64 ? nf - S.m : 64;
-            wc_fill_merge(L, S.m, nt, lane);
-            S.m += nt;
-        }
-        if (S.n < cap) return;
-        S.tau = L.key[cap - 1];
-        if (S.n == cap) return;
+    const unsigned long long m = __ballot(in);
+    if (!m) return;
+    const int cnt = __popcll(m), rank = __popcll(m & lane_lt(lane));
+    const int room = S.n < cap ? cap - S.n : 0;  // the fill's share
+    if (in) {
+        if (rank < room)
+            wc_fill_pos(L)[S.n + rank] = p;
+        else
+            L.qp[S.q + rank - room] = p;
     }
-    const bool pot = pend && k < S.tau;
-    const unsigned long long pm = __ballot(pot);
-    if (!pm) return;
-    if (pot) {
-        const int qp = S.q + __popcll(pm & lane_lt(lane));
-        L.qkey[qp] = k;
-        L.qo[qp] = o;
-    }
-    S.q += __popcll(pm);
+    const int f = cnt < room ? cnt : room;
+    S.n += f;
+    S.q += cnt - f;
     wave_sync();
-    if (S.q >= 64) {
-        wc_block(L, so, 64, cap, lane, S.tau);
-        // the rest of the queue moves to its front
-        const bool mv = 64 + lane < S.q;
-        unsigned long long k2 = 0;
-        int o2 = 0;
-        if (mv) {
-            k2 = L.qkey[64 + lane];
-            o2 = L.qo[64 + lane];
-        }
-        wave_sync();
-        if (mv) {
-            L.qkey[lane] = k2;
-            L.qo[lane] = o2;
-        }
-        S.q -= 64;
-        wave_sync();
-    }
 }
 
-// End of the stream: the last queued block.  Returns the kept count; the
-// kept candidates are so[0 .. kept) in slot order (visible to the wave's
-// loads after a workgroup-scope fence).
-__device__ int wc_finish(WaveCap& L, int* so, WcState& S, int cap, int lane)
+// Blocks that are due: the fill's once S has cap entries, the queue's when kWcB
+// candidates wait, or any with last.
+template <class Eval>
+__device__ __forceinline__ void wc_service(WaveCap& L, int* so, WcState& S, int cap, int lane,
+                                           bool last, Eval eval)
 {
-    if (S.q > 0) wc_block(L, so, S.q, cap, lane, S.tau);
-    S.q = 0;
-    wave_sync();
-    return S.n < cap ? S.n : cap;
+    while (S.n >= cap) {
+        const bool filling = S.m < cap;
+        if (!filling && S.q < kWcB && !(last && S.q > 0)) break;
+        const int have = filling ? cap - S.m : S.q;
+        const int np = have < kWcB ? have : kWcB;
+        S.tau = wc_block(L, so, filling ? wc_fill_pos(L) + S.m : L.qp, np, filling ? S.m : -1, cap,
+                         lane, S.tau, eval);
+        if (filling) {
+            S.m += np;
+        } else {
+            // the rest of the queue (fewer than 64) moves to its front
+            S.q -= np;
+            int o = 0;
+            if (lane < S.q) o = L.qp[kWcB + lane];
+            wave_sync();
+            if (lane < S.q) L.qp[lane] = o;
+            wave_sync();
+        }
+    }
 }
 
 // Persistent selection: workgroup g handles points g, g + gridDim.x, ...
@@ -922,22 +1132,19 @@ __global__ __launch_bounds__(kSelT) void reg_select(RegionalArgs A, long npt)
 // persistent, one point per workgroup, wave t caps bucket t's stream (NW =
 // nbkt waves).  A bucket's candidates in the point's rectangle are, row by
 // row, one contiguous range of the bucket-by-bucket obs copy, in the
-// reference's scan order restricted to the bucket; each is evaluated once
-// (eval_rec) and fed to the wave's cap.  The lists are written bucket by
-// bucket in slot order, rho recomputed from the kept obs.
-struct RowTab {
-    int beg[64];
-    int pre[65];
-};
-
+// reference's scan order restricted to the bucket.  The scan reads a 16-byte
+// FP32 record per candidate and decides in FP32 where its error bound allows:
+// candidates within the bound of the cutoff while S fills are evaluated exactly,
+// later ones whose key may be below tau go to the wave's queue and are evaluated
+// exactly there (eval_rec), so the lists are the reference's.  They are written
+// bucket by bucket in slot order, rho recomputed from the kept obs.
 constexpr int kTileX = 16, kTileY = 8;  // columns of a selection tile
 
 template <int NW>
-__global__ __launch_bounds__(64 * NW) void reg_select_wave(RegionalArgs A, long npt)
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3)))
+void reg_select_wave(RegionalArgs A, long npt)
 {
     __shared__ WaveCap L[NW];
-    __shared__ RowTab R[NW];
-    __shared__ int kept_s[NW];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int nij = A.nx * A.ny;
     const int cap = A.nobs_max;
@@ -945,13 +1152,22 @@ __global__ __launch_bounds__(64 * NW) void reg_select_wave(RegionalArgs A, long 
     int bs = 0;  // bucket wv's first position in the bucket-by-bucket copy
     for (int u = 0; u < wv; ++u) bs += A.bcc[(size_t)u * nij + nij - 1];
     WaveCap& W = L[wv];
-    RowTab& T = R[wv];
-    int* so = A.wc_so + ((size_t)blockIdx.x * NW + wv) * LEKF_CAP_LDS;  // slot -> obs
+    int* so = A.wc_so + ((size_t)blockIdx.x * NW + wv) * LEKF_CAP_LDS;  // slot -> position
     const double r2cut = kNdMax * A.sigma_h * A.sigma_h * (1.0 + 1e-9);
     // the bucket's smallest err^2 (NaN for an empty bucket: never used)
     const double e2min = A.err2_min ? __longlong_as_double((long long)A.err2_min[wv]) : 0.0;
-    const float ish2 = (float)(1.0 / (A.sigma_h * A.sigma_h));
-    const float isv2 = (float)(1.0 / (A.sigma_v * A.sigma_v));
+    const double ish2 = 1.0 / (A.sigma_h * A.sigma_h);
+    const float cx = (float)(A.dx * A.dx * ish2), cy = (float)(A.dy * A.dy * ish2);
+    const float cv = (float)(1.0 / (A.sigma_v * A.sigma_v));
+    // rounding of a horizontal coordinate difference in FP32, in units of sigma_h
+    const double eh = (A.nx > A.ny ? A.nx : A.ny) * 1.2e-7 *
+                      (A.dx > A.dy ? A.dx : A.dy) / A.sigma_h;
+    // the position's record, evaluated exactly
+    auto load_rec = [&](int p) {
+        const double2 rij = *reinterpret_cast<const double2*>(A.brec + 4 * (size_t)p);
+        const double2 zer = *reinterpret_cast<const double2*>(A.brec + 4 * (size_t)p + 2);
+        return ObsRec{rij.x, rij.y, zer.x, zer.y, wv};
+    };
 
     // XCD-aware tile order: workgroup w runs on XCD w % 8 (round-robin
     // dispatch); the XCD's workgroups take the points of one kTileX x kTileY
@@ -983,127 +1199,129 @@ __global__ __launch_bounds__(64 * NW) void reg_select_wave(RegionalArgs A, long 
         if (imax > A.nx) imax = A.nx;
         if (jmin < 1) jmin = 1;
         if (jmax > A.ny) jmax = A.ny;
+        const float fri = (float)(ix + 1), frj = (float)(iy + 1), frz = (float)rz;
+        // bound of the FP32 nd's error for nd up to the cutoff (sqrt 13.4 < 3.7):
+        // 2 sqrt(nd) (e_x + e_y + e_z) + the squares + the arithmetic's 1e-5
+        const double ev = (fabs(rz) + 4.0 * A.sigma_v) * 1.2e-7 / A.sigma_v;
+        const double es = 2.0 * eh + ev;
+        const float em = (float)(7.4 * es + es * es + 1.0e-4);
+        const float nd_out = (float)kNdMax + em, nd_in = (float)kNdMax - em;
+        float l2tau = 3.0e38f;  // log2 tau and the bound
         WcState S{0, 0, 0, ~0ull};
-        if (imin <= imax) {
-            for (int j0 = jmin; j0 <= jmax; j0 += 64) {
-                const int nr = jmax - j0 + 1 < 64 ? jmax - j0 + 1 : 64;
-                int beg = 0, len = 0;
-                if (lane < nr) {
-                    // the row's cells that can hold an obs within the cutoff: a
-                    // cell's obs lie on its side of the faces at i +- 0.5, so one
-                    // whose nearest face is beyond the cutoff radius holds none
-                    // (nd >= nd_h^2 > kNdMax); a 1e-9 margin covers rounding
-                    const int j = j0 + lane;
-                    const double dyg = fmax(0.0, fabs((double)j - rj) - 0.5) * A.dy;
-                    const double rem = r2cut - dyg * dyg;
-                    int ilo = imin, ihi = imax;
-                    if (rem < 0.0) {
-                        ihi = ilo - 1;
-                    } else {
-                        const double rx = sqrt(rem) / A.dx + 0.5;
-                        const int a = (int)ceil(ri - rx), z = (int)floor(ri + rx);
-                        ilo = a > imin ? a : imin;
-                        ihi = z < imax ? z : imax;
-                    }
-                    if (ilo <= ihi) {
-                        const int rowbase = (j - 1) * A.nx;
-                        const int lo = rowbase + ilo - 1, hi = rowbase + ihi - 1;
-                        const int c0 = lo > 0 ? cc[lo - 1] : 0;
-                        beg = bs + c0;
-                        len = cc[hi] - c0;
-                    }
+        auto eval = [&](int p, bool& ok) {
+            const Cand c = eval_rec(A, load_rec(p), p, ri, rj, rz);
+            ok = c.ok;
+            return c.bits;
+        };
+        bool fin = imin > imax;
+        for (int j0 = jmin;; j0 += 64) {
+            fin |= j0 > jmax;
+            const int nr = fin ? 0 : (jmax - j0 + 1 < 64 ? jmax - j0 + 1 : 64);
+            int beg = 0, len = 0;
+            if (lane < nr) {
+                // the row's cells that can hold an obs within the cutoff: a
+                // cell's obs lie on its side of the faces at i +- 0.5, so one
+                // whose nearest face is beyond the cutoff radius holds none
+                // (nd >= nd_h^2 > kNdMax); a 1e-9 margin covers rounding
+                const int j = j0 + lane;
+                const double dyg = fmax(0.0, fabs((double)j - rj) - 0.5) * A.dy;
+                const double rem = r2cut - dyg * dyg;
+                int ilo = imin, ihi = imax;
+                if (rem < 0.0) {
+                    ihi = ilo - 1;
+                } else {
+                    const double rx = sqrt(rem) / A.dx + 0.5;
+                    const int a = (int)ceil(ri - rx), z = (int)floor(ri + rx);
+                    ilo = a > imin ? a : imin;
+                    ihi = z < imax ? z : imax;
                 }
-                int pre = len;
-#pragma unroll
-                for (int d = 1; d < 64; d <<= 1) {
-                    const int v = __shfl_up(pre, d, 64);
-                    if (lane >= d) pre += v;
+                if (ilo <= ihi) {
+                    const int rowbase = (j - 1) * A.nx;
+                    const int lo = rowbase + ilo - 1, hi = rowbase + ihi - 1;
+                    const int c0 = lo > 0 ? cc[lo - 1] : 0;
+                    beg = bs + c0;
+                    len = cc[hi] - c0;
                 }
-                T.beg[lane] = beg;
-                T.pre[lane + 1] = pre;
-                if (lane == 0) T.pre[0] = 0;
-                const int tot = __shfl(pre, 63, 64);
-                wave_sync();
-                // candidate q of the row group -> its position; loads of the next
-                // chunk are issued before the current one is evaluated
-                int r0 = 0;
-                ObsRec nrec;
-                int no = -1;
-                auto fetch = [&](int qb) {
-                    while (r0 < nr && T.pre[r0 + 1] <= qb) ++r0;
-                    const int q = qb + lane;
-                    no = -1;
-                    if (q < tot) {
-                        int r = r0;
-                        while (T.pre[r + 1] <= q) ++r;
-                        const int p = T.beg[r] + (q - T.pre[r]);
-                        const double2 rij = *reinterpret_cast<const double2*>(A.brec + 4 * (size_t)p);
-                        const double2 zer = *reinterpret_cast<const double2*>(A.brec + 4 * (size_t)p + 2);
-                        nrec.ri = rij.x;
-                        nrec.rj = rij.y;
-                        nrec.z = zer.x;
-                        nrec.err = zer.y;
-                        nrec.b = wv;
-                        no = A.bo[p];
-                    }
-                };
-                fetch(0);
-                for (int q0 = 0; q0 < tot; q0 += 64) {
-                    if (S.n >= cap && (double)(j0 + r0) - rj > 0.5) {
-                        // rows from this chunk's first one on lie beyond the
-                        // point: an obs of row j has |rj_o - rj| > j - rj - 0.5,
-                        // so nd > ((j - rj - 0.5) dy / sigma_h)^2 and its key
+            }
+            // the rows that hold candidates, 64 of one row at a time; the next chunk's
+            // loads are on their way while one is tested
+            unsigned long long rows = __ballot(len > 0);
+            int r = 0, rbeg = 0, rlen = 0, at = 0, np = -1;
+            float4 nrec = make_float4(0.f, 0.f, 0.f, 0.f);
+            auto row = [&]() {
+                r = __builtin_ctzll(rows);
+                rbeg = __builtin_amdgcn_readlane(beg, r);
+                rlen = __builtin_amdgcn_readlane(len, r);
+                at = 0;
+            };
+            auto fetch = [&]() {
+                np = at + lane < rlen ? rbeg + at + lane : -1;
+                if (np >= 0) nrec = A.brf[np];
+            };
+            if (rows) {
+                row();
+                fetch();
+            }
+            do {
+                if (rows) {
+                    if (at == 0 && S.m >= cap && (double)(j0 + r) - rj > 0.5) {
+                        // rows from this one on lie beyond the point: an obs of
+                        // row j has |rj_o - rj| > j - rj - 0.5, so
+                        // nd > ((j - rj - 0.5) dy / sigma_h)^2 and its key
                         // err^2 / rho exceeds err2_min exp(nd / 2); once that
                         // bound (less a 1e-9 margin for rounding) reaches tau,
                         // which only falls, no later candidate can enter
-                        const double g = ((double)(j0 + r0) - rj - 0.5) * A.dy / A.sigma_h;
+                        const double g = ((double)(j0 + r) - rj - 0.5) * A.dy / A.sigma_h;
                         const double lb = e2min * exp(0.5 * g * g) * (1.0 - 1e-9);
-                        if (lb >= __longlong_as_double((long long)S.tau)) break;
+                        if (lb >= __longlong_as_double((long long)S.tau)) {
+                            fin = true;
+                            rows = 0;
+                        }
                     }
-                    const ObsRec cur = nrec;
-                    const int co = no;
-                    if (q0 + 64 < tot)
-                        fetch(q0 + 64);
-                    else
-                        no = -1;
-                    Cand c;
-                    c.ok = false;
-                    c.bits = 0;
-                    // once the kept set is full, a float bound in the log2 domain
-                    // (errors near 1e-5 for candidates within the cutoff, against
-                    // a 1e-3 margin) skips the exact evaluation of a candidate whose
-                    // key certainly exceeds tau: it could not enter, and past the
-                    // fill the stream count no longer matters
-                    bool need = co >= 0;
-                    if (need && S.n >= cap) {
-                        const float fx = (float)((ri - cur.ri) * A.dx);
-                        const float fy = (float)((rj - cur.rj) * A.dy);
-                        const float fz = (float)(cur.z - rz);
-                        const float nd = (fx * fx + fy * fy) * ish2 + fz * fz * isv2;
-                        const float l2 = __log2f((float)(cur.err * cur.err)) + 0.72134752f * nd;
-                        need = !(l2 > __log2f((float)__longlong_as_double((long long)S.tau)) + 1e-3f);
-                    }
-                    if (need) c = eval_rec(A, cur, co, ri, rj, rz);
-                    wc_push(W, so, S, c.ok, c.bits, co, cap, lane);
                 }
-                wave_sync();
-            }
+                if (rows) {
+                    const float4 cur = nrec;
+                    const int p = np;
+                    at += 64;
+                    if (at >= rlen) {
+                        rows &= rows - 1;
+                        if (rows) row();
+                    }
+                    if (rows) fetch();
+                    const float fx = fri - cur.x, fy = frj - cur.y, fz = cur.z - frz;
+                    const float nd = __builtin_fmaf(fx * fx, cx,
+                                                    __builtin_fmaf(fy * fy, cy, fz * fz * cv));
+                    bool in = p >= 0 && !(nd > nd_out);
+                    if (S.n < cap) {
+                        if (in && !(nd < nd_in)) in = eval_rec(A, load_rec(p), p, ri, rj, rz).ok;
+                    } else if (S.m >= cap) {
+                        in = in && !(__builtin_fmaf(0.72134752f, nd, cur.w) > l2tau);
+                    }
+                    wc_push(W, S, in, p, cap, lane);
+                }
+                const unsigned long long tau0 = S.tau;
+                wc_service(W, so, S, cap, lane, fin, eval);
+                if (S.tau != tau0)
+                    // 0.73 em for nd's error, 1e-3 for the logarithms'
+                    l2tau = (float)log2(__longlong_as_double((long long)S.tau)) + 0.73f * em + 1.0e-3f;
+            } while (rows);
+            if (fin) break;
         }
-        const int kept = wc_finish(W, so, S, cap, lane);
-        if (lane == 0) kept_s[wv] = kept;
+        const int kept = S.n < cap ? S.n : cap;
+        if (lane == 0) W.cnt[0] = (unsigned)kept;  // (the counts are spent)
         __syncthreads();
         int off = 0, tot = 0;
         for (int u = 0; u < NW; ++u) {
-            const int k = kept_s[u];
+            const int k = (int)L[u].cnt[0];
             off += u < wv ? k : 0;
             tot += k;
         }
         const long obase = A.list_off[b] - A.list_base;  // relative to this chunk's list buffer
+        const int* from = S.n < cap ? wc_fill_pos(W) : so;
         for (int sl = lane; sl < kept; sl += 64) {
-            const int o = so[sl];
-            const Cand c = eval_rec(A, load_obs(A, o), o, ri, rj, rz);
-            A.loc_idx[obase + off + sl] = o;
-            A.loc_rho[obase + off + sl] = c.rho;
+            const int p = from[sl];
+            A.loc_idx[obase + off + sl] = A.bo[p];
+            A.loc_rho[obase + off + sl] = eval_rec(A, load_rec(p), p, ri, rj, rz).rho;
         }
         if (threadIdx.x == 0) {
             A.loc_off[b] = obase;
@@ -1132,8 +1350,8 @@ __global__ void reg_bucket_count(const int* cellcum, const int* obkt, int ncell,
 
 __global__ void reg_bucket_scatter(const int* cellcum, const double* ori, const double* orj,
                                    const double* oz, const double* oerr, const int* obkt,
-                                   int ncell, int nbkt, const int* bcc, double* brec, int* bo,
-                                   unsigned long long* err2_min)
+                                   int ncell, int nbkt, const int* bcc, double* brec,
+                                   float4* brf, int* bo, unsigned long long* err2_min)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= ncell) return;
@@ -1155,6 +1373,8 @@ __global__ void reg_bucket_scatter(const int* cellcum, const double* ori, const 
         r[1] = orj[i];
         r[2] = oz[i];
         r[3] = oerr[i];
+        brf[p] = make_float4((float)ori[i], (float)orj[i], (float)oz[i],
+                             (float)log2(rn_mul(oerr[i], oerr[i])));
         bo[p] = i;
         // err^2 >= 0: its bits order as the values do
         const unsigned long long b2 = (unsigned long long)__double_as_longlong(rn_mul(oerr[i], oerr[i]));
@@ -1202,9 +1422,13 @@ __global__ __launch_bounds__(64) void list_cap_wave(ListCapArgs A)
                 const double rc = rn;
                 const int i = i0 + lane;
                 rn = i + 64 < n ? ir[i + 64] : 0.0;
-                wc_push(L, so, S, i < n, rho_key(rc), i, A.cap, lane);
+                wc_push(L, S, i < n && rho_key(rc) < S.tau, i, A.cap, lane);
+                wc_service(L, so, S, A.cap, lane, i0 + 64 >= n, [&](int p, bool& ok) {
+                    ok = true;
+                    return rho_key(ir[p]);
+                });
             }
-            kept = wc_finish(L, so, S, A.cap, lane);
+            kept = A.cap;
             for (int sl = lane; sl < kept; sl += 64) {
                 const int i = so[sl];
                 A.out_idx[ob + sl] = ii[i];
@@ -1424,6 +1648,11 @@ long lekf_reg_wave_slots_max()
     return 16L * (ncu > 0 ? ncu : 256);
 }
 
+// Workgroups of `lds` bytes that a CU holds: 160 KB in granules of 1280 bytes (the
+// occupancy query counts bytes, and a persistent workgroup too many waits for a whole
+// one to end, which nearly doubles the launch)
+static constexpr int lds_fit(size_t lds) { return (int)(128 / ((lds + 1279) / 1280)); }
+
 hipError_t lekf_list_cap_launch(const ListCapArgs& A, int nslots, hipStream_t st)
 {
     const long npt = (long)A.ncols * A.nlev;
@@ -1435,6 +1664,7 @@ hipError_t lekf_list_cap_launch(const ListCapArgs& A, int nslots, hipStream_t st
         if (hipGetDevice(&dev) == hipSuccess)
             (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, list_cap_wave, 64, 0);
+        per_cu = std::min(per_cu, lds_fit(sizeof(WaveCap) + sizeof(int) * LEKF_CAP_LDS));
         long g = (long)(per_cu > 0 ? per_cu : 1) * (ncu > 0 ? ncu : 256);
         if (g > npt) g = npt;
         hipLaunchKernelGGL(list_cap_wave, dim3((unsigned)g), dim3(64), 0, st, A);
@@ -1453,6 +1683,7 @@ static hipError_t launch_select_wave(const RegionalArgs& A, long npt, hipStream_
     if (hipGetDevice(&dev) == hipSuccess)
         (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
     (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reg_select_wave<NW>, 64 * NW, 0);
+    per_cu = std::min(per_cu, lds_fit(NW * sizeof(WaveCap)));
     long g = (long)(per_cu > 0 ? per_cu : 1) * (ncu > 0 ? ncu : 256);
     if (g * NW > A.wc_so_waves) g = A.wc_so_waves / NW;  // one slot map per wave
     if (g > npt) g = npt;
@@ -1480,7 +1711,7 @@ hipError_t lekf_reg_select_launch(const RegionalArgs& A, long npt, int nslots, h
 }
 
 hipError_t lekf_reg_buckets_launch(const RegObsArgs& A, int nbinned, const int* cellcum, int nbkt,
-                                   int* bcnt, int* bcc, double* brec, int* bo,
+                                   int* bcnt, int* bcc, double* brec, float4* brf, int* bo,
                                    unsigned long long* err2_min, hipStream_t st)
 {
     (void)nbinned;
@@ -1493,6 +1724,6 @@ hipError_t lekf_reg_buckets_launch(const RegObsArgs& A, int nbinned, const int* 
         hipLaunchKernelGGL(scan_inclusive_int, dim3(1), dim3(1024), 0, st, bcnt + (size_t)t * ncell,
                            bcc + (size_t)t * ncell, ncell);
     hipLaunchKernelGGL(reg_bucket_scatter, dim3(nb), dim3(256), 0, st, cellcum, A.o_ri, A.o_rj,
-                       A.o_z, A.o_err, A.o_bkt, ncell, nbkt, bcc, brec, bo, err2_min);
+                       A.o_z, A.o_err, A.o_bkt, ncell, nbkt, bcc, brec, brf, bo, err2_min);
     return hipGetLastError();
 }

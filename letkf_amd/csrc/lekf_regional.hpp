@@ -39,10 +39,11 @@ struct RegionalArgs {
     // aligned); bo = the obs's position in the sorted order
     const int* bcc;
     const double* brec;
+    const float4* brf;                      // in FP32: (ri, rj, z, log2 err^2)
     const int* bo;
     // per bucket, the smallest err^2 of its obs (double bits)
     const unsigned long long* err2_min;
-    // the fused selection's slot -> obs map, LEKF_CAP_LDS ints per wave, for
+    // the fused selection's slot -> position map, LEKF_CAP_LDS ints per wave, for
     // wc_so_waves waves (the launch holds no more waves than that)
     int* wc_so;
     long wc_so_waves;
@@ -96,7 +97,7 @@ hipError_t lekf_reg_keys_launch(const RegObsArgs& A, hipStream_t st);
 // the bucket-by-bucket copy of the sorted obs (RegionalArgs bcc, bri .. bo):
 // bcnt (nbkt * ncell ints) is work space
 hipError_t lekf_reg_buckets_launch(const RegObsArgs& A, int nbinned, const int* cellcum, int nbkt,
-                                   int* bcnt, int* bcc, double* brec, int* bo,
+                                   int* bcnt, int* bcc, double* brec, float4* brf, int* bo,
                                    unsigned long long* err2_min, hipStream_t st);
 // the capped selection keeps its kept sets in LDS, one wave per bucket
 inline bool lekf_reg_select_fused(int nobs_max) { return nobs_max > 0 && nobs_max <= LEKF_CAP_LDS; }

@@ -23,7 +23,7 @@ FSRC = os.path.join(HERE, "fortran")
 LIB = os.path.join(HERE, "liblekf_hip.so")
 FLIB = os.path.join(FSRC, "liblekf_fortran.so")
 
-HIP_SOURCES = ["lekf_solve.hip", "lekf_trf.hip", "lekf_cull.hip", "lekf_obsope.hip", "lekf_regional.hip",
+HIP_SOURCES = ["lekf_solve.hip", "lekf_gram.hip", "lekf_trf.hip", "lekf_cull.hip", "lekf_obsope.hip", "lekf_regional.hip",
                "lekf_relax.hip", "lekf_l96.hip", "lekf_radar.hip", "lekf_capi.hip"]
 F_SOURCES = ["common_letkf.f90", "letkf_tools_gpu.f90", "letkf_speedy_gpu.f90"]
 

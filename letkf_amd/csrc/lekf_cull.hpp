@@ -79,7 +79,6 @@ hipError_t lekf_logpfm_launch(const double* x2b, int nij, int nv2d, int ips, int
 // solve (lekf_solve.hip)
 size_t lekf_solve_lds_bytes(int k, int nvmax);
 size_t lekf_solve_ws_bytes(long npt, int kmax, int outs);
-int lekf_solve_nt(int k);
 int lekf_solve_class(int k);
 hipError_t lekf_solve_launch(const LekfJob* djobs, int njobs, long npt, int kmax, int nvmax,
                              int mode, int outs, void* ws, size_t ws_bytes, hipStream_t st);

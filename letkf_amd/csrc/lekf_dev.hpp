@@ -83,6 +83,24 @@ __device__ __forceinline__ double rsq_nr(double x)
     return r;
 }
 
+// Pointers to device memory as such: a pointer read from a job descriptor is otherwise
+// loaded through with flat accesses, and read again at every use.
+template <class T>
+using gptr = const __attribute__((address_space(1))) T*;
+
+// a value that is the same in every lane, in scalar registers
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long x)
+{
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)x);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(x >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+template <class T>
+__device__ __forceinline__ gptr<T> uniform_ptr(const T* p)
+{
+    return (gptr<T>)uniform64((unsigned long long)p);
+}
+
 // Jacobi: rotate a pair while |a_pq| > tol * sqrt(a_pp a_qq); stop after a
 // sweep with no rotation.
 #define LEKF_JACOBI_TOL 1.0e-15

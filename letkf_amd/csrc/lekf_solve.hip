@@ -35,6 +35,7 @@
 #include "lekf_dev.hpp"
 #include "lekf_tune.hpp"
 #include "lekf_ktime.hpp"
+#include "lekf_gram.hpp"
 #include "lekf_split.hpp"
 
 namespace {
@@ -46,271 +47,6 @@ __device__ __forceinline__ double lane_bcast(double x, int src)
     const int lo = __builtin_amdgcn_readlane((int)b, src);
     const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// ---------------------------------------------------------------------------
-// Gram products.  Lane l holds A[i = l%16][kk = l/16] and B[kk][j = l%16] of
-// each 16x16x4 step (16x16x32 BF16: kk = 8*(l/16) .. +7).
-//
-// The local list is read in chunks of 64 entries: lane l loads entry q0 + l
-// (obs index, weight rho/rdiag, departure) with one coalesced access, and the
-// MFMA steps of the chunk take them from the owning lanes by shuffles.  All
-// gathers of the chunk's Y rows are then independent loads, issued together,
-// instead of one dependent index -> row chain per step.  Wave wv of nw takes
-// every nw-th chunk.
-// ---------------------------------------------------------------------------
-struct ObsChunk {
-    int o;       // obs index (0 when past the end: a valid row, weighted 0)
-    double w;    // rho / rdiag (1 / rdiag with rdiag_wloc), 0 past the end
-    double d;    // departure
-};
-
-__device__ __forceinline__ ObsChunk stage_chunk(const LekfJob& J, long off, int p, int q0,
-                                                int lane, bool wloc, double& p3)
-{
-    ObsChunk c{0, 0.0, 0.0};
-    const int q = q0 + lane;
-    if (q < p) {
-        c.o = J.loc_idx[off + q];
-        const double rho = J.loc_rho[off + q];
-        const double rd = J.loc_rdiag ? J.loc_rdiag[off + q] : J.rdiag[c.o];
-        c.w = (wloc ? 1.0 : rho) / rd;
-        c.d = J.dep[c.o];
-        p3 += rho;
-    }
-    return c;
-}
-
-template <int NT>
-__device__ __forceinline__ void gram_f64(const LekfJob& J, long off, int p, int k, int lane,
-                                         lekf_d4* acc, double& p3, int wv, int nw)
-{
-    // 4-obs steps whose rows are gathered at once (bounded by the registers
-    // the rows and the NT (NT + 1) / 2 accumulator tiles take)
-    constexpr int SUB = NT == 1 ? 16 : NT == 2 ? 8 : NT == 3 ? 4 : NT == 4 ? 2 : 1;
-    const int lr = lane & 15, kq = lane >> 4;
-    const bool wloc = (J.flags & LEKF_F_WLOC) != 0;
-    for (int q0 = 64 * wv; q0 < p; q0 += 64 * nw) {
-        const ObsChunk ch = stage_chunk(J, off, p, q0, lane, wloc, p3);
-#pragma unroll 1
-        for (int h = 0; h < 16 && q0 + 4 * h < p; h += SUB) {
-            double v[SUB][NT], wt[SUB];
-#pragma unroll
-            for (int st = 0; st < SUB; ++st) {
-                const int src = 4 * (h + st) + kq;
-                const int o = __shfl(ch.o, src, 64);
-                const double w = __shfl(ch.w, src, 64);
-                const double dd = __shfl(ch.d, src, 64);
-                wt[st] = w;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const int c = 16 * t + lr;
-                    double x = 0.0;
-                    if (c < k)
-                        x = J.hdxf[(long)o * J.y_so + (long)c * J.y_sm];
-                    else if (c == k)
-                        x = dd;
-                    v[st][t] = x;
-                }
-            }
-#pragma unroll
-            for (int st = 0; st < SUB; ++st) {
-                int a = 0;
-#pragma unroll
-                for (int I = 0; I < NT; ++I) {
-                    const double ai = wt[st] * v[st][I];
-#pragma unroll
-                    for (int Jt = I; Jt < NT; ++Jt) {
-                        acc[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, v[st][Jt], acc[a], 0, 0, 0);
-                        ++a;
-                    }
-                }
-            }
-        }
-    }
-}
-
-// Mixed form: Y from the FP32 table, products accumulated in FP32 on MFMA.
-// FP32: v_mfma_f32_16x16x4f32 (operands rounded to FP32).
-// BF16x3: each FP32 operand split x = h + l (h = bf16(x), l = bf16(x - h));
-// A*B ~ Ah*Bh + Ah*Bl + Al*Bh on v_mfma_f32_16x16x32_bf16.
-// FP32 form: the FP32 accumulators are added into FP64 ones (accd) after each
-// chunk of 64 obs, so no FP32 sum runs over more than 64 products and the
-// rounding of long local lists (p ~ 10^3) does not build up.  The BF16x3 form
-// keeps FP32 accumulation: its two-term split carries about 16 significant
-// bits, which dominates its error, and the FP64 accumulators would cost it
-// occupancy.
-template <int NT>
-__device__ __forceinline__ void mix_flush(lekf_f4* acc, lekf_d4* accd)
-{
-#pragma unroll
-    for (int a = 0; a < NT * (NT + 1) / 2; ++a) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) accd[a][r] += (double)acc[a][r];
-        acc[a] = lekf_f4{0.f, 0.f, 0.f, 0.f};
-    }
-}
-
-template <int NT>
-__device__ __forceinline__ void gram_f32(const LekfJob& J, long off, int p, int k, int lane,
-                                         lekf_f4* acc, lekf_d4* accd, double& p3, int wv, int nw)
-{
-    constexpr int SUB = NT == 1 ? 16 : NT == 2 ? 8 : NT == 3 ? 4 : NT == 4 ? 2 : 1;
-    const int lr = lane & 15, kq = lane >> 4;
-    const bool wloc = (J.flags & LEKF_F_WLOC) != 0;
-    for (int q0 = 64 * wv; q0 < p; q0 += 64 * nw) {
-        const ObsChunk ch = stage_chunk(J, off, p, q0, lane, wloc, p3);
-        const float wf = (float)ch.w, df = (float)ch.d;  // one dword each across lanes
-#pragma unroll 1
-        for (int h = 0; h < 16 && q0 + 4 * h < p; h += SUB) {
-            float v[SUB][NT], wt[SUB];
-#pragma unroll
-            for (int st = 0; st < SUB; ++st) {
-                const int src = 4 * (h + st) + kq;
-                const int o = __shfl(ch.o, src, 64);
-                const float w = __shfl(wf, src, 64);
-                const float dd = __shfl(df, src, 64);
-                wt[st] = w;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const int c = 16 * t + lr;
-                    float x = 0.0f;
-                    if (c < k)
-                        x = J.hdxf32[(long)o * k + c];
-                    else if (c == k)
-                        x = dd;
-                    v[st][t] = x;
-                }
-            }
-#pragma unroll
-            for (int st = 0; st < SUB; ++st) {
-                int a = 0;
-#pragma unroll
-                for (int I = 0; I < NT; ++I) {
-                    const float ai = wt[st] * v[st][I];
-#pragma unroll
-                    for (int Jt = I; Jt < NT; ++Jt) {
-                        acc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai, v[st][Jt], acc[a], 0, 0, 0);
-                        ++a;
-                    }
-                }
-            }
-        }
-        mix_flush<NT>(acc, accd);
-    }
-}
-
-// Split-BF16x3: K = 32 obs per MFMA step, two steps per chunk.  Lane l
-// supplies 8 consecutive k values (kk = 8*(l/16) .. +7) of row/col l%16.
-template <int NT>
-__device__ __forceinline__ void gram_bf16x3(const LekfJob& J, long off, int p, int k, int lane,
-                                            lekf_f4* acc, double& p3, int wv, int nw)
-{
-    const int lr = lane & 15, kq = lane >> 4;
-    const bool wloc = (J.flags & LEKF_F_WLOC) != 0;
-    for (int q0 = 64 * wv; q0 < p; q0 += 64 * nw) {
-        const ObsChunk ch = stage_chunk(J, off, p, q0, lane, wloc, p3);
-        // the weight and departure in the precision the products use, so each
-        // crosses lanes as one dword
-        const float wf = (float)ch.w, df = (float)ch.d;
-        for (int h = 0; h < 64 && q0 + h < p; h += 32) {
-            lekf_bf8 ah[NT], al[NT], bh[NT], bl[NT];
-            float wv8[8], dv8[8];
-            int ov[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int src = h + 8 * kq + e;
-                ov[e] = __shfl(ch.o, src, 64);
-                wv8[e] = __shfl(wf, src, 64);
-                dv8[e] = __shfl(df, src, 64);
-            }
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const int c = 16 * t + lr;
-                float x[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    x[e] = 0.0f;
-                    if (c < k)
-                        x[e] = J.hdxf32[(long)ov[e] * k + c];
-                    else if (c == k)
-                        x[e] = dv8[e];
-                }
-                // two elements per rounding instruction (round to nearest even,
-                // as the scalar conversion does)
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    const lekf_f2v xv = {x[e], x[e + 1]};
-                    const lekf_f2v xa = {wv8[e] * x[e], wv8[e + 1] * x[e + 1]};
-                    const lekf_b2v hb = __builtin_convertvector(xv, lekf_b2v);
-                    const lekf_b2v ha = __builtin_convertvector(xa, lekf_b2v);
-                    const lekf_f2v rb = {x[e] - (float)hb.x, x[e + 1] - (float)hb.y};
-                    const lekf_f2v ra = {xa.x - (float)ha.x, xa.y - (float)ha.y};
-                    const lekf_b2v lb = __builtin_convertvector(rb, lekf_b2v);
-                    const lekf_b2v la = __builtin_convertvector(ra, lekf_b2v);
-                    bh[t][e] = hb.x;
-                    bh[t][e + 1] = hb.y;
-                    bl[t][e] = lb.x;
-                    bl[t][e + 1] = lb.y;
-                    ah[t][e] = ha.x;
-                    ah[t][e + 1] = ha.y;
-                    al[t][e] = la.x;
-                    al[t][e + 1] = la.y;
-                }
-            }
-            int a = 0;
-#pragma unroll
-            for (int I = 0; I < NT; ++I) {
-#pragma unroll
-                for (int Jt = I; Jt < NT; ++Jt) {
-                    acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[I], bh[Jt], acc[a], 0, 0, 0);
-                    acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[I], bl[Jt], acc[a], 0, 0, 0);
-                    acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[I], bh[Jt], acc[a], 0, 0, 0);
-                    ++a;
-                }
-            }
-        }
-    }
-}
-
-// Write the upper tiles of G into LDS: C (k x k at A, leading dimension lda,
-// exactly symmetric), b and sum w d^2; with add, accumulate onto what an
-// earlier wave stored.  Only (row <= col) elements are taken so C is
-// symmetric bit for bit.  Result-tile layouts (measured on gfx950): the FP64
-// 16x16x4 MFMA puts element (row = l/16 + 4r, col = l%16) in register r of
-// lane l; the FP32 and BF16 16x16 forms put (row = 4*(l/16) + r, col = l%16)
-// there.
-template <int NT, bool F64, typename ACC>
-__device__ __forceinline__ void store_gram(const ACC* acc, int k, int lda, int lane, double* A,
-                                           double* B, double* sumwd2, bool add)
-{
-    const int lr = lane & 15, kq = lane >> 4;
-    int a = 0;
-#pragma unroll
-    for (int I = 0; I < NT; ++I) {
-#pragma unroll
-        for (int Jt = I; Jt < NT; ++Jt) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 16 * I + (F64 ? kq + 4 * r : 4 * kq + r);
-                const int col = 16 * Jt + lr;
-                const double val = (double)acc[a][r];
-                if (row <= col) {
-                    if (col < k) {
-                        const double v = add ? A[row * lda + col] + val : val;
-                        A[row * lda + col] = v;
-                        A[col * lda + row] = v;
-                    } else if (col == k) {
-                        if (row < k)
-                            B[row] = add ? B[row] + val : val;
-                        else
-                            *sumwd2 = add ? *sumwd2 + val : val;
-                    }
-                }
-            }
-            ++a;
-        }
-    }
 }
 
 // ===========================================================================
@@ -411,7 +147,7 @@ __device__ __forceinline__ void fused_gram(const LekfJob& J, int b, SolveLds& L,
             lekf_d4 acc[NT * (NT + 1) / 2];
 #pragma unroll
             for (int a = 0; a < NT * (NT + 1) / 2; ++a) acc[a] = lekf_d4{0.0, 0.0, 0.0, 0.0};
-            gram_f64<NT>(J, off, p, k, lane, acc, p3, 0, 1);
+            gram_f64<NT>(gram_in(J, off, p), lane, acc, p3, 0, 1);
             store_gram<NT, true>(acc, k, lda, lane, L.A, L.B, &L.sc[0], false);
         } else {
             lekf_f4 acc[NT * (NT + 1) / 2];
@@ -421,10 +157,10 @@ __device__ __forceinline__ void fused_gram(const LekfJob& J, int b, SolveLds& L,
                 lekf_d4 accd[NT * (NT + 1) / 2];
 #pragma unroll
                 for (int a = 0; a < NT * (NT + 1) / 2; ++a) accd[a] = lekf_d4{0.0, 0.0, 0.0, 0.0};
-                gram_f32<NT>(J, off, p, k, lane, acc, accd, p3, 0, 1);
+                gram_f32<NT>(gram_in(J, off, p), lane, acc, accd, p3, 0, 1);
                 store_gram<NT, false>(accd, k, lda, lane, L.A, L.B, &L.sc[0], false);
             } else {
-                gram_bf16x3<NT>(J, off, p, k, lane, acc, p3, 0, 1);
+                gram_bf16x3<NT>(gram_in(J, off, p), lane, acc, p3, 0, 1);
                 store_gram<NT, false>(acc, k, lda, lane, L.A, L.B, &L.sc[0], false);
             }
         }
@@ -775,91 +511,6 @@ void lekf_solve_kernel(const LekfJob* __restrict__ jobs, int njobs, long npt, in
 // ===========================================================================
 // 32 < k <= LEKF_KMAX: Gram kernel + eigen/assembly/apply kernel
 // ===========================================================================
-
-// Waves per SIMD asked of the Gram kernel: the FP64 and FP32 forms with
-// 4 x 4 tiles (49 <= k <= 64) take 214 and 188 registers, two waves per
-// SIMD, unless held to three's budget (which they fit without spilling)
-constexpr int gram_waves_per_simd(int nt, int mode)
-{
-    return (nt == 4 && mode != 2) ? 3 : (nt == 3 && mode != 2) ? 4 : 1;
-}
-
-// W waves per point; wave w takes every W-th chunk of 64 local obs, and the
-// partial Grams are summed in LDS in wave order (deterministic for a given W).
-template <int NT, int MODE, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(gram_waves_per_simd(NT, MODE))))
-void lekf_gram_kernel(
-    const LekfJob* __restrict__ jobs, int njobs, long gp0, double* __restrict__ ws, long gstride,
-    const int* __restrict__ rlist, int* __restrict__ zlist)
-{
-    extern __shared__ double smem[];
-    const long slot = blockIdx.x;
-    // the launch's first sub-batch empties the redo list before any kernel adds to it
-    if (zlist && blockIdx.x == 0 && threadIdx.x == 0) zlist[0] = 0;
-    long gp = gp0 + slot;
-    if (rlist) {  // FP64 pass of a split launch: slot i holds the redo list's i-th point
-        if (slot >= rlist[0]) return;
-        gp = rlist[1 + slot];
-    }
-    const int tid = threadIdx.x;
-    const int lane = tid & (LEKF_WAVE - 1), wv = tid / LEKF_WAVE;
-    const int ji = lekf_job_of(jobs, njobs, gp);
-    const LekfJob& J = jobs[ji];
-    const int b = (int)(gp - J.pt_begin + J.pt0);
-    const int k = J.k, lda = k + 1;
-    const long off = J.loc_off[b];
-    const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - off);
-    if (p <= 0) return;
-    double* A = smem;
-    double* B = A + (size_t)k * lda;
-    double* sc = B + k;  // [0] sum w d^2, [4 + w] P3 of wave w (4 + W slots)
-    double p3 = 0.0;
-    if (MODE == 0) {
-        lekf_d4 acc[NT * (NT + 1) / 2];
-#pragma unroll
-        for (int a = 0; a < NT * (NT + 1) / 2; ++a) acc[a] = lekf_d4{0.0, 0.0, 0.0, 0.0};
-        gram_f64<NT>(J, off, p, k, lane, acc, p3, wv, W);
-        for (int w = 0; w < W; ++w) {
-            if (wv == w) store_gram<NT, true>(acc, k, lda, lane, A, B, &sc[0], w > 0);
-            __syncthreads();
-        }
-    } else {
-        lekf_f4 acc[NT * (NT + 1) / 2];
-#pragma unroll
-        for (int a = 0; a < NT * (NT + 1) / 2; ++a) acc[a] = lekf_f4{0.f, 0.f, 0.f, 0.f};
-        if (MODE == 1) {
-            lekf_d4 accd[NT * (NT + 1) / 2];
-#pragma unroll
-            for (int a = 0; a < NT * (NT + 1) / 2; ++a) accd[a] = lekf_d4{0.0, 0.0, 0.0, 0.0};
-            gram_f32<NT>(J, off, p, k, lane, acc, accd, p3, wv, W);
-            for (int w = 0; w < W; ++w) {
-                if (wv == w) store_gram<NT, false>(accd, k, lda, lane, A, B, &sc[0], w > 0);
-                __syncthreads();
-            }
-        } else {
-            gram_bf16x3<NT>(J, off, p, k, lane, acc, p3, wv, W);
-            for (int w = 0; w < W; ++w) {
-                if (wv == w) store_gram<NT, false>(acc, k, lda, lane, A, B, &sc[0], w > 0);
-                __syncthreads();
-            }
-        }
-    }
-    p3 = wave_sum(p3);
-    if (lane == 0) sc[4 + wv] = p3;
-    __syncthreads();
-    double* out = ws + slot * gstride;
-    for (int t = tid; t < k * k; t += 64 * W) {
-        const int i = t / k, j = t - i * k;
-        out[t] = A[i * lda + j];
-    }
-    for (int i = tid; i < k; i += 64 * W) out[(size_t)k * k + i] = B[i];
-    if (tid == 0) {
-        double s = sc[4];
-        for (int w = 1; w < W; ++w) s += sc[4 + w];
-        out[(size_t)k * k + k] = sc[0];
-        out[(size_t)k * k + k + 1] = s;
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Block Gram for LEKF_KSPLIT < k <= LEKF_KMAX: the augmented (k+1)^2 Gram is
@@ -3252,11 +2903,9 @@ __global__ __launch_bounds__(64) void lekf_big_kernel(const LekfJob* __restrict_
 // ---------------------------------------------------------------------------
 // host-side launchers (called from lekf_capi.hip)
 // ---------------------------------------------------------------------------
-int lekf_solve_nt(int k) { return (k + 1 + 15) / 16; }
-
 // Kernel class of an ensemble size: KR * 8 + NT for k <= 32 (register
-// Jacobi, KR = k rounded up to a multiple of 4); NT for k <= LEKF_KSPLIT;
-// kClassBig above (block Gram + eigensolver in global memory).
+// Jacobi, KR = k rounded up to a multiple of 4); the Gram's column tiles and strips for
+// k <= LEKF_KSPLIT; kClassBig above (block Gram + eigensolver in global memory).
 constexpr int kClassBig = 1000;
 
 int lekf_solve_class(int k)
@@ -3267,7 +2916,8 @@ int lekf_solve_class(int k)
         return kr * 8 + nt;
     }
     if (k > LEKF_KSPLIT) return kClassBig;
-    return lekf_solve_nt(k);
+    // every job of a launch has the same cut of the Gram's columns
+    return 500 + 8 * gram_ntf(k) + gram_ns(k);
 }
 
 // points per wave of the fused kernel for Jacobi rows KR: lane groups of KR,
@@ -3450,27 +3100,10 @@ static hipError_t launch_fix(int kr, long nb, size_t elds, hipStream_t st, const
     return hipGetLastError();
 }
 
-template <int NT, int MODE>
-static hipError_t launch_gram(int W, long nb, size_t glds, hipStream_t st, const LekfJob* djobs,
-                              int njobs, long g0, double* ws, long gs, const int* rlist,
-                              int* zlist)
-{
-    KTime kt(rlist ? "redo_gram" : "gram", st);
-    if (W == 2)
-        hipLaunchKernelGGL((lekf_gram_kernel<NT, MODE, 2>), dim3((unsigned)nb), dim3(128), glds, st,
-                           djobs, njobs, g0, ws, gs, rlist, zlist);
-    else if (W == 8)
-        hipLaunchKernelGGL((lekf_gram_kernel<NT, MODE, 8>), dim3((unsigned)nb), dim3(512), glds, st,
-                           djobs, njobs, g0, ws, gs, rlist, zlist);
-    else
-        hipLaunchKernelGGL((lekf_gram_kernel<NT, MODE, 4>), dim3((unsigned)nb), dim3(256), glds, st,
-                           djobs, njobs, g0, ws, gs, rlist, zlist);
-    return hipGetLastError();
-}
-
-template <int NT, int MODE>
+template <int MODE>
 static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int kmax, int nvmax,
-                               int outs, void* ws, size_t ws_bytes, hipStream_t st)
+                               int outs, void* ws, size_t ws_bytes,
+                               hipStream_t st)
 {
     const SplitPlan plan = split_plan(kmax, outs);
     const long gs = split_rec_stride(kmax, plan);
@@ -3482,7 +3115,6 @@ static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int km
     int* rlist = (int*)(ridx + (plan.streams ? (size_t)per * split_ridx_stride(kmax) : 0));
     const int W = g_lekf_tune.gram_waves;
     const int kr = eig_kr(kmax);
-    const size_t glds = ((size_t)kmax * (kmax + 1) + kmax + 4 + W) * sizeof(double);
     const size_t elds = eig_lds_doubles(kmax, nvmax) * sizeof(double);
     // mixed forms on the split eigensolver: the points whose C is worse conditioned
     // than kthr are listed (up to one sub-batch of them per launch), and after the
@@ -3511,16 +3143,16 @@ static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int km
     };
     for (long g0 = 0; g0 < npt; g0 += per) {
         const long nb = per < npt - g0 ? per : npt - g0;
-        hipError_t e = launch_gram<NT, MODE>(W, nb, glds, st, djobs, njobs, g0, (double*)ws, gs,
-                                             nullptr, g0 == 0 ? rlist : nullptr);
+        hipError_t e = lekf_gram_launch(MODE, W, kmax, nb, st, djobs, njobs, g0, (double*)ws, gs,
+                                        nullptr, g0 == 0 ? rlist : nullptr);
         if (e == hipSuccess) e = solve(g0, nb, 0, kthr);
         if (e != hipSuccess) return e;
     }
     if (kthr > 0.0) {
         // grids of one sub-batch; the slots past the list's length return at once
         const long nl = per < npt ? per : npt;
-        hipError_t e = launch_gram<NT, 0>(W, nl, glds, st, djobs, njobs, 0, (double*)ws, gs, rlist,
-                                          nullptr);
+        hipError_t e = lekf_gram_launch(0, W, kmax, nl, st, djobs, njobs, 0, (double*)ws, gs, rlist,
+                                        nullptr);
         if (e == hipSuccess) e = solve(0, nl, 1, 0.0);
         if (e != hipSuccess) return e;
     }
@@ -3565,12 +3197,11 @@ static hipError_t launch_mode(int cls, const LekfJob* djobs, int njobs, long npt
     case 24 * 8 + 2: return launch_fused<2, 24, MODE>(djobs, njobs, npt, kmax, nvmax, st);
     case 28 * 8 + 2: return launch_fused<2, 28, MODE>(djobs, njobs, npt, kmax, nvmax, st);
     case 32 * 8 + 3: return launch_fused<3, 32, MODE>(djobs, njobs, npt, kmax, nvmax, st);
-    case 3: return launch_split<3, MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
-    case 4: return launch_split<4, MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
-    case 5: return launch_split<5, MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
-    case 6: return launch_split<6, MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
     case kClassBig: return launch_big<MODE>(djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
-    default: return hipErrorInvalidValue;
+    default:
+        if (kmax > 32 && kmax <= LEKF_KSPLIT)
+            return launch_split<MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
+        return hipErrorInvalidValue;
     }
 }
 
@@ -3580,7 +3211,8 @@ static hipError_t launch_mode(int cls, const LekfJob* djobs, int njobs, long npt
 // of them outputs trans or pao, and whether any does not; ws is the Gram workspace
 // of lekf_solve_ws_bytes(npt, kmax, outs) bytes (k > 32).
 hipError_t lekf_solve_launch(const LekfJob* djobs, int njobs, long npt, int kmax, int nvmax,
-                             int mode, int outs, void* ws, size_t ws_bytes, hipStream_t st)
+                             int mode, int outs, void* ws, size_t ws_bytes,
+                             hipStream_t st)
 {
     if (npt <= 0) return hipSuccess;
     if (nvmax > LEKF_NVMAX) return hipErrorInvalidValue;

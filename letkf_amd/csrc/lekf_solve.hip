@@ -25,9 +25,11 @@
 //     method of EISPACK tred2/tql2, the reference's own eigensolver), assembly
 //     of W and the apply, with the matrix in registers (k <= 64) or LDS.
 //   * LEKF_KSPLIT < k <= LEKF_KMAX: a block Gram kernel (one wave per 64 x 64
-//     block of a point) writes the same workspace record, and the eigen
-//     kernel runs the same steps with the matrix left in that record in
-//     global memory (a k = 256 FP64 matrix is 512 KB, beyond the LDS).
+//     block of a point) writes the same workspace record, and the matrix stays
+//     there in global memory (a k = 256 FP64 matrix is 512 KB, beyond the LDS).
+//     Jobs without trans and pao: four waves per point, tridiagonalisation and
+//     the rational form of its functions (lekf_bigvec_kernel); the others the
+//     eigen kernel's steps, one wave per point (lekf_big_kernel).
 // A point's arithmetic depends only on its own data, so its result is the
 // same whatever else shares the launch.
 #include <algorithm>
@@ -37,6 +39,7 @@
 #include "lekf_ktime.hpp"
 #include "lekf_gram.hpp"
 #include "lekf_split.hpp"
+#include "lekf_trf.hpp"
 
 namespace {
 
@@ -563,7 +566,7 @@ __device__ __forceinline__ bool big_dual(const LekfJob& J, int p, int k)
 
 // One upper 64 x 64 block of G (p x p, row-major at out) over the k members.
 template <int MODE>
-__device__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk, double* out,
+__device__ __forceinline__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk, double* out,
                               int lane)
 {
     constexpr int NB = kBlkNB;
@@ -572,6 +575,10 @@ __device__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk
     int bi, bj;
     blk_pair(tblk, nbp, bi, bj);
     const int cI = 16 * NB * bi, cJ = 16 * NB * bj;
+    // tiles with columns of the product in them, on or above its diagonal
+    const bool diag = bi == bj;
+    const int nI = (p - cI + 15) / 16, nJ = (p - cJ + 15) / 16;
+    auto live = [&](int I, int Jt) { return I < nI && Jt < nJ && (!diag || I <= Jt); };
     const int lr = lane & 15, kq = lane >> 4;
     const bool wloc = (J.flags & LEKF_F_WLOC) != 0;
     long orow[NB], ocol[NB];
@@ -614,7 +621,8 @@ __device__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk
             for (int I = 0; I < NB; ++I)
 #pragma unroll
                 for (int Jt = 0; Jt < NB; ++Jt)
-                    acc[I][Jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(xr[I], xc[Jt], acc[I][Jt], 0, 0, 0);
+                    if (live(I, Jt))
+                        acc[I][Jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(xr[I], xc[Jt], acc[I][Jt], 0, 0, 0);
         }
 #pragma unroll
         for (int I = 0; I < NB; ++I)
@@ -652,7 +660,8 @@ __device__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk
             for (int I = 0; I < NB; ++I)
 #pragma unroll
                 for (int Jt = 0; Jt < NB; ++Jt)
-                    acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xr[I], xc[Jt], acc[I][Jt], 0, 0, 0);
+                    if (live(I, Jt))
+                        acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xr[I], xc[Jt], acc[I][Jt], 0, 0, 0);
         }
 #pragma unroll
         for (int I = 0; I < NB; ++I)
@@ -701,6 +710,7 @@ __device__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk
             for (int I = 0; I < NB; ++I)
 #pragma unroll
                 for (int Jt = 0; Jt < NB; ++Jt) {
+                    if (!live(I, Jt)) continue;
                     acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[I], bh[Jt], acc[I][Jt], 0, 0, 0);
                     acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[I], bl[Jt], acc[I][Jt], 0, 0, 0);
                     acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[I], bh[Jt], acc[I][Jt], 0, 0, 0);
@@ -725,7 +735,7 @@ __device__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk
 // record out: [C | b | sum w d^2 | P3] (64 x 64 blocks of the augmented
 // (k+1)^2 product), or a block of G in the dual form.
 template <int MODE>
-__device__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out, int lane)
+__device__ __forceinline__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out, int lane)
 {
     constexpr int NB = kBlkNB;
     const int k = J.k;
@@ -741,6 +751,10 @@ __device__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out, i
         gram_dual_blk<MODE>(J, off, p, k, tblk, out, lane);
         return;
     }
+    // tiles with columns of the product in them, on or above its diagonal
+    const bool diag = bi == bj;
+    const int nI = (k + 1 - cI + 15) / 16, nJ = (k + 1 - cJ + 15) / 16;
+    auto live = [&](int I, int Jt) { return I < nI && Jt < nJ && (!diag || I <= Jt); };
     const int lr = lane & 15, kq = lane >> 4;
     const bool wloc = (J.flags & LEKF_F_WLOC) != 0;
     double p3 = 0.0;
@@ -779,7 +793,8 @@ __device__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out, i
             for (int I = 0; I < NB; ++I)
 #pragma unroll
                 for (int Jt = 0; Jt < NB; ++Jt)
-                    acc[I][Jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(xr[I], xc[Jt], acc[I][Jt], 0, 0, 0);
+                    if (live(I, Jt))
+                        acc[I][Jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(xr[I], xc[Jt], acc[I][Jt], 0, 0, 0);
         }
 #pragma unroll
         for (int I = 0; I < NB; ++I)
@@ -823,7 +838,8 @@ __device__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out, i
             for (int I = 0; I < NB; ++I)
 #pragma unroll
                 for (int Jt = 0; Jt < NB; ++Jt)
-                    acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xr[I], xc[Jt], acc[I][Jt], 0, 0, 0);
+                    if (live(I, Jt))
+                        acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xr[I], xc[Jt], acc[I][Jt], 0, 0, 0);
         }
 #pragma unroll
         for (int I = 0; I < NB; ++I)
@@ -886,6 +902,7 @@ __device__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out, i
             for (int I = 0; I < NB; ++I)
 #pragma unroll
                 for (int Jt = 0; Jt < NB; ++Jt) {
+                    if (!live(I, Jt)) continue;
                     acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[I], bh[Jt], acc[I][Jt], 0, 0, 0);
                     acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[I], bl[Jt], acc[I][Jt], 0, 0, 0);
                     acc[I][Jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[I], bh[Jt], acc[I][Jt], 0, 0, 0);
@@ -906,13 +923,15 @@ __device__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out, i
     }
 }
 
+constexpr int kBigW = 4;  // waves per point of the large-k vector path
+
 // LDS of the eigen/assembly kernel (doubles)
 struct EigLds {
     double* Z;    // k x lda: C, then Householder vectors + Q, then eigenvectors (columns)
     double* d;    // k  diagonal -> eigenvalues
     double* e;    // k  sub-diagonal
     double* tau;  // k  Householder scalars
-    double* rot;  // 2k (c, s) of one QL sweep
+    double* rot;  // 2k (c, s) of one QL sweep (large k: kBigW * k, the waves' sums)
     double* B;    // k  Y^T R^-1 d
     double* U;    // k
     double* Wb;   // k  w-bar
@@ -938,7 +957,7 @@ __host__ __device__ inline size_t eig_lds_doubles(int k, int nvmax)
 // record in global memory (zg)
 __host__ __device__ inline size_t eig_lds_doubles_big(int k, int nvmax)
 {
-    return 10 * (size_t)k + 8 + 2 * (size_t)nvmax * k + 3 * (size_t)nvmax + 128;
+    return (8 + kBigW) * (size_t)k + 8 + 2 * (size_t)nvmax * k + 3 * (size_t)nvmax + 128;
 }
 
 // the split path's tridiagonalisation uses only Z, d, e, tau, vb and wb
@@ -977,7 +996,7 @@ __device__ inline EigLds eig_carve(double* s, int k, int nvmax, double* zg = nul
     L.tau = s;
     s += k;
     L.rot = s;
-    s += 2 * k;
+    s += (zg ? kBigW : 2) * k;
     L.B = s;
     s += k;
     L.U = s;
@@ -1475,42 +1494,77 @@ __device__ void big_tridiag(double* A, int n, int lda, double* d, double* e, dou
     __syncthreads();
 }
 
-// The same reduction for the vector paths, with a third of the memory
-// traffic: only the upper triangle (row c, columns >= c) is kept, and step
-// s's rank-2 update is applied during step s+1's single pass over the
-// trailing block, which also forms step s+1's product B v (p_r gets
-// A[c][r] v_c from rows c < r and the row-r sums, reduced across lanes).
-// vP, wP (pending update) and vN (current reflector) are LDS vectors of n
-// indexed absolutely.  On exit d, e, tau and the reflectors (row s,
-// columns s+1..) are as big_tridiag leaves them, the elementwise update
-// being rounded identically.
-template <int NR>
-__device__ void big_tridiag_sym(double* A, int n, int lda, double* d, double* e, double* tauv,
-                                double* vP, double* wP, double* vN, int lane)
+// LDS and global memory ordered within one wave (a wave that works alone)
+__device__ __forceinline__ void wave_sync()
 {
-    for (int r = lane; r < n; r += 64) {
-        vP[r] = 0.0;
-        wP[r] = 0.0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// a[u] summed over the wave for all u at once: lane l gets the sum of u = l % 8
+__device__ __forceinline__ double wave_sum8(const double (&a)[8], int lane)
+{
+    double h[4], q[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const double mine = (lane & 1) ? a[2 * i + 1] : a[2 * i];
+        h[i] = mine + __shfl_xor((lane & 1) ? a[2 * i] : a[2 * i + 1], 1, 64);
     }
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const double mine = (lane & 2) ? h[2 * i + 1] : h[2 * i];
+        q[i] = mine + __shfl_xor((lane & 2) ? h[2 * i] : h[2 * i + 1], 2, 64);
+    }
+    double x = (lane & 4) ? q[1] : q[0];
+    x += __shfl_xor((lane & 4) ? q[0] : q[1], 4, 64);
+#pragma unroll
+    for (int o = 8; o <= 32; o <<= 1) x += __shfl_xor(x, o, 64);
+    return x;
+}
+
+// The same reduction for the vector path, by the kBigW waves of a workgroup and with a
+// third of the memory traffic: only the upper triangle (row c, columns >= c) is kept, and
+// step s's rank-2 update is applied during step s+1's single pass over the trailing
+// block, which also forms step s+1's product B v (p_r gets A[c][r] v_c from rows c < r
+// and the row-r sums).  Lane l of every wave holds elements l, l + 64, .. of the
+// reflector v and of the pending update (vp, wp) in registers, so a row's coefficients
+// are lane reads; the waves take the rows in turns of eight and add their parts of B v
+// in LDS (red: kBigW * n), in wave order.  On exit d, e, tau and the reflectors (row s,
+// columns s+1..) are as big_tridiag leaves them, the elementwise update being rounded
+// identically.
+template <int NR>
+__device__ __forceinline__ void big_tridiag_sym(double* A, int n, int lda, double* d, double* e, double* tauv,
+                                double* red, int lane, int wv)
+{
+    double vp[NR], wp[NR], v[NR];
+#pragma unroll
+    for (int t = 0; t < NR; ++t) vp[t] = wp[t] = v[t] = 0.0;
+    // element r of a register vector, r uniform
+    auto at = [&](const double (&x)[NR], int r) -> double {
+        double y = x[0];
+#pragma unroll
+        for (int t = 1; t < NR; ++t) y = (r >> 6) == t ? x[t] : y;
+        return lane_bcast(y, r & 63);
+    };
     for (int s = 0; s + 2 < n; ++s) {
-        const int o = s + 1, m = n - o;
+        const int o = s + 1;
         // row s with the pending update: diagonal and x = A[s][o..]
-        const double vps = vP[s], wps = wP[s];
+        const double vps = at(vp, s), wps = at(wp, s);
         double* rows = A + (size_t)s * lda;
         double x[NR];
         double s2 = 0.0;
 #pragma unroll
         for (int t = 0; t < NR; ++t) {
-            const int i = lane + 64 * t, r = o + i;
+            const int r = lane + 64 * t;
             x[t] = 0.0;
-            if (i < m)
-                x[t] = rn_sub(rows[r], rn_add(rn_mul(vps, wP[r]), rn_mul(wps, vP[r])));
-            if (i > 0) s2 = fma(x[t], x[t], s2);
+            if (r >= s && r < n)
+                x[t] = rn_sub(rows[r], rn_add(rn_mul(vps, wp[t]), rn_mul(wps, vp[t])));
+            if (r > o) s2 = fma(x[t], x[t], s2);
         }
-        const double dss = rn_sub(rows[s], rn_add(rn_mul(vps, wps), rn_mul(wps, vps)));
+        const double dss = at(x, s);
         const double sigma = wave_sum(s2);
-        const double alpha = lane_bcast(x[0], 0);
+        const double alpha = at(x, o);
         double tau = 0.0, beta = alpha, scal = 0.0;
         if (sigma > 0.0) {
             const double nrm = sqrt(fma(alpha, alpha, sigma));
@@ -1518,104 +1572,103 @@ __device__ void big_tridiag_sym(double* A, int n, int lda, double* d, double* e,
             tau = (beta - alpha) / beta;
             scal = 1.0 / (alpha - beta);
         }
-        double v[NR];
+        __syncthreads();  // every wave has read row s, and red of the step before
 #pragma unroll
         for (int t = 0; t < NR; ++t) {
-            const int i = lane + 64 * t;
-            v[t] = i == 0 ? 1.0 : (tau == 0.0 ? 0.0 : x[t] * scal);
-            if (i < m) {
-                rows[o + i] = v[t];
-                vN[o + i] = v[t];
-            }
+            const int r = lane + 64 * t;
+            v[t] = r == o ? 1.0 : (r < o || tau == 0.0 ? 0.0 : x[t] * scal);
+            if (wv == 0 && r >= o && r < n) rows[r] = v[t];
         }
-        if (lane == 0) {
+        if (wv == 0 && lane == 0) {
             d[s] = dss;
             e[s] = beta;
             tauv[s] = tau;
         }
-        __syncthreads();
         // one pass over rows c = o.. (columns r >= c): pending update, store,
         // and p = B v of this step
-        double wpr[NR], vpr[NR], vnr[NR], pp[NR];
+        double pp[NR];
 #pragma unroll
-        for (int t = 0; t < NR; ++t) {
-            const int i = lane + 64 * t, r = o + i;
-            wpr[t] = i < m ? wP[r] : 0.0;
-            vpr[t] = i < m ? vP[r] : 0.0;
-            vnr[t] = i < m ? v[t] : 0.0;
-            pp[t] = 0.0;
-        }
+        for (int t = 0; t < NR; ++t) pp[t] = 0.0;
 #pragma unroll
         for (int cb = 0; cb < NR; ++cb) {
-            const int cn = m - 64 * cb < 64 ? m - 64 * cb : 64;
-            if (cn <= 0) break;
-            for (int c0 = 0; c0 < cn; c0 += kRowBatch) {
-                double a[kRowBatch][NR];
+            const int cn = n - 64 * cb < 64 ? n - 64 * cb : 64;
+            const int lo = o - 64 * cb > 0 ? o - 64 * cb : 0;  // first row within the block
+            for (int c0 = (lo & ~7) + 8 * ((wv - (lo >> 3)) & (kBigW - 1)); c0 < cn;
+                 c0 += 8 * kBigW) {
+                double a[8][NR], rs[8];
 #pragma unroll
-                for (int u = 0; u < kRowBatch; ++u) {
-                    const int ic = 64 * cb + c0 + u;  // row index relative to o
-                    const double* row = A + (size_t)(o + ic) * lda + o;
+                for (int u = 0; u < 8; ++u) {
+                    const int c = 64 * cb + c0 + u;
+                    const double* row = A + (size_t)c * lda;
 #pragma unroll
-                    for (int t = 0; t < NR; ++t) {
-                        const int i = lane + 64 * t;
-                        a[u][t] = (c0 + u < cn && t >= cb && i >= ic && i < m) ? row[i] : 0.0;
+                    for (int t = cb; t < NR; ++t) {
+                        const int r = lane + 64 * t;
+                        a[u][t] = (c >= o && r >= c && r < n) ? row[r] : 0.0;
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < kRowBatch; ++u) {
-                    const int ic = 64 * cb + c0 + u;
-                    const bool rv = c0 + u < cn;
-                    const int c = o + (rv ? ic : 0);
-                    const double vpc = vP[c], wpc = wP[c], vnc = vN[c];
-                    double* row = A + (size_t)(o + ic) * lda + o;
-                    double rs = 0.0;
+                for (int u = 0; u < 8; ++u) {
+                    const int c = 64 * cb + c0 + u;  // (rows below o or past n: no lane takes part)
+                    const double vpc = lane_bcast(vp[cb], c0 + u), wpc = lane_bcast(wp[cb], c0 + u);
+                    const double vnc = lane_bcast(v[cb], c0 + u);
+                    double* row = A + (size_t)c * lda;
+                    rs[u] = 0.0;
 #pragma unroll
-                    for (int t = 0; t < NR; ++t) {
-                        const int i = lane + 64 * t;
-                        if (rv && t >= cb && i >= ic && i < m) {
+                    for (int t = cb; t < NR; ++t) {
+                        const int r = lane + 64 * t;
+                        if (c >= o && r >= c && r < n) {
                             const double an = rn_sub(
-                                a[u][t], rn_add(rn_mul(vpc, wpr[t]), rn_mul(wpc, vpr[t])));
-                            row[i] = an;
-                            if (i > ic) {
+                                a[u][t], rn_add(rn_mul(vpc, wp[t]), rn_mul(wpc, vp[t])));
+                            row[r] = an;
+                            if (r > c) {
                                 pp[t] = fma(an, vnc, pp[t]);
-                                rs = fma(an, vnr[t], rs);
+                                rs[u] = fma(an, v[t], rs[u]);
                             } else {
-                                rs = fma(an, vnc, rs);
+                                rs[u] = fma(an, vnc, rs[u]);
                             }
                         }
                     }
-                    rs = wave_sum(rs);
-                    if (rv && lane == ((c0 + u) & 63)) pp[cb] += rs;
                 }
+                const double rsum = wave_sum8(rs, lane);
+                if ((lane & ~7) == c0) pp[cb] += rsum;
             }
         }
-        __syncthreads();  // every lane is done reading this step's vP, wP, vN
+#pragma unroll
+        for (int t = 0; t < NR; ++t)
+            if (lane + 64 * t < n) red[wv * n + lane + 64 * t] = pp[t];
+        __syncthreads();
         double pv = 0.0;
 #pragma unroll
         for (int t = 0; t < NR; ++t) {
-            pp[t] *= tau;
+            const int r = lane + 64 * t;
+            double sum = 0.0;
+            if (r < n) {
+                sum = red[r];
+#pragma unroll
+                for (int w = 1; w < kBigW; ++w) sum += red[w * n + r];
+            }
+            pp[t] = tau * sum;
             pv = fma(pp[t], v[t], pv);
         }
         const double K = 0.5 * tau * wave_sum(pv);
 #pragma unroll
         for (int t = 0; t < NR; ++t) {
-            const int i = lane + 64 * t;
-            if (i < m) {
-                vP[o + i] = v[t];
-                wP[o + i] = fma(-K, v[t], pp[t]);
-            }
+            vp[t] = v[t];
+            wp[t] = lane + 64 * t >= o ? fma(-K, v[t], pp[t]) : 0.0;
         }
-        __syncthreads();
     }
-    if (lane == 0) {
-        const int a0 = n - 2, a1 = n - 1;
-        d[a0] = rn_sub(A[(size_t)a0 * lda + a0],
-                          rn_add(rn_mul(vP[a0], wP[a0]), rn_mul(wP[a0], vP[a0])));
-        e[a0] = rn_sub(A[(size_t)a0 * lda + a1],
-                          rn_add(rn_mul(vP[a0], wP[a1]), rn_mul(wP[a0], vP[a1])));
-        d[a1] = rn_sub(A[(size_t)a1 * lda + a1],
-                          rn_add(rn_mul(vP[a1], wP[a1]), rn_mul(wP[a1], vP[a1])));
+    const int a0 = n - 2, a1 = n - 1;
+    const double v1 = at(vp, a1), w1 = at(wp, a1);
+    if (wv == 0 && lane == 0) {
+        d[a1] = rn_sub(A[(size_t)a1 * lda + a1], rn_add(rn_mul(v1, w1), rn_mul(w1, v1)));
         e[a1] = 0.0;
+    }
+    if (a0 >= 0) {
+        const double v0 = at(vp, a0), w0 = at(wp, a0);
+        if (wv == 0 && lane == 0) {
+            d[a0] = rn_sub(A[(size_t)a0 * lda + a0], rn_add(rn_mul(v0, w0), rn_mul(w0, v0)));
+            e[a0] = rn_sub(A[(size_t)a0 * lda + a1], rn_add(rn_mul(v0, w1), rn_mul(w0, v1)));
+        }
     }
     __syncthreads();
 }
@@ -1880,44 +1933,160 @@ struct VecSet {
 
 // y <- Q^T y (transpose: H_0 first) or y <- Q y (H_{n-3} first) for nvec
 // vectors, H_j = I - tau_j v_j v_j^T with v_j in row j, columns j+1.., of A.
-// Lane r owns elements r, r + 64, ... of every vector.
+// The waves take the vectors in turns of two, held in registers (lane l: elements
+// l, l + 64, ..); the next reflector is loaded while one is applied.
 template <int NR>
-__device__ void big_refl_vecs(const double* A, int n, int lda, const double* tauv, const VecSet& V,
-                              int nvec, bool transpose, int lane)
+__device__ __forceinline__ void big_refl_vecs(const double* A, int n, int lda, const double* tauv, const VecSet& V,
+                              int nvec, bool transpose, int lane, int wv)
 {
-    for (int s = 0; s + 2 < n; ++s) {
+    auto load = [&](int s, double (&v)[NR]) {
         const int j = transpose ? s : n - 3 - s;
-        const double tau = tauv[j];
-        if (tau == 0.0) continue;
-        const int o = j + 1, m = n - o;
-        double v[NR];
 #pragma unroll
         for (int t = 0; t < NR; ++t) {
             const int r = lane + 64 * t;
-            v[t] = r < m ? A[(size_t)j * lda + o + r] : 0.0;
+            v[t] = r > j && r < n ? A[(size_t)j * lda + r] : 0.0;
         }
-        for (int q = 0; q < nvec; ++q) {
-            double* y = V.at(q) + o;
-            double sum = 0.0;
+    };
+    for (int q0 = wv; q0 < nvec; q0 += 2 * kBigW) {
+        const int q1 = q0 + kBigW;
+        const bool two = q1 < nvec;
+        double y0[NR], y1[NR], v[NR], vn[NR];
 #pragma unroll
-            for (int t = 0; t < NR; ++t)
-                if (lane + 64 * t < m) sum = fma(v[t], y[lane + 64 * t], sum);
-            sum = tau * wave_sum(sum);
-#pragma unroll
-            for (int t = 0; t < NR; ++t)
-                if (lane + 64 * t < m) y[lane + 64 * t] = fma(-sum, v[t], y[lane + 64 * t]);
+        for (int t = 0; t < NR; ++t) {
+            const int r = lane + 64 * t;
+            y0[t] = r < n ? V.at(q0)[r] : 0.0;
+            y1[t] = two && r < n ? V.at(q1)[r] : 0.0;
+            vn[t] = 0.0;
         }
-        // element o + r belongs to lane r, so ownership shifts by one lane per
-        // reflector: order this step's LDS stores before the next step's loads
+        if (n > 2) load(0, vn);
+        for (int s = 0; s + 2 < n; ++s) {
+#pragma unroll
+            for (int t = 0; t < NR; ++t) v[t] = vn[t];
+            if (s + 3 < n) load(s + 1, vn);
+            const double tau = tauv[transpose ? s : n - 3 - s];
+            double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+            for (int t = 0; t < NR; ++t) {
+                s0 = fma(v[t], y0[t], s0);
+                s1 = fma(v[t], y1[t], s1);
+            }
+            s0 = tau * wave_sum(s0);
+            s1 = tau * wave_sum(s1);
+#pragma unroll
+            for (int t = 0; t < NR; ++t) {
+                y0[t] = fma(-s0, v[t], y0[t]);
+                y1[t] = fma(-s1, v[t], y1[t]);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < NR; ++t) {
+            const int r = lane + 64 * t;
+            if (r < n) V.at(q0)[r] = y0[t];
+            if (two && r < n) V.at(q1)[r] = y1[t];
+        }
+    }
+}
+
+// The functions of T without eigenvalues (lekf_invsqrt.hpp): v1 <- (T + g0)^-1 v1, then
+// Cw_q = row q . v1, then row q <- sum_j w_j (T + g0 + m sg_j)^-1 row q with w_j =
+// scale om_j, or in the dual form (gam > 0) -scale om_j / (gam + m sg_j): the divided
+// difference of the same sum.  A thread solves one row at one shift, its factors and
+// solution in the workspace wsp ([element][thread], 2 n wth doubles).
+__device__ __forceinline__ void big_function(const EigLds& L, int n, double g0, double m,
+                                             double scale, double gam, int lev, const VecSet& V,
+                                             double* wsp, int wth, int tid)
+{
+    const int lane = tid & 63, wv = tid >> 6;
+    const int N = 8 + 4 * lev, per = (wth - 1) / N;
+    double* const tw = wsp + (size_t)n * wth;
+    for (int r0 = 0; r0 == 0 || r0 < V.nrow; r0 += per) {
+        const int nr = V.nrow - r0 < per ? V.nrow - r0 : per;
+        const int q = (tid - 1) / N, j = tid - 1 - q * N;
+        const bool own = tid == 0 && r0 == 0;  // b's solve
+        if (own || (tid > 0 && q < nr)) {
+            double sh = g0, wt = 1.0;
+            const double* z = V.v1;
+            if (!own) {
+                const double ms = m * g_invsqrt.sg[lev][j];
+                sh = g0 + ms;
+                wt = scale * g_invsqrt.om[lev][j];
+                if (gam > 0.0) wt = -wt / (gam + ms);
+                z = V.at(r0 + q);
+            }
+            double t = 0.0, yp = 0.0, ep = 0.0;
+#pragma unroll 4
+            for (int i = 0; i < n; ++i) {
+                const double rr = rcp_nr(fma(-ep, t, L.d[i] + sh));
+                yp = fma(-t, yp, wt * z[i]);
+                ep = L.e[i];
+                t = ep * rr;
+                wsp[(size_t)i * wth + tid] = yp * rr;
+                tw[(size_t)i * wth + tid] = t;
+            }
+            double x = 0.0;
+            for (int i0 = (n - 1) & ~7; i0 >= 0; i0 -= 8) {
+                double y8[8], t8[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const bool in = i0 + u < n;
+                    y8[u] = in ? wsp[(size_t)(i0 + u) * wth + tid] : 0.0;
+                    t8[u] = in ? tw[(size_t)(i0 + u) * wth + tid] : 0.0;
+                }
+#pragma unroll
+                for (int u = 7; u >= 0; --u)
+                    if (i0 + u < n) {
+                        x = fma(-t8[u], x, y8[u]);
+                        wsp[(size_t)(i0 + u) * wth + tid] = x;
+                    }
+            }
+        }
+        __syncthreads();
+        if (r0 == 0) {
+            if (tid < n) V.v1[tid] = wsp[(size_t)tid * wth];
+            __syncthreads();
+            for (int r = wv; r < V.nrow; r += kBigW) {
+                double c = 0.0;
+                for (int i = lane; i < n; i += 64) c = fma(V.at(r)[i], V.v1[i], c);
+                c = wave_sum(c);
+                if (lane == 0) L.Cw[r] = c;
+            }
+            __syncthreads();
+        }
+        if (tid < n)
+            for (int r = 0; r < nr; ++r) {
+                const double* src = wsp + (size_t)tid * wth + 1 + r * N;
+                double c = src[0];
+                for (int u = 1; u < N; ++u) c += src[u];
+                V.at(r0 + r)[tid] = c;
+            }
         __syncthreads();
     }
+}
+
+// Table level for the spectrum of T + g0 in [m, hi], kLevels or more if none reaches it
+__device__ __forceinline__ int big_level(const EigLds& L, int n, double g0, double m, int lane)
+{
+    double hi = 0.0;
+    bool bad = false;
+    for (int i = lane; i < n; i += 64) {
+        const double h = fabs(L.d[i] + g0) + fabs(L.e[i]) + (i > 0 ? fabs(L.e[i - 1]) : 0.0);
+        bad |= !(h <= 1.0e300);
+        hi = h > hi ? h : hi;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const double h = __shfl_xor(hi, o, 64);
+        hi = h > hi ? h : hi;
+    }
+    if (__ballot(bad) != 0ull) return lekf_invsqrt::kLevels;
+    return trf_level(hi, m);
 }
 
 // eig_ql on (d, e) without eigenvectors: each sweep's rotations are applied
 // to the nvec vectors (lane q owns vector q; the same update as a row of Z,
 // so u = Z^T y is maintained) and appended to rbuf.  Returns nonzero if an
 // eigenvalue needed more than kQlMaxIter sweeps; ovf is set if rbuf filled.
-__device__ int eig_ql_vec(EigLds& L, int n, int lane, const VecSet& V, int nvec, double* rbuf,
+__device__ __forceinline__ int eig_ql_vec(EigLds& L, int n, int lane, const VecSet& V, int nvec, double* rbuf,
                           long rcap, long& rpos, bool& ovf)
 {
     double* d = L.d;
@@ -1967,7 +2136,7 @@ __device__ int eig_ql_vec(EigLds& L, int n, int lane, const VecSet& V, int nvec,
                 ei = eprev;
                 di1 = di;
             }
-            __syncthreads();
+            wave_sync();
             const int ilo = split ? i + 1 : l;
             const int cnt = m - ilo;
             if (!ovf && rpos + 2L * cnt + 2 <= rcap) {
@@ -1997,7 +2166,7 @@ __device__ int eig_ql_vec(EigLds& L, int n, int lane, const VecSet& V, int nvec,
                 e[l] = g;
                 e[m] = 0.0;
             }
-            __syncthreads();
+            wave_sync();
         }
     }
     return 0;
@@ -2005,7 +2174,7 @@ __device__ int eig_ql_vec(EigLds& L, int n, int lane, const VecSet& V, int nvec,
 
 // y <- S y: the recorded sweeps in reverse order, each sweep's rotations in
 // increasing index (the inverse of the forward update)
-__device__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec, const double* rbuf, long rpos,
+__device__ __forceinline__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec, const double* rbuf, long rpos,
                             int lane)
 {
     long pos = rpos;
@@ -2015,7 +2184,7 @@ __device__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec, const double* 
         const long base = pos - 2 - 2L * cnt;
         for (int q = lane; q < 2 * cnt; q += 64)
             L.rot[2 * (m - 1 - (q >> 1)) + (q & 1)] = rbuf[base + q];
-        __syncthreads();
+        wave_sync();
         if (lane < nvec) {
             double* z = V.at(lane);
             double zl = z[ilo];
@@ -2027,16 +2196,95 @@ __device__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec, const double* 
             }
             z[m] = zl;
         }
-        __syncthreads();
+        wave_sync();
         pos = base;
     }
 }
 
-// one point of the large-k vector path (no trans/pao outputs)
-__device__ void big_vec_point(const LekfJob& J, int b, double* rec, double* rbuf, long rcap,
-                              EigLds& L, int lane)
+// The analysis' functions applied in T's basis, for both forms: L.B = Q^T b and the rows
+// of V = Q^T rows are replaced by f(T)'s, L.Cw by the rows' products with (T + g0)^-1 b.
+// The rational form where its tables reach the condition number (they do up to 4 8^6 in
+// FP64; 4 8^4 in the mixed forms, whose C is only positive semidefinite to 1e-6 of its
+// norm), else QL by wave 0 with its rotations kept in wsp.  shift = (k-1)/alpha bounds
+// the spectrum from below; gam > 0: the dual form (g0 = gam = shift).  Returns the status
+// bits.
+template <int MODE>
+__device__ __forceinline__ int big_spectral(EigLds& L, int n, int k, double shift, double gam, const VecSet& V,
+                            double* wsp, long wcap, int tid)
 {
-    const int k = J.k, lda = k;
+    const int lane = tid & 63, wv = tid >> 6;
+    const double g0 = gam;  // T + g0 has the spectrum of C + (k-1)/alpha
+    const double m = shift * (MODE == 0 ? 0.999 : 0.75);
+    const int lev = big_level(L, n, g0, m, lane);
+    int status = 0;
+    if (lev < (MODE == 0 ? lekf_invsqrt::kLevels : 5)) {
+        const long w = wcap / (2 * n);
+        big_function(L, n, g0, m, sqrt((double)(k - 1) * m), gam, lev, V, wsp,
+                     w < 64 * kBigW ? (int)w : 64 * kBigW, tid);
+        return status;
+    }
+    const int nrow = V.nrow, ks = V.k;
+    if (wv == 0) {
+        long rpos = 0;
+        bool ovf = false;
+        if (eig_ql_vec(L, n, lane, V, nrow + 1, wsp, wcap, rpos, ovf)) status |= LEKF_PT_NOCONV;
+        if (ovf) status |= LEKF_PT_NOCONV;
+        wave_sync();
+        // eigenvalues of C (dual: gamma + s_j and gamma); truncation test
+        // (common_mtx.f90:66-74)
+        double smax = L.d[0], smin = L.d[0];
+        for (int j = 1; j < n; ++j) {
+            smax = L.d[j] > smax ? L.d[j] : smax;
+            smin = L.d[j] < smin ? L.d[j] : smin;
+        }
+        const double lmax = gam > 0.0 ? gam + (smax > 0.0 ? smax : 0.0) : smax;
+        const double lmin = gam > 0.0 ? (smin < 0.0 ? gam + smin : gam) : smin;
+        if (!(lmax > 0.0) || lmin < fabs(lmax) * 1.4901161193847656e-08) status |= LEKF_PT_RANKDEF;
+        // u = L^-1 V^T b;  X' w-bar = (V^T x')^T u
+        for (int j = lane; j < n; j += 64) V.v1[j] = V.v1[j] / (g0 + L.d[j]);
+        wave_sync();
+        for (int r = lane; r < nrow; r += 64) {
+            double s = 0.0;
+            for (int j = 0; j < n; ++j) s = fma(V.R[r * ks + j], V.v1[j], s);
+            L.Cw[r] = s;
+        }
+        wave_sync();
+        // f of the eigenvalues; dual: (f(gamma + s) - f(gamma)) / s without cancellation
+        const double sg = sqrt(gam), skm1 = sqrt((double)(k - 1));
+        for (int w = lane; w < nrow * n; w += 64) {
+            const int r = w / n, j = w - r * n;
+            if (gam > 0.0) {
+                const double sgs = sqrt(gam + L.d[j]);
+                V.R[r * ks + j] *= -skm1 / (sg * sgs * (sg + sgs));
+            } else {
+                V.R[r * ks + j] *= sqrt((double)(k - 1) / L.d[j]);
+            }
+        }
+        wave_sync();
+        if (!ovf) ql_back_vec(L, V, nrow + 1, wsp, rpos, lane);
+    }
+    __syncthreads();
+    return status;
+}
+
+// One point of the large-k path without trans/pao outputs, kBigW waves.
+//
+// p >= k, the k x k form: C's tridiagonalisation carries b and the state rows.
+//
+// 0 < p < k, the dual form: with B = diag(sqrt w) Y (p x k), G = B B^T = U S U^T (in the
+// workspace record, p x p) and gamma = (k-1)/alpha, C = gamma I + B^T B has the
+// eigenvalues gamma + s_j (eigenvectors B^T u_j / sqrt(s_j)) and gamma (k - p times), so
+//   f(C) x = f(gamma) x + B^T U diag((f(gamma + s) - f(gamma)) / s) U^T B x
+// for f(l) = sqrt((k-1)/l), and C^-1 B^T = B^T (gamma I + G)^-1 gives
+//   w-bar = B^T U diag(1/(gamma + s)) U^T (sqrt(w) d).
+// G's tridiagonalisation runs exactly as C's, carrying sqrt(w) d and B x'_r.
+template <int MODE>
+__device__ __forceinline__ void big_vec_point(const LekfJob& J, int b, double* rec, double* wsp, long wcap,
+                              EigLds& L, int tid)
+{
+    constexpr int NT = 64 * kBigW;
+    const int lane = tid & 63, wv = tid >> 6;
+    const int k = J.k;
     const long off = J.loc_off[b];
     const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - off);
     double alpha = J.infl_in ? J.infl_in[b] : J.infl_fixed;
@@ -2047,279 +2295,157 @@ __device__ void big_vec_point(const LekfJob& J, int b, double* rec, double* rbuf
     const int n3 = apply ? J.nv3d : 0, n2 = (apply && lev == 0) ? J.nv2d : 0;
     const int nrow = n3 + n2;
     const int ks = k + 1;  // row stride of R: odd, so lane-per-row LDS accesses spread over banks
+    const bool dual = big_dual(J, p, k);
+    const bool want_wb = J.transm != nullptr;
+    const int n = dual ? p : k;
     if (nrow > 0) {
-        for (int w = lane; w < nrow * k; w += 64) {
+        for (int w = tid; w < nrow * k; w += NT) {
             const int r = w / k, m = w - r * k;
             const double* src = (r < n3) ? J.x3b + ((size_t)b * n3 + r) * k
                                          : J.x2b + ((size_t)ij * J.nv2d + (r - n3)) * k;
             L.X[r * k + m] = src[m];
         }
         __syncthreads();
-        for (int r = lane; r < nrow; r += 64) {
+        for (int r = tid; r < nrow; r += NT) {
             double s = L.X[r * k];
             for (int m = 1; m < k; ++m) s += L.X[r * k + m];
             L.M[r] = s / (double)k;
         }
         __syncthreads();
-        for (int w = lane; w < nrow * k; w += 64) L.X[w] -= L.M[w / k];
+        for (int w = tid; w < nrow * k; w += NT) L.X[w] -= L.M[w / k];
         __syncthreads();
     }
     if (p > 0) {
-        for (int i = lane; i < k; i += 64) L.B[i] = rec[(size_t)k * k + i];
-        const double p1 = rec[(size_t)k * k + k], p3 = rec[(size_t)k * k + k + 1];
+        double p1, p3;
+        for (int i = tid; i < n; i += NT) L.U[i] = rec[(size_t)i * n + i];
+        if (dual) {
+            // weights, sqrt(w) d, P1 = sum w d^2, P3 = sum rho (common_letkf.f90:219-227),
+            // the sums by every wave alike
+            const bool wloc = (J.flags & LEKF_F_WLOC) != 0;
+            p1 = p3 = 0.0;
+            for (int i = lane; i < p; i += 64) {
+                const long o = J.loc_idx[off + i];
+                const double rho = J.loc_rho[off + i];
+                const double rd = J.loc_rdiag ? J.loc_rdiag[off + i] : J.rdiag[o];
+                const double w = (wloc ? 1.0 : rho) / rd;
+                const double dd = J.dep[o];
+                if (wv == 0) {
+                    L.sw[i] = sqrt(w);
+                    L.B[i] = sqrt(w) * dd;
+                }
+                p1 = fma(w * dd, dd, p1);
+                p3 += rho;
+            }
+            p1 = wave_sum(p1);
+            p3 = wave_sum(p3);
+        } else {
+            for (int i = tid; i < k; i += NT) L.B[i] = rec[(size_t)k * k + i];
+            p1 = rec[(size_t)k * k + k];
+            p3 = rec[(size_t)k * k + k + 1];
+        }
         __syncthreads();
         double tr = 0.0;
-        for (int i = 0; i < k; ++i) tr += rec[(size_t)i * lda + i];
+        for (int i = 0; i < n; ++i) tr += L.U[i];
         const double p2 = tr / (double)(k - 1);
         if ((J.flags & LEKF_F_MINFL) && J.minfl > 0.0 && alpha < J.minfl) alpha = J.minfl;
         const double rho = 1.0 / alpha;
-        __syncthreads();
-        for (int i = lane; i < k; i += 64) rec[(size_t)i * lda + i] += (double)(k - 1) * rho;
-        for (int w = lane; w < nrow * k; w += 64) L.R[(w / k) * ks + w % k] = L.X[w];
-        __syncthreads();
-        big_tridiag_sym<4>(rec, k, lda, L.d, L.e, L.tau, L.rot, L.rot + k, L.U, lane);
-        const VecSet Vf{L.R, nrow, ks, L.B, nullptr};
-        big_refl_vecs<4>(rec, k, lda, L.tau, Vf, nrow + 1, true, lane);
-        __syncthreads();
-        long rpos = 0;
-        bool ovf = false;
-        if (eig_ql_vec(L, k, lane, Vf, nrow + 1, rbuf, rcap, rpos, ovf)) status |= LEKF_PT_NOCONV;
-        if (ovf) status |= LEKF_PT_NOCONV;
-        __syncthreads();
-        double lmax = 0.0, lmin = 1.0e308;
-        for (int j = 0; j < k; ++j) {
-            const double lj = L.d[j];
-            lmax = lj > lmax ? lj : lmax;
-            lmin = lj < lmin ? lj : lmin;
-        }
-        if (!(lmax > 0.0) || lmin < fabs(lmax) * 1.4901161193847656e-08) status |= LEKF_PT_RANKDEF;
-        // u = L^-1 V^T b;  X' w-bar = (V^T x')^T u;  rows <- sqrt((k-1)/L) V^T x'
-        for (int j = lane; j < k; j += 64) L.U[j] = L.B[j] / L.d[j];
-        __syncthreads();
-        for (int r = lane; r < nrow; r += 64) {
-            double s = 0.0;
-            for (int j = 0; j < k; ++j) s = fma(L.R[r * ks + j], L.U[j], s);
-            L.Cw[r] = s;
-        }
-        const bool want_wb = J.transm != nullptr;
-        if (want_wb)
-            for (int j = lane; j < k; j += 64) L.Wb[j] = L.U[j];
-        __syncthreads();
-        for (int w = lane; w < nrow * k; w += 64) {
-            const int j = w % k;
-            L.R[(w / k) * ks + j] *= sqrt((double)(k - 1) / L.d[j]);
+        const double gam = (double)(k - 1) / alpha;
+        if (dual) {
+            // y_r = B x'_r: the waves take the local obs rows in turns, lanes over members
+            for (int i = wv; i < p; i += kBigW) {
+                const long o = J.loc_idx[off + i];
+                double y[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int m = lane + 64 * t;
+                    y[t] = m < k ? J.hdxf[o * J.y_so + (long)m * J.y_sm] : 0.0;
+                }
+                for (int r = 0; r < nrow; ++r) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        if (lane + 64 * t < k) s = fma(y[t], L.X[r * k + lane + 64 * t], s);
+                    s = wave_sum(s);
+                    if (lane == 0) L.R[r * ks + i] = L.sw[i] * s;
+                }
+            }
+        } else {
+            for (int i = tid; i < k; i += NT) rec[(size_t)i * k + i] += (double)(k - 1) * rho;
+            for (int w = tid; w < nrow * k; w += NT) L.R[(w / k) * ks + w % k] = L.X[w];
         }
         __syncthreads();
-        const VecSet Vb{L.R, nrow, ks, L.Wb, nullptr};
-        const int nvb = nrow + (want_wb ? 1 : 0);
-        if (!ovf) ql_back_vec(L, Vb, nvb, rbuf, rpos, lane);
-        big_refl_vecs<4>(rec, k, lda, L.tau, Vb, nvb, false, lane);
+        big_tridiag_sym<4>(rec, n, n, L.d, L.e, L.tau, L.rot, lane, wv);
+        const VecSet V{L.R, nrow, ks, L.B, nullptr};
+        big_refl_vecs<4>(rec, n, n, L.tau, V, nrow + 1, true, lane, wv);
         __syncthreads();
-        if (want_wb)
-            for (int i = lane; i < k; i += 64) J.transm[(size_t)b * k + i] = L.Wb[i];
-        if (lane == 0 && J.infl_out)
+        status |= big_spectral<MODE>(L, n, k, gam, dual ? gam : 0.0, V, wsp, wcap, tid);
+        big_refl_vecs<4>(rec, n, n, L.tau, V, nrow + (want_wb ? 1 : 0), false, lane, wv);
+        __syncthreads();
+        if (dual) {
+            // coefficients of the local obs rows: sqrt(w_i) times the p-vectors
+            for (int w = tid; w < nrow * p; w += NT) {
+                const int r = w / p, i = w - r * p;
+                L.R[r * ks + i] *= L.sw[i];
+            }
+            if (want_wb)
+                for (int i = tid; i < p; i += NT) L.B[i] *= L.sw[i];
+            __syncthreads();
+            if (want_wb && tid < k) {
+                double acc = 0.0;
+                for (int i = 0; i < p; ++i)
+                    acc = fma(L.B[i],
+                              J.hdxf[J.loc_idx[off + i] * (long)J.y_so + (long)tid * J.y_sm], acc);
+                J.transm[(size_t)b * k + tid] = acc;
+            }
+        } else if (want_wb) {
+            for (int i = tid; i < k; i += NT) J.transm[(size_t)b * k + i] = L.B[i];
+        }
+        if (tid == 0 && J.infl_out)
             J.infl_out[b] = (J.flags & LEKF_F_FIXED_INFL) ? J.infl_fixed
                                                           : adaptive_alpha(alpha, p1, p2, p3);
     } else {
         if (J.transm)
-            for (int i = lane; i < k; i += 64) J.transm[(size_t)b * k + i] = 0.0;
-        if (lane == 0 && J.infl_out)
+            for (int i = tid; i < k; i += NT) J.transm[(size_t)b * k + i] = 0.0;
+        if (tid == 0 && J.infl_out)
             J.infl_out[b] = (J.flags & LEKF_F_FIXED_INFL) ? J.infl_fixed : alpha;
     }
-    if (lane == 0 && J.status) J.status[b] = status;
+    if (tid == 0 && J.status) J.status[b] = status;
     if (nrow == 0) return;
     const uint32_t mask = J.upd_mask ? J.upd_mask[lev] : 0xffffffffu;
-    for (int w = lane; w < nrow * k; w += 64) {
-        const int r = w / k, m = w - r * k;
-        const bool upd = (r >= n3) || ((mask >> r) & 1u);
-        double a;
-        if (!upd)
-            a = L.M[r] + L.X[r * k + m];
-        else if (p > 0)
-            a = L.M[r] + (L.Cw[r] + L.R[r * ks + m]);
-        else
-            a = L.M[r] + sa * L.X[r * k + m];
-        double* dst = (r < n3) ? J.x3a + ((size_t)b * n3 + r) * k
-                               : J.x2a + ((size_t)ij * J.nv2d + (r - n3)) * k;
-        dst[m] = a;
-    }
-}
-
-// One point of the large-k dual form (0 < p < k, no trans/pao).  With
-// B = diag(sqrt w) Y (p x k), G = B B^T = U S U^T (in the workspace record,
-// p x p) and gamma = (k-1)/alpha, C = gamma I + B^T B has the eigenvalues
-// gamma + s_j (eigenvectors B^T u_j / sqrt(s_j)) and gamma (k - p times), so
-//   f(C) x = f(gamma) x + B^T U diag((f(gamma + s) - f(gamma)) / s) U^T B x
-// for f(l) = sqrt((k-1)/l), and C^-1 B^T = B^T (gamma I + G)^-1 gives
-//   w-bar = B^T U diag(1/(gamma + s)) U^T (sqrt(w) d).
-// The p x p eigenproblem runs exactly as the k x k one of big_vec_point,
-// carrying sqrt(w) d and B x'_r through Q^T and the QL rotations.
-__device__ void big_dual_point(const LekfJob& J, int b, double* rec, double* rbuf, long rcap,
-                               EigLds& L, int lane)
-{
-    const int k = J.k;
-    const long off = J.loc_off[b];
-    const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - off);
-    double alpha = J.infl_in ? J.infl_in[b] : J.infl_fixed;
-    int status = 0;
-    const bool wloc = (J.flags & LEKF_F_WLOC) != 0;
-    const bool apply = (J.flags & LEKF_F_APPLY) != 0;
-    const int lev = apply ? b / J.nij : 0, ij = apply ? b - lev * J.nij : 0;
-    const int n3 = apply ? J.nv3d : 0, n2 = (apply && lev == 0) ? J.nv2d : 0;
-    const int nrow = n3 + n2;
-    const int ks = k + 1;
-    if (nrow > 0) {
-        for (int w = lane; w < nrow * k; w += 64) {
-            const int r = w / k, m = w - r * k;
-            const double* src = (r < n3) ? J.x3b + ((size_t)b * n3 + r) * k
-                                         : J.x2b + ((size_t)ij * J.nv2d + (r - n3)) * k;
-            L.X[r * k + m] = src[m];
-        }
-        __syncthreads();
-        for (int r = lane; r < nrow; r += 64) {
-            double s = L.X[r * k];
-            for (int m = 1; m < k; ++m) s += L.X[r * k + m];
-            L.M[r] = s / (double)k;
-        }
-        __syncthreads();
-        for (int w = lane; w < nrow * k; w += 64) L.X[w] -= L.M[w / k];
-        __syncthreads();
-    }
-    // weights, sqrt(w) d, P1 = sum w d^2, P3 = sum rho (common_letkf.f90:219-227)
-    double p1 = 0.0, p3 = 0.0;
-    for (int i = lane; i < p; i += 64) {
-        const long o = J.loc_idx[off + i];
-        const double rho = J.loc_rho[off + i];
-        const double rd = J.loc_rdiag ? J.loc_rdiag[off + i] : J.rdiag[o];
-        const double w = (wloc ? 1.0 : rho) / rd;
-        const double dd = J.dep[o];
-        L.sw[i] = sqrt(w);
-        L.B[i] = L.sw[i] * dd;
-        p1 = fma(w * dd, dd, p1);
-        p3 += rho;
-    }
-    p1 = wave_sum(p1);
-    p3 = wave_sum(p3);
-    double tr = 0.0;
-    for (int i = 0; i < p; ++i) tr += rec[(size_t)i * p + i];
-    const double p2 = tr / (double)(k - 1);
-    if ((J.flags & LEKF_F_MINFL) && J.minfl > 0.0 && alpha < J.minfl) alpha = J.minfl;
-    const double gam = (double)(k - 1) / alpha;
-    __syncthreads();
-    // y_r = B x'_r: one local obs row at a time, lanes over members
-    for (int i = 0; i < p; ++i) {
-        const long o = J.loc_idx[off + i];
-        double y[4];
+    const double fg = sqrt((double)(k - 1) / ((double)(k - 1) / alpha));
+    const int m = tid;
+    if (m >= k) return;
+    constexpr int kRows = 8;  // rows summed at once over the obs of the dual form
+    for (int r0 = 0; r0 < nrow; r0 += kRows) {
+        double acc[kRows];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int m = lane + 64 * t;
-            y[t] = m < k ? J.hdxf[o * J.y_so + (long)m * J.y_sm] : 0.0;
-        }
-        for (int r = 0; r < nrow; ++r) {
-            double s = 0.0;
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                if (lane + 64 * t < k) s = fma(y[t], L.X[r * k + lane + 64 * t], s);
-            s = wave_sum(s);
-            if (lane == 0) L.R[r * ks + i] = L.sw[i] * s;
-        }
-    }
-    __syncthreads();
-    big_tridiag_sym<4>(rec, p, p, L.d, L.e, L.tau, L.rot, L.rot + k, L.U, lane);
-    const VecSet Vf{L.R, nrow, ks, L.B, nullptr};
-    big_refl_vecs<4>(rec, p, p, L.tau, Vf, nrow + 1, true, lane);
-    __syncthreads();
-    long rpos = 0;
-    bool ovf = false;
-    if (eig_ql_vec(L, p, lane, Vf, nrow + 1, rbuf, rcap, rpos, ovf)) status |= LEKF_PT_NOCONV;
-    if (ovf) status |= LEKF_PT_NOCONV;
-    __syncthreads();
-    // eigenvalues of C: gamma + s_j and gamma; truncation test (common_mtx.f90:66-74)
-    double smax = L.d[0], smin = L.d[0];
-    for (int j = 1; j < p; ++j) {
-        smax = L.d[j] > smax ? L.d[j] : smax;
-        smin = L.d[j] < smin ? L.d[j] : smin;
-    }
-    const double lmax = gam + (smax > 0.0 ? smax : 0.0);
-    const double lmin = smin < 0.0 ? gam + smin : gam;
-    if (!(lmax > 0.0) || lmin < fabs(lmax) * 1.4901161193847656e-08) status |= LEKF_PT_RANKDEF;
-    // c_b = (gamma + s)^-1 U^T sqrt(w) d;  X' w-bar = (U^T B x')^T c_b
-    for (int j = lane; j < p; j += 64) L.U[j] = L.B[j] / (gam + L.d[j]);
-    __syncthreads();
-    for (int r = lane; r < nrow; r += 64) {
-        double s = 0.0;
-        for (int j = 0; j < p; ++j) s = fma(L.R[r * ks + j], L.U[j], s);
-        L.Cw[r] = s;
-    }
-    const bool want_wb = J.transm != nullptr;
-    if (want_wb)
-        for (int j = lane; j < p; j += 64) L.Wb[j] = L.U[j];
-    __syncthreads();
-    // (f(gamma + s) - f(gamma)) / s without cancellation
-    const double sg = sqrt(gam), skm1 = sqrt((double)(k - 1));
-    for (int w = lane; w < nrow * p; w += 64) {
-        const int r = w / p, j = w - r * p;
-        const double sgs = sqrt(gam + L.d[j]);
-        L.R[r * ks + j] *= -skm1 / (sg * sgs * (sg + sgs));
-    }
-    __syncthreads();
-    const VecSet Vb{L.R, nrow, ks, L.Wb, nullptr};
-    const int nvb = nrow + (want_wb ? 1 : 0);
-    if (!ovf) ql_back_vec(L, Vb, nvb, rbuf, rpos, lane);
-    big_refl_vecs<4>(rec, p, p, L.tau, Vb, nvb, false, lane);
-    __syncthreads();
-    // coefficients of the local obs rows: sqrt(w_i) times the p-vectors
-    for (int w = lane; w < nrow * p; w += 64) {
-        const int r = w / p, i = w - r * p;
-        L.R[r * ks + i] *= L.sw[i];
-    }
-    if (want_wb)
-        for (int i = lane; i < p; i += 64) L.Wb[i] *= L.sw[i];
-    __syncthreads();
-    if (want_wb) {
-        double acc[4] = {0.0, 0.0, 0.0, 0.0};
-        for (int i = 0; i < p; ++i) {
-            const long o = J.loc_idx[off + i];
-            const double c = L.Wb[i];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int m = lane + 64 * t;
-                if (m < k) acc[t] = fma(c, J.hdxf[o * J.y_so + (long)m * J.y_sm], acc[t]);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            if (lane + 64 * t < k) J.transm[(size_t)b * k + lane + 64 * t] = acc[t];
-    }
-    if (lane == 0 && J.infl_out)
-        J.infl_out[b] = (J.flags & LEKF_F_FIXED_INFL) ? J.infl_fixed
-                                                      : adaptive_alpha(alpha, p1, p2, p3);
-    if (lane == 0 && J.status) J.status[b] = status;
-    if (nrow == 0) return;
-    const uint32_t mask = J.upd_mask ? J.upd_mask[lev] : 0xffffffffu;
-    const double fg = sqrt((double)(k - 1) / gam);
-    for (int r = 0; r < nrow; ++r) {
-        const bool upd = (r >= n3) || ((mask >> r) & 1u);
-        double acc[4] = {0.0, 0.0, 0.0, 0.0};
-        if (upd)
+        for (int u = 0; u < kRows; ++u) acc[u] = 0.0;
+        if (dual)
+#pragma unroll 4
             for (int i = 0; i < p; ++i) {
-                const long o = J.loc_idx[off + i];
-                const double c = L.R[r * ks + i];
+                const double y = J.hdxf[J.loc_idx[off + i] * (long)J.y_so + (long)m * J.y_sm];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int m = lane + 64 * t;
-                    if (m < k) acc[t] = fma(c, J.hdxf[o * J.y_so + (long)m * J.y_sm], acc[t]);
-                }
+                for (int u = 0; u < kRows; ++u)
+                    if (r0 + u < nrow) acc[u] = fma(L.R[(r0 + u) * ks + i], y, acc[u]);
             }
-        double* dst = (r < n3) ? J.x3a + ((size_t)b * n3 + r) * k
-                               : J.x2a + ((size_t)ij * J.nv2d + (r - n3)) * k;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int m = lane + 64 * t;
-            if (m < k) {
-                const double xp = L.X[r * k + m];
-                dst[m] = upd ? L.M[r] + (L.Cw[r] + fma(fg, xp, acc[t])) : L.M[r] + xp;
-            }
+        for (int u = 0; u < kRows; ++u) {
+            const int r = r0 + u;
+            if (r >= nrow) break;
+            const bool upd = (r >= n3) || ((mask >> r) & 1u);
+            const double xp = L.X[r * k + m];
+            double a;
+            if (!upd)
+                a = L.M[r] + xp;
+            else if (dual)
+                a = L.M[r] + (L.Cw[r] + fma(fg, xp, acc[u]));
+            else if (p > 0)
+                a = L.M[r] + (L.Cw[r] + L.R[r * ks + m]);
+            else
+                a = L.M[r] + sa * xp;
+            double* dst = (r < n3) ? J.x3a + ((size_t)b * n3 + r) * k
+                                   : J.x2a + ((size_t)ij * J.nv2d + (r - n3)) * k;
+            dst[m] = a;
         }
     }
 }
@@ -2434,21 +2560,10 @@ __device__ void eig_replay(EigLds& L, int n, int lda, int lane, const double* re
 
 template <int KR, int BIG, bool REPLAY = false>
 __device__ void eig_point(const LekfJob& J, int b, double* const rec, long gstride, int nvmax,
-                          long rot_off, double* smem, int lane, const SplitRec* SR = nullptr)
+                          double* smem, int lane, const SplitRec* SR = nullptr)
 {
     const int k = J.k, lda = BIG ? k : eig_lda(k);
     EigLds L = eig_carve(smem, k, nvmax, BIG ? rec : nullptr);
-    if constexpr (BIG > 0) {
-        if (!J.trans && !J.pao) {
-            const long o0 = J.loc_off[b];
-            const int pp = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - o0);
-            if (big_dual(J, pp, k))
-                big_dual_point(J, b, rec, rec + rot_off, gstride - rot_off, L, lane);
-            else
-                big_vec_point(J, b, rec, rec + rot_off, gstride - rot_off, L, lane);
-            return;
-        }
-    }
     // Z_ij (component i of eigenvector j once the eigendecomposition is done)
     auto Zv = [&](int i, int j) -> double {
         return BIG ? L.Z[i + (size_t)j * lda] : L.Z[i * lda + j];
@@ -2643,7 +2758,7 @@ void lekf_eig_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
     const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
     if (!all && !J.trans && !J.pao) return;  // lekf_trd_kernel's
     eig_point<KR, 0>(J, (int)(gp - J.pt_begin + J.pt0), ws + (gp - gp0) * gstride, gstride, nvmax,
-                     0L, smem, threadIdx.x);
+                     smem, threadIdx.x);
 }
 
 // --- split eigensolver, 32 < k <= 64 --------------------------------------
@@ -2829,7 +2944,7 @@ void lekf_eig3_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
     const SplitRec S = split_rec(kmax, rot + slot * 2 * split_rcap(kmax));
     // no local obs: pass 0 writes the outputs; else the pass the flag names
     if (p <= 0 ? pass != 0 : split_other_pass(rec, S.flagoff, pass)) return;
-    eig_point<KR, 0, true>(J, b, rec, gstride, nvmax, 0L, smem, threadIdx.x, &S);
+    eig_point<KR, 0, true>(J, b, rec, gstride, nvmax, smem, threadIdx.x, &S);
     if (pass && threadIdx.x == 0 && J.status) J.status[b] |= LEKF_PT_FP64;
 }
 
@@ -2868,7 +2983,7 @@ __global__ __launch_bounds__(64) void lekf_eig_fix_kernel(const LekfJob* __restr
         const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
         const int b = (int)(gp - J.pt_begin + J.pt0);
         __syncthreads();
-        eig_point<KR, 0>(J, b, ws + slot * gstride, gstride, nvmax, 0L, smem, threadIdx.x);
+        eig_point<KR, 0>(J, b, ws + slot * gstride, gstride, nvmax, smem, threadIdx.x);
         if (pass && threadIdx.x == 0 && J.status) J.status[b] |= LEKF_PT_FP64;
     }
 }
@@ -2882,19 +2997,52 @@ __global__ __launch_bounds__(64) void lekf_eig_fix_kernel(const LekfJob* __restr
 template <int MODE>
 __global__ __launch_bounds__(64) void lekf_big_kernel(const LekfJob* __restrict__ jobs, int njobs,
                                                       long npt, double* __restrict__ ws,
-                                                      long gstride, int nvmax, long rot_off,
-                                                      int nblk)
+                                                      long gstride, int nvmax, int nblk)
 {
     extern __shared__ double smem[];
     const int lane = threadIdx.x;
     double* const rec = ws + (size_t)blockIdx.x * gstride;
     for (long gp = blockIdx.x; gp < npt; gp += gridDim.x) {
         const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
+        if (!J.trans && !J.pao) continue;  // lekf_bigvec_kernel's
         const int b = (int)(gp - J.pt_begin + J.pt0);
         __syncthreads();  // the previous point is done with the record
         for (int t = 0; t < nblk; ++t) gram_blk_point<MODE>(J, b, t, rec, lane);
         __syncthreads();
-        eig_point<0, 4>(J, b, rec, gstride, nvmax, rot_off, smem, lane);
+        eig_point<0, 4>(J, b, rec, gstride, nvmax, smem, lane);
+    }
+}
+
+// The same for the jobs that output neither trans nor pao, kBigW waves per point.
+// The k x k matrix stays in global memory, so a wave alone waits for it; four waves share
+// the rows, the blocks of the Gram and the vectors, and at <= 256 registers two
+// workgroups fit a CU.  QL's scalar recurrence was half of a point's time: the rational
+// form of the functions of T takes its place (big_function).  48 x 24 x 7 points,
+// k = 256: 505 ms with one wave and QL, 116 ms with four waves and the rational form, 73 ms
+// with two workgroups per CU and the Gram's empty tiles left out; 960 points, k = 200,
+// p = 21: 0.60, 0.84 and 0.41 ms.  Bound by the traffic of the reduction (k^3 / 6 values
+// read and written per point) and its 2 barriers per step.
+template <int MODE>
+__global__ __launch_bounds__(64 * kBigW) __attribute__((amdgpu_waves_per_eu(2)))
+void lekf_bigvec_kernel(const LekfJob* __restrict__ jobs,
+                                                                 int njobs, long npt,
+                                                                 double* __restrict__ ws,
+                                                                 long gstride, int nvmax, int kmax)
+{
+    extern __shared__ double smem[];
+    const int tid = threadIdx.x, nblk = gram_nblk(kmax);
+    const long rot_off = gram_stride(kmax);
+    double* const rec = ws + (size_t)blockIdx.x * gstride;
+    for (long gp = blockIdx.x; gp < npt; gp += gridDim.x) {
+        const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
+        if (J.trans || J.pao) continue;
+        const int b = (int)(gp - J.pt_begin + J.pt0);
+        __syncthreads();  // the previous point is done with the record and the LDS
+        for (int t = tid / 64; t < nblk; t += kBigW)
+            gram_blk_point<MODE>(J, b, t, rec, tid & 63);
+        __syncthreads();
+        EigLds L = eig_carve(smem, J.k, nvmax, rec);
+        big_vec_point<MODE>(J, b, rec, rec + rot_off, gstride - rot_off, L, tid);
     }
 }
 
@@ -3164,23 +3312,32 @@ static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int km
 // workspace record
 template <int MODE>
 static hipError_t launch_big(const LekfJob* djobs, int njobs, long npt, int kmax, int nvmax,
-                             void* ws, size_t ws_bytes, hipStream_t st)
+                             int outs, void* ws, size_t ws_bytes, hipStream_t st)
 {
     const long gs = big_stride(kmax);
     const long slots = (long)(ws_bytes / ((size_t)gs * sizeof(double)));
     if (slots < 1 || !ws) return hipErrorInvalidValue;
     const size_t elds = eig_lds_doubles_big(kmax, nvmax) * sizeof(double);
-    // as many workgroups as can be resident at once (LDS bounds the count)
-    int dev = 0, ncu = 256, per_cu = 1;
+    int dev = 0, ncu = 256;
     if (hipGetDevice(&dev) == hipSuccess)
         (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lekf_big_kernel<MODE>, LEKF_WAVE, elds);
-    long nwg = (long)(per_cu > 0 ? per_cu : 1) * (ncu > 0 ? ncu : 256);
-    if (nwg > slots) nwg = slots;
-    if (nwg > npt) nwg = npt;
+    // as many workgroups as can be resident at once (LDS bounds the count)
+    auto count = [&](const void* fn, int threads) {
+        int per_cu = 1;
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, elds);
+        const long nwg = (long)(per_cu > 0 ? per_cu : 1) * (ncu > 0 ? ncu : 256);
+        return dim3((unsigned)std::min(std::min(nwg, slots), npt));
+    };
     KTime kt("big", st);
-    hipLaunchKernelGGL((lekf_big_kernel<MODE>), dim3((unsigned)nwg), dim3(LEKF_WAVE), elds, st, djobs,
-                       njobs, npt, (double*)ws, gs, nvmax, (long)gram_stride(kmax), gram_nblk(kmax));
+    if (outs & LEKF_OUT_PLAIN)
+        hipLaunchKernelGGL((lekf_bigvec_kernel<MODE>),
+                           count((const void*)lekf_bigvec_kernel<MODE>, 64 * kBigW),
+                           dim3(64 * kBigW), elds, st, djobs, njobs, npt, (double*)ws, gs, nvmax,
+                           kmax);
+    if (outs & LEKF_OUT_TRANS)
+        hipLaunchKernelGGL((lekf_big_kernel<MODE>),
+                           count((const void*)lekf_big_kernel<MODE>, LEKF_WAVE), dim3(LEKF_WAVE),
+                           elds, st, djobs, njobs, npt, (double*)ws, gs, nvmax, gram_nblk(kmax));
     return hipGetLastError();
 }
 
@@ -3197,7 +3354,7 @@ static hipError_t launch_mode(int cls, const LekfJob* djobs, int njobs, long npt
     case 24 * 8 + 2: return launch_fused<2, 24, MODE>(djobs, njobs, npt, kmax, nvmax, st);
     case 28 * 8 + 2: return launch_fused<2, 28, MODE>(djobs, njobs, npt, kmax, nvmax, st);
     case 32 * 8 + 3: return launch_fused<3, 32, MODE>(djobs, njobs, npt, kmax, nvmax, st);
-    case kClassBig: return launch_big<MODE>(djobs, njobs, npt, kmax, nvmax, ws, ws_bytes, st);
+    case kClassBig: return launch_big<MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
     default:
         if (kmax > 32 && kmax <= LEKF_KSPLIT)
             return launch_split<MODE>(djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);

@@ -2559,7 +2559,7 @@ __device__ void eig_replay(EigLds& L, int n, int lda, int lane, const double* re
 }
 
 template <int KR, int BIG, bool REPLAY = false>
-__device__ void eig_point(const LekfJob& J, int b, double* const rec, long gstride, int nvmax,
+__device__ __forceinline__ void eig_point(const LekfJob& J, int b, double* const rec, long gstride, int nvmax,
                           double* smem, int lane, const SplitRec* SR = nullptr)
 {
     const int k = J.k, lda = BIG ? k : eig_lda(k);

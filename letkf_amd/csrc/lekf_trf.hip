@@ -100,6 +100,7 @@ void lekf_trd_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
                      double* __restrict__ ws, long gstride, int nvmax, int kmax, int pass,
                      int mode, double kthr, int* __restrict__ rlist, long lcap)
 {
+#pragma clang fp contract(off)
     extern __shared__ double smem[];
     constexpr int P = 8, LD = trf_ld(P, NB);
     long gp;
@@ -263,6 +264,7 @@ void lekf_trf_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
                      const double* __restrict__ ws, long gstride, int nvmax, int kmax, int pass,
                      const int* __restrict__ rlist)
 {
+#pragma clang fp contract(off)
     extern __shared__ __align__(16) double smem[];
     constexpr int P = 8, KP = P * NB, ldz = trf_ldz(KP);
     long gp;

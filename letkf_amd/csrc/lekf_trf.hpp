@@ -18,7 +18,9 @@
 // (which gives the reflector in both directions, M being symmetric), and all sums
 // over grid rows or columns are DPP butterflies.  The reflectors stay in M's
 // finished rows.  Sums run in an order that depends on the indices alone, and
-// slots past k add exact zeros, so a point's bits do not depend on the launch.
+// slots past k add exact zeros; products are fused into sums only where an fma is
+// written (the compiler's own choice differs between numbers of slots, which come from
+// the launch's largest k), so a point's bits do not depend on the launch.
 #pragma once
 #include "lekf_dev.hpp"
 #include "lekf_invsqrt.hpp"
@@ -105,6 +107,7 @@ __device__ __forceinline__ void trf_stage(double (&M)[NB][NB], double (&X)[NE][N
                                           int r, int c, int lane, double* vx, double* vw,
                                           double* es, double* ts, bool& bad)
 {
+#pragma clang fp contract(off)
     constexpr int LD = trf_ld(P, NB);
     constexpr int T1 = T + 1 < NB ? T + 1 : T;
 #pragma unroll 1
@@ -249,6 +252,7 @@ __device__ __forceinline__ void trf_function(const double* zrow, const double2* 
                                              int nmax, double m, double scale, int rb, int r, int c,
                                              double* tl, int ldt, double (&out)[NB])
 {
+#pragma clang fp contract(off)
 #pragma unroll
     for (int b = 0; b < NB; ++b) out[b] = 0.0;
     const int N = 8 + 4 * lev;
@@ -306,6 +310,7 @@ template <int T, int P, int NB, int NE>
 __device__ __forceinline__ void trf_back_stage(double (&out)[NE][NB], int k, int kw, int c,
                                                const double* vst, const double* ts)
 {
+#pragma clang fp contract(off)
     constexpr int LD = trf_ld(P, NB);
 #pragma unroll 1
     for (int u = P - 1; u >= 0; --u) {

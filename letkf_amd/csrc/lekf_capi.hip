@@ -208,8 +208,7 @@ int run_solve(const lekf_job* djobs, int njobs, long npt, int kmax, int nvmax, i
 // state rows a job's points apply their transform to (0 without the apply)
 int job_rows(const lekf_job& j) { return (j.flags & LEKF_F_APPLY) ? j.nv3d + j.nv2d : 0; }
 
-// whether a job asks for the k x k outputs
-int job_outs(const lekf_job& j) { return j.trans || j.pao ? LEKF_OUT_TRANS : LEKF_OUT_PLAIN; }
+int job_outs(const lekf_job& j) { return lekf_solve_outs(j.k, j.trans || j.pao); }
 
 // The grouped launches of launch_grouped over caller-provided device memory:
 // descriptors at dj (room for J.size()), workspace ws of ws_bytes.  Nothing is
@@ -619,7 +618,7 @@ int lekf_core_f64(int ne, int nobs, int nobsl, const double* hdxb, const double*
     J.pao = pao ? c.pa.as<double>() : nullptr;
     J.status = c.stat.as<int>();
     HIPCHK(hipMemcpyAsync(c.job.p, &J, sizeof(J), hipMemcpyHostToDevice, st));
-    rc = run_solve(c.job.as<lekf_job>(), 1, 1, ne, 0, 0, LEKF_OUT_TRANS, c.gws, st);
+    rc = run_solve(c.job.as<lekf_job>(), 1, 1, ne, 0, 0, job_outs(J), c.gws, st);
     if (rc) return rc;
     int pst = 0;
     HIPCHK(hipMemcpyAsync(trans, c.tr.p, sizeof(double) * k * k, hipMemcpyDeviceToHost, st));

@@ -80,5 +80,6 @@ hipError_t lekf_logpfm_launch(const double* x2b, int nij, int nv2d, int ips, int
 size_t lekf_solve_lds_bytes(int k, int nvmax);
 size_t lekf_solve_ws_bytes(long npt, int kmax, int outs);
 int lekf_solve_class(int k);
+int lekf_solve_outs(int k, bool kxk);
 hipError_t lekf_solve_launch(const LekfJob* djobs, int njobs, long npt, int kmax, int nvmax,
                              int mode, int outs, void* ws, size_t ws_bytes, hipStream_t st);

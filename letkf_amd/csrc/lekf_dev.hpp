@@ -59,9 +59,11 @@ __device__ __forceinline__ double rn_div(double a, double b)
     return a / b;
 }
 
-// what the jobs of a solve launch ask for: any without trans and pao, any with
+// what the jobs of a solve launch ask for: any without trans and pao, any with; and, from
+// bit LEKF_OUT_CUT0 on, the cuts of the Gram's columns (gram_cut) among them
 #define LEKF_OUT_PLAIN 1
 #define LEKF_OUT_TRANS 2
+#define LEKF_OUT_CUT0 8
 
 // Reciprocal and reciprocal square root: hardware estimate refined by Newton
 // steps to full FP64 accuracy (a Jacobi rotation only needs c^2 + s^2 = 1 to

@@ -84,6 +84,7 @@ void lekf_gram_f64_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
     extern __shared__ double smem[];
     GramPoint P;
     if (!gram_point(jobs, njobs, gp0, rlist, zlist, P)) return;
+    if (gram_ntf(P.k) != NTF || gram_ns(P.k) != NS) return;  // another launch's
     const LekfJob& J = *P.J;
     const int lane = threadIdx.x & (LEKF_WAVE - 1), wv = threadIdx.x / LEKF_WAVE;
     const int k = P.k, lda = k + 1;
@@ -124,6 +125,7 @@ void lekf_gram_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
     extern __shared__ double smem[];
     GramPoint P;
     if (!gram_point(jobs, njobs, gp0, rlist, zlist, P)) return;
+    if ((P.k + 16) / 16 != NT) return;  // another launch's
     const LekfJob& J = *P.J;
     const int lane = threadIdx.x & (LEKF_WAVE - 1), wv = threadIdx.x / LEKF_WAVE;
     const int k = P.k, lda = k + 1;
@@ -154,66 +156,88 @@ void lekf_gram_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
     gram_out<W>(A, B, sc, p3, k, ws + P.slot * gstride);
 }
 
+struct GramLaunch {
+    int W;
+    size_t lds;
+    unsigned nb;
+    hipStream_t st;
+    const LekfJob* djobs;
+    int njobs;
+    long g0;
+    double* ws;
+    long gs;
+    const int* rlist;
+    int* zlist;
+};
+using GramKernel = void (*)(const LekfJob*, int, long, double*, long, const int*, int*);
+
+// the form of a kernel for the waves asked for
+void gram_go(GramKernel w2, GramKernel w4, GramKernel w8, const GramLaunch& G)
+{
+    KTime kt(G.rlist ? "redo_gram" : "gram", G.st);
+    const int W = G.W == 2 || G.W == 8 ? G.W : 4;
+    hipLaunchKernelGGL(W == 2 ? w2 : W == 8 ? w8 : w4, dim3(G.nb), dim3(64 * W), G.lds, G.st,
+                       G.djobs, G.njobs, G.g0, G.ws, G.gs, G.rlist, G.zlist);
+}
+
+template <int NTF, int NS>
+void gram_f64_go(int cuts, const GramLaunch& G)
+{
+    if (cuts >> gram_cut(NTF, NS) & 1)
+        gram_go(lekf_gram_f64_kernel<NTF, NS, 2>, lekf_gram_f64_kernel<NTF, NS, 4>,
+                lekf_gram_f64_kernel<NTF, NS, 8>, G);
+}
+
+template <int NT, int MODE>
+void gram_mixed_go(int cuts, const GramLaunch& G)
+{
+    // NT tiles: NT whole ones, or strips after NT - 1
+    const int of = 1 << gram_cut(NT, 0) | 1 << gram_cut(NT - 1, 1) | 1 << gram_cut(NT - 1, 2);
+    if (cuts & of)
+        gram_go(lekf_gram_kernel<NT, MODE, 2>, lekf_gram_kernel<NT, MODE, 4>,
+                lekf_gram_kernel<NT, MODE, 8>, G);
+}
+
 }  // namespace
 
-hipError_t lekf_gram_launch(int mode, int W, int kmax, long nb, hipStream_t st,
+// The jobs of a launch may have several cuts: each has its own kernel, whose workgroups
+// leave the other points alone.  (Splitting the batch by cut instead repeats the solve's
+// other kernels too, whose latencies do not shrink with it: 15 trans jobs of k = 33..47,
+// two points each, take 1.7 ms in one launch and took 3.7 ms split.)
+hipError_t lekf_gram_launch(int mode, int W, int kmax, int outs, long nb, hipStream_t st,
                             const LekfJob* djobs, int njobs, long g0, double* ws, long gs,
                             const int* rlist, int* zlist)
 {
-    KTime kt(rlist ? "redo_gram" : "gram", st);
-    const size_t lds = gram_lds_doubles(kmax, W) * sizeof(double);
-#define LEKF_GRAM_W(K, W)                                                                        \
-    hipLaunchKernelGGL((K), dim3((unsigned)nb), dim3(64 * W), lds, st, djobs, njobs, g0, ws, gs, \
-                       rlist, zlist)
-#define LEKF_GRAM_F64(T, S)                                                                      \
-    case 8 * T + S:                                                                              \
-        if (W == 2)                                                                              \
-            LEKF_GRAM_W((lekf_gram_f64_kernel<T, S, 2>), 2);                                     \
-        else if (W == 8)                                                                         \
-            LEKF_GRAM_W((lekf_gram_f64_kernel<T, S, 8>), 8);                                     \
-        else                                                                                     \
-            LEKF_GRAM_W((lekf_gram_f64_kernel<T, S, 4>), 4);                                     \
+    const GramLaunch G{W, gram_lds_doubles(kmax, W) * sizeof(double), (unsigned)nb, st, djobs,
+                       njobs, g0, ws, gs, rlist, zlist};
+    const int cuts = outs >> LEKF_OUT_CUT0;
+    if (cuts <= 0 || cuts >> kGramCuts) return hipErrorInvalidValue;
+    switch (mode) {
+    case 0:
+        gram_f64_go<2, 1>(cuts, G);
+        gram_f64_go<2, 2>(cuts, G);
+        gram_f64_go<3, 0>(cuts, G);
+        gram_f64_go<3, 1>(cuts, G);
+        gram_f64_go<3, 2>(cuts, G);
+        gram_f64_go<4, 0>(cuts, G);
+        gram_f64_go<4, 1>(cuts, G);
+        gram_f64_go<4, 2>(cuts, G);
+        gram_f64_go<5, 0>(cuts, G);
+        gram_f64_go<5, 1>(cuts, G);
+        gram_f64_go<5, 2>(cuts, G);
+        gram_f64_go<6, 0>(cuts, G);
         break;
-#define LEKF_GRAM_MIXED(T, M)                                                                    \
-    case 8 * T + M:                                                                              \
-        if (W == 2)                                                                              \
-            LEKF_GRAM_W((lekf_gram_kernel<T, M, 2>), 2);                                         \
-        else if (W == 8)                                                                         \
-            LEKF_GRAM_W((lekf_gram_kernel<T, M, 8>), 8);                                         \
-        else                                                                                     \
-            LEKF_GRAM_W((lekf_gram_kernel<T, M, 4>), 4);                                         \
+    case 1:
+        gram_mixed_go<3, 1>(cuts, G);
+        gram_mixed_go<4, 1>(cuts, G);
+        gram_mixed_go<5, 1>(cuts, G);
+        gram_mixed_go<6, 1>(cuts, G);
         break;
-    if (mode == 0) {
-        switch (8 * gram_ntf(kmax) + gram_ns(kmax)) {
-            LEKF_GRAM_F64(2, 1)
-            LEKF_GRAM_F64(2, 2)
-            LEKF_GRAM_F64(3, 0)
-            LEKF_GRAM_F64(3, 1)
-            LEKF_GRAM_F64(3, 2)
-            LEKF_GRAM_F64(4, 0)
-            LEKF_GRAM_F64(4, 1)
-            LEKF_GRAM_F64(4, 2)
-            LEKF_GRAM_F64(5, 0)
-            LEKF_GRAM_F64(5, 1)
-            LEKF_GRAM_F64(5, 2)
-            LEKF_GRAM_F64(6, 0)
-        default: return hipErrorInvalidValue;
-        }
-    } else {
-        switch (8 * ((kmax + 16) / 16) + mode) {
-            LEKF_GRAM_MIXED(3, 1)
-            LEKF_GRAM_MIXED(4, 1)
-            LEKF_GRAM_MIXED(5, 1)
-            LEKF_GRAM_MIXED(6, 1)
-            LEKF_GRAM_MIXED(3, 2)
-            LEKF_GRAM_MIXED(4, 2)
-            LEKF_GRAM_MIXED(5, 2)
-            LEKF_GRAM_MIXED(6, 2)
-        default: return hipErrorInvalidValue;
-        }
+    default:
+        gram_mixed_go<3, 2>(cuts, G);
+        gram_mixed_go<4, 2>(cuts, G);
+        gram_mixed_go<5, 2>(cuts, G);
+        gram_mixed_go<6, 2>(cuts, G);
     }
-#undef LEKF_GRAM_MIXED
-#undef LEKF_GRAM_F64
-#undef LEKF_GRAM_W
     return hipGetLastError();
 }

@@ -314,6 +314,10 @@ __host__ __device__ constexpr int gram_ns(int k)
     return r <= 0 ? 0 : (r + 3) / 4;
 }
 
+// the cuts of 32 < k <= 95, numbered
+constexpr int kGramCuts = 13;
+__host__ __device__ constexpr int gram_cut(int ntf, int ns) { return 3 * (ntf - 2) + ns; }
+
 template <int NTF, int NS>
 struct GramAcc {
     static constexpr int NT = NTF * (NTF + 1) / 2;
@@ -460,7 +464,8 @@ __device__ __forceinline__ void store_strips(const GramAcc<NTF, NS>& G, int k, i
 
 }  // namespace
 
-// the Gram of nb slots into the workspace records (lekf_gram.hip)
-hipError_t lekf_gram_launch(int mode, int W, int kmax, long nb, hipStream_t st,
+// the Gram of nb slots into the workspace records (lekf_gram.hip), one launch per form
+// that the jobs' sizes take (outs: their cuts)
+hipError_t lekf_gram_launch(int mode, int W, int kmax, int outs, long nb, hipStream_t st,
                             const LekfJob* djobs, int njobs, long g0, double* ws, long gs,
                             const int* rlist, int* zlist);

@@ -3052,8 +3052,10 @@ void lekf_bigvec_kernel(const LekfJob* __restrict__ jobs,
 // host-side launchers (called from lekf_capi.hip)
 // ---------------------------------------------------------------------------
 // Kernel class of an ensemble size: KR * 8 + NT for k <= 32 (register
-// Jacobi, KR = k rounded up to a multiple of 4); the Gram's column tiles and strips for
-// k <= LEKF_KSPLIT; kClassBig above (block Gram + eigensolver in global memory).
+// Jacobi, KR = k rounded up to a multiple of 4); for k <= LEKF_KSPLIT the 16-column tiles of
+// k + 1 columns, but 64 with the sizes below it (up to 64 the eigensolvers hold the matrix
+// in registers, above in LDS, and only the former redo mixed-precision points in FP64);
+// kClassBig above (block Gram + eigensolver in global memory).
 constexpr int kClassBig = 1000;
 
 int lekf_solve_class(int k)
@@ -3064,8 +3066,16 @@ int lekf_solve_class(int k)
         return kr * 8 + nt;
     }
     if (k > LEKF_KSPLIT) return kClassBig;
-    // every job of a launch has the same cut of the Gram's columns
-    return 500 + 8 * gram_ntf(k) + gram_ns(k);
+    return 500 + ((k == 64 ? 63 : k) + 16) / 16;
+}
+
+// what a job of ensemble size k adds to its launch's outs; kxk: it outputs trans or pao
+int lekf_solve_outs(int k, bool kxk)
+{
+    int outs = kxk ? LEKF_OUT_TRANS : LEKF_OUT_PLAIN;
+    if (k > 32 && k <= LEKF_KSPLIT)
+        outs |= 1 << (LEKF_OUT_CUT0 + gram_cut(gram_ntf(k), gram_ns(k)));
+    return outs;
 }
 
 // points per wave of the fused kernel for Jacobi rows KR: lane groups of KR,
@@ -3291,16 +3301,16 @@ static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int km
     };
     for (long g0 = 0; g0 < npt; g0 += per) {
         const long nb = per < npt - g0 ? per : npt - g0;
-        hipError_t e = lekf_gram_launch(MODE, W, kmax, nb, st, djobs, njobs, g0, (double*)ws, gs,
-                                        nullptr, g0 == 0 ? rlist : nullptr);
+        hipError_t e = lekf_gram_launch(MODE, W, kmax, outs, nb, st, djobs, njobs, g0, (double*)ws,
+                                        gs, nullptr, g0 == 0 ? rlist : nullptr);
         if (e == hipSuccess) e = solve(g0, nb, 0, kthr);
         if (e != hipSuccess) return e;
     }
     if (kthr > 0.0) {
         // grids of one sub-batch; the slots past the list's length return at once
         const long nl = per < npt ? per : npt;
-        hipError_t e = lekf_gram_launch(0, W, kmax, nl, st, djobs, njobs, 0, (double*)ws, gs, rlist,
-                                        nullptr);
+        hipError_t e = lekf_gram_launch(0, W, kmax, outs, nl, st, djobs, njobs, 0, (double*)ws, gs,
+                                        rlist, nullptr);
         if (e == hipSuccess) e = solve(0, nl, 1, 0.0);
         if (e != hipSuccess) return e;
     }
@@ -3364,9 +3374,9 @@ static hipError_t launch_mode(int cls, const LekfJob* djobs, int njobs, long npt
 
 // Launch the solve over npt flat points of njobs jobs (device array djobs).
 // Every job of a launch has the same kernel class; kmax (the largest k) and
-// nvmax (the most state rows a point applies to) size the LDS; outs: whether any
-// of them outputs trans or pao, and whether any does not; ws is the Gram workspace
-// of lekf_solve_ws_bytes(npt, kmax, outs) bytes (k > 32).
+// nvmax (the most state rows a point applies to) size the LDS; outs: the jobs'
+// lekf_solve_outs together; ws is the Gram workspace of lekf_solve_ws_bytes(npt, kmax,
+// outs) bytes (k > 32).
 hipError_t lekf_solve_launch(const LekfJob* djobs, int njobs, long npt, int kmax, int nvmax,
                              int mode, int outs, void* ws, size_t ws_bytes,
                              hipStream_t st)

@@ -1,11 +1,12 @@
-"""Jobs of different ensemble sizes and outputs in one batch (32 < k <= 95): they share
-records, flags and the FP64 redo list, and every job's outputs equal, bit for bit, those
-of the same job launched alone.
+"""Jobs of different ensemble sizes and outputs in one batch (32 < k <= 95): jobs of one
+kernel class share the solve's launches, the Gram taking one launch per column cut, and
+jobs with and without trans share records, flags and the FP64 redo list.  Every job's
+outputs equal, bit for bit, those of the same job launched alone.
 """
 import numpy as np
 import pytest
 
-from letkf_amd import _lib, core, tune
+from letkf_amd import _lib, core, device, tune
 from letkf_amd.device import DeviceArray, sync
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +79,19 @@ def test_job_alone_equals_job_in_batch(gpu, knobs, specs, prec):
         redone = (b["status"] & _lib.LEKF_PT_FP64) != 0
         assert redone.any() == (prec != "f64" and k <= 64), (k, tr)
         assert not redone.all()
+
+
+@pytest.mark.parametrize("ks", [range(33, 48), range(48, 65)])
+def test_one_solve_launch_per_class(gpu, ks):
+    """Trans jobs of one class: one tridiagonalisation, QL and apply for all of them, and
+    one Gram launch per cut of the columns."""
+    js = [_job(k, True, k, "f64") for k in ks]
+    sync()
+    device.ktime_enable(True)
+    core.letkf_core_batch([j for j, _ in js], "f64")
+    sync()
+    kt = device.ktime_all()
+    device.ktime_enable(False)
+    assert {n: kt[n][1] for n in ("eig_tri", "eig_ql", "eig_apply")} == \
+        {"eig_tri": 1, "eig_ql": 1, "eig_apply": 1}
+    assert 1 <= kt["gram"][1] <= 4  # k + 1 = 33 .. 48 or 49 .. 65 columns: three or four cuts

@@ -2559,8 +2559,9 @@ __device__ void eig_replay(EigLds& L, int n, int lda, int lane, const double* re
 }
 
 template <int KR, int BIG, bool REPLAY = false>
-__device__ __forceinline__ void eig_point(const LekfJob& J, int b, double* const rec, long gstride, int nvmax,
-                          double* smem, int lane, const SplitRec* SR = nullptr)
+__device__ __forceinline__ void eig_point(const LekfJob& J, int b, double* const rec, long gstride,
+                                          int nvmax, double* smem, int lane,
+                                          const SplitRec* SR = nullptr)
 {
     const int k = J.k, lda = BIG ? k : eig_lda(k);
     EigLds L = eig_carve(smem, k, nvmax, BIG ? rec : nullptr);
@@ -2740,6 +2741,29 @@ __device__ __forceinline__ void eig_point(const LekfJob& J, int b, double* const
     }
 }
 
+// eig_point as a call of its own.  The register eigensolvers and the large-k one run
+// faster so than inlined into their kernels, where the loops over points and the job's
+// fields take scalar registers that the unrolled QL needs (177 to 401 of them spilled):
+// 1000 points, LEKF_TUNE_EIG_SPLIT = 0, k = 36 / 48 / 60: 0.56 / 0.90 / 1.24 ms against 0.62 /
+// 1.01 / 1.50 inlined; 600 points with trans, k = 120 / 200: 27.7 / 115 ms against 33.9 / 137.
+// The LDS eigensolver (KR = 0) is better inlined: 600 points with trans, k = 72 / 90: 7.1 /
+// 11.2 ms against 7.7 / 12.1.
+template <int KR, int BIG>
+__device__ __noinline__ void eig_point_call(const LekfJob& J, int b, double* rec, long gstride,
+                                            int nvmax, double* smem, int lane)
+{
+    eig_point<KR, BIG>(J, b, rec, gstride, nvmax, smem, lane);
+}
+template <int KR>
+__device__ __forceinline__ void eig_point_split(const LekfJob& J, int b, double* rec, long gstride,
+                                                int nvmax, double* smem, int lane)
+{
+    if constexpr (KR > 0)
+        eig_point_call<KR, 0>(J, b, rec, gstride, nvmax, smem, lane);
+    else
+        eig_point<KR, 0>(J, b, rec, gstride, nvmax, smem, lane);
+}
+
 // Waves per SIMD asked of the register eigen kernel: at KR = 40..48 the
 // register QL fits two waves per SIMD with a few spills, which hides more of
 // its latency than the spills cost (measured on the GFS-sized problem: the
@@ -2757,8 +2781,8 @@ void lekf_eig_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
     const long gp = gp0 + blockIdx.x;
     const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
     if (!all && !J.trans && !J.pao) return;  // lekf_trd_kernel's
-    eig_point<KR, 0>(J, (int)(gp - J.pt_begin + J.pt0), ws + (gp - gp0) * gstride, gstride, nvmax,
-                     smem, threadIdx.x);
+    eig_point_split<KR>(J, (int)(gp - J.pt_begin + J.pt0), ws + (gp - gp0) * gstride, gstride,
+                        nvmax, smem, threadIdx.x);
 }
 
 // --- split eigensolver, 32 < k <= 64 --------------------------------------
@@ -2983,7 +3007,7 @@ __global__ __launch_bounds__(64) void lekf_eig_fix_kernel(const LekfJob* __restr
         const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
         const int b = (int)(gp - J.pt_begin + J.pt0);
         __syncthreads();
-        eig_point<KR, 0>(J, b, ws + slot * gstride, gstride, nvmax, smem, threadIdx.x);
+        eig_point_split<KR>(J, b, ws + slot * gstride, gstride, nvmax, smem, threadIdx.x);
         if (pass && threadIdx.x == 0 && J.status) J.status[b] |= LEKF_PT_FP64;
     }
 }
@@ -3009,7 +3033,7 @@ __global__ __launch_bounds__(64) void lekf_big_kernel(const LekfJob* __restrict_
         __syncthreads();  // the previous point is done with the record
         for (int t = 0; t < nblk; ++t) gram_blk_point<MODE>(J, b, t, rec, lane);
         __syncthreads();
-        eig_point<0, 4>(J, b, rec, gstride, nvmax, smem, lane);
+        eig_point_call<0, 4>(J, b, rec, gstride, nvmax, smem, lane);
     }
 }
 

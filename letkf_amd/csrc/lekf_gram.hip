@@ -22,11 +22,15 @@ struct GramPoint {
     long slot, off;
 };
 __device__ __forceinline__ bool gram_point(const LekfJob* jobs, int njobs, long gp0,
-                                           const int* rlist, int* zlist, GramPoint& P)
+                                           const int* rlist, int* zlist, int* flist, GramPoint& P)
 {
     P.slot = blockIdx.x;
-    // the launch's first sub-batch empties the redo list before any kernel adds to it
-    if (zlist && blockIdx.x == 0 && threadIdx.x == 0) zlist[0] = 0;
+    // before any kernel adds to them: the launch's first sub-batch empties the redo list,
+    // every one the list of flagged slots
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (zlist) zlist[0] = 0;
+        flist[0] = 0;
+    }
     long gp = gp0 + P.slot;
     if (rlist) {  // FP64 pass of a split launch: slot i holds the redo list's i-th point
         if (P.slot >= rlist[0]) return false;
@@ -79,11 +83,11 @@ template <int NTF, int NS, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(gram_f64_waves(NTF, NS))))
 void lekf_gram_f64_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
                           double* __restrict__ ws, long gstride, const int* __restrict__ rlist,
-                          int* __restrict__ zlist)
+                          int* __restrict__ zlist, int* __restrict__ flist)
 {
     extern __shared__ double smem[];
     GramPoint P;
-    if (!gram_point(jobs, njobs, gp0, rlist, zlist, P)) return;
+    if (!gram_point(jobs, njobs, gp0, rlist, zlist, flist, P)) return;
     if (gram_ntf(P.k) != NTF || gram_ns(P.k) != NS) return;  // another launch's
     const LekfJob& J = *P.J;
     const int lane = threadIdx.x & (LEKF_WAVE - 1), wv = threadIdx.x / LEKF_WAVE;
@@ -120,11 +124,11 @@ template <int NT, int MODE, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(gram_waves_per_simd(NT, MODE))))
 void lekf_gram_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
                       double* __restrict__ ws, long gstride, const int* __restrict__ rlist,
-                      int* __restrict__ zlist)
+                      int* __restrict__ zlist, int* __restrict__ flist)
 {
     extern __shared__ double smem[];
     GramPoint P;
-    if (!gram_point(jobs, njobs, gp0, rlist, zlist, P)) return;
+    if (!gram_point(jobs, njobs, gp0, rlist, zlist, flist, P)) return;
     if ((P.k + 16) / 16 != NT) return;  // another launch's
     const LekfJob& J = *P.J;
     const int lane = threadIdx.x & (LEKF_WAVE - 1), wv = threadIdx.x / LEKF_WAVE;
@@ -168,8 +172,9 @@ struct GramLaunch {
     long gs;
     const int* rlist;
     int* zlist;
+    int* flist;
 };
-using GramKernel = void (*)(const LekfJob*, int, long, double*, long, const int*, int*);
+using GramKernel = void (*)(const LekfJob*, int, long, double*, long, const int*, int*, int*);
 
 // the form of a kernel for the waves asked for
 void gram_go(GramKernel w2, GramKernel w4, GramKernel w8, const GramLaunch& G)
@@ -177,7 +182,7 @@ void gram_go(GramKernel w2, GramKernel w4, GramKernel w8, const GramLaunch& G)
     KTime kt(G.rlist ? "redo_gram" : "gram", G.st);
     const int W = G.W == 2 || G.W == 8 ? G.W : 4;
     hipLaunchKernelGGL(W == 2 ? w2 : W == 8 ? w8 : w4, dim3(G.nb), dim3(64 * W), G.lds, G.st,
-                       G.djobs, G.njobs, G.g0, G.ws, G.gs, G.rlist, G.zlist);
+                       G.djobs, G.njobs, G.g0, G.ws, G.gs, G.rlist, G.zlist, G.flist);
 }
 
 template <int NTF, int NS>
@@ -206,10 +211,10 @@ void gram_mixed_go(int cuts, const GramLaunch& G)
 // two points each, take 1.7 ms in one launch and took 3.7 ms split.)
 hipError_t lekf_gram_launch(int mode, int W, int kmax, int outs, long nb, hipStream_t st,
                             const LekfJob* djobs, int njobs, long g0, double* ws, long gs,
-                            const int* rlist, int* zlist)
+                            const int* rlist, int* zlist, int* flist)
 {
     const GramLaunch G{W, gram_lds_doubles(kmax, W) * sizeof(double), (unsigned)nb, st, djobs,
-                       njobs, g0, ws, gs, rlist, zlist};
+                       njobs, g0, ws, gs, rlist, zlist, flist};
     const int cuts = outs >> LEKF_OUT_CUT0;
     if (cuts <= 0 || cuts >> kGramCuts) return hipErrorInvalidValue;
     switch (mode) {

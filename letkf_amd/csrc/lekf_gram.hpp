@@ -468,4 +468,4 @@ __device__ __forceinline__ void store_strips(const GramAcc<NTF, NS>& G, int k, i
 // that the jobs' sizes take (outs: their cuts)
 hipError_t lekf_gram_launch(int mode, int W, int kmax, int outs, long nb, hipStream_t st,
                             const LekfJob* djobs, int njobs, long g0, double* ws, long gs,
-                            const int* rlist, int* zlist);
+                            const int* rlist, int* zlist, int* flist);

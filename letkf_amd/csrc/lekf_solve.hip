@@ -2837,7 +2837,8 @@ __global__ __launch_bounds__(64) void lekf_ql_kernel(const LekfJob* __restrict__
                                                       long gstride, double* __restrict__ rot,
                                                       short* __restrict__ ridx, int kmax,
                                                       long rlim, int pass, double kthr,
-                                                      int* __restrict__ rlist, long lcap, int all)
+                                                      int* __restrict__ rlist, long lcap,
+                                                      int* __restrict__ flist, int all)
 {
     extern __shared__ double sm[];
     const int lane = threadIdx.x;
@@ -2944,6 +2945,7 @@ __global__ __launch_bounds__(64) void lekf_ql_kernel(const LekfJob* __restrict__
     }
     rec[S.cntoff] = (double)(nr < rcap ? nr : rcap);
     rec[S.flagoff] = (double)(bad | (nr > rcap ? kSplitOverflow : 0) | redo);
+    if (nr > rcap && (redo != 0) == (pass != 0)) split_flag_slot(flist, pt);
 }
 
 // Kernel 3 for jobs that output trans or pao (one wave per point): the
@@ -2972,36 +2974,24 @@ void lekf_eig3_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
     if (pass && threadIdx.x == 0 && J.status) J.status[b] |= LEKF_PT_FP64;
 }
 
-// The points of a launch that the other kernels flagged kSplitOverflow (a rotation
-// stream that overflowed, a condition number past the rational form's tables): the
-// fused eigen kernel's work, from the Gram still at the start of the record.  A
-// workgroup looks through 64 slots' flags and solves the flagged ones in turn.
+// The points of a sub-batch that the other kernels flagged and listed (a rotation stream
+// that overflowed, a condition number past the rational form's tables): the fused eigen
+// kernel's work, from the Gram still at the start of the record.  The workgroups stride
+// over the list, one point at a time, so a batch of which every point is listed takes the
+// fused kernel's time (300 points, k = 40 / 64 / 80: 0.68 / 1.4 / 4.5 ms; 30 / 72 / 271 when
+// a workgroup looked through 64 slots and solved the flagged ones in turn).
 template <int KR>
 __global__ __launch_bounds__(64) void lekf_eig_fix_kernel(const LekfJob* __restrict__ jobs,
                                                            int njobs, long gp0, long nb,
                                                            double* __restrict__ ws, long gstride,
-                                                           int nvmax, int kmax, int pass, int all,
-                                                           const int* __restrict__ rlist)
+                                                           int nvmax, int pass,
+                                                           const int* __restrict__ rlist,
+                                                           const int* __restrict__ flist)
 {
     extern __shared__ double smem[];
-    const long slot0 = (long)blockIdx.x * 64;
-    bool mine = false;
-    {
-        const long slot = slot0 + threadIdx.x;
-        long gp;
-        if (slot < nb && split_slot_point(slot, gp0, nb, pass, rlist, gp)) {
-            const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
-            const int b = (int)(gp - J.pt_begin + J.pt0);
-            const int p = J.loc_cnt ? J.loc_cnt[b] : (int)(J.loc_off[b + 1] - J.loc_off[b]);
-            // (points that no kernel of this launch flags have no flag to read)
-            if (p > 0 && (all || (!J.trans && !J.pao))) {
-                const int flag = (int)ws[slot * gstride + gram_stride(kmax)];
-                mine = (flag & kSplitOverflow) && ((flag & kSplitRedo) != 0) == (pass != 0);
-            }
-        }
-    }
-    for (unsigned long long left = __ballot(mine); left; left &= left - 1) {
-        const long slot = slot0 + (__ffsll(left) - 1);
+    const int n = flist[0];
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        const long slot = flist[1 + i];
         long gp;
         (void)split_slot_point(slot, gp0, nb, pass, rlist, gp);
         const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
@@ -3151,12 +3141,12 @@ static long split_rec_stride(int kmax, const SplitPlan& P)
 }
 
 // bytes per point of a sub-batch: the record, the rotation stream where one is
-// recorded, a redo-list entry
+// recorded, entries of the redo list and of the flagged slots' list
 static size_t ws_rec_bytes(int kmax, int outs)
 {
     if (kmax > LEKF_KSPLIT) return (size_t)big_stride(kmax) * sizeof(double);
     const SplitPlan P = split_plan(kmax, outs);
-    long n = split_rec_stride(kmax, P) + 1;
+    long n = split_rec_stride(kmax, P) + 2;  // (per + 1 ints each: 2 per + 2 <= 4 per)
     if (P.streams) n += 2 * split_rcap(kmax) + split_ridx_doubles(kmax);
     return (size_t)n * sizeof(double);
 }
@@ -3218,7 +3208,7 @@ static hipError_t launch_eig(int kr, long nb, size_t elds, hipStream_t st, const
 static hipError_t launch_streams(int kr, long nb, size_t elds, hipStream_t st,
                                  const LekfJob* djobs, int njobs, long g0, double* ws, long gs,
                                  int nvmax, int kmax, double* rot, short* ridx, int pass,
-                                 double kthr, int* rlist, long lcap, int all)
+                                 double kthr, int* rlist, long lcap, int* flist, int all)
 {
     const unsigned nwq = (unsigned)((nb + 63) / 64);
     const size_t qlds = 2 * (size_t)kr * 64 * sizeof(double);
@@ -3235,7 +3225,7 @@ static hipError_t launch_streams(int kr, long nb, size_t elds, hipStream_t st,
             KTime kt(pass ? "redo_ql" : "eig_ql", st);                                           \
             hipLaunchKernelGGL(lekf_ql_kernel<K>, dim3(nwq), dim3(LEKF_WAVE), qlds, st, djobs,    \
                                njobs, g0, nb, ws, gs, rot, ridx, kmax,                           \
-                               g_lekf_tune.split_rcap, pass, kthr, rlist, lcap, all);           \
+                               g_lekf_tune.split_rcap, pass, kthr, rlist, lcap, flist, all);    \
         }                                                                                        \
         KTime kt(pass ? "redo_apply" : "eig_apply", st);                                         \
         hipLaunchKernelGGL(lekf_eig3_kernel<K>, dim3((unsigned)nb), dim3(LEKF_WAVE), elds, st,    \
@@ -3257,15 +3247,16 @@ static hipError_t launch_streams(int kr, long nb, size_t elds, hipStream_t st,
 }
 
 static hipError_t launch_fix(int kr, long nb, size_t elds, hipStream_t st, const LekfJob* djobs,
-                             int njobs, long g0, double* ws, long gs, int nvmax, int kmax, int pass,
-                             int all, const int* rlist)
+                             int njobs, long g0, double* ws, long gs, int nvmax, int pass,
+                             const int* rlist, const int* flist)
 {
-    const unsigned nwg = (unsigned)((nb + 63) / 64);
+    // four workgroups per CU, as many as fit; without listed points they end at once
+    const unsigned nwg = (unsigned)std::min(nb, 1024L);
     switch (kr) {
 #define LEKF_FIX_CASE(K)                                                                          \
     case K:                                                                                       \
         hipLaunchKernelGGL(lekf_eig_fix_kernel<K>, dim3(nwg), dim3(LEKF_WAVE), elds, st, djobs,   \
-                           njobs, g0, nb, ws, gs, nvmax, kmax, pass, all, rlist);                 \
+                           njobs, g0, nb, ws, gs, nvmax, pass, rlist, flist);                     \
         break;
         LEKF_FIX_CASE(36)
         LEKF_FIX_CASE(40)
@@ -3295,6 +3286,7 @@ static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int km
     short* ridx = (short*)(rot + (plan.streams ? (size_t)per * 2 * split_rcap(kmax) : 0));
     // then their columns, then the redo list
     int* rlist = (int*)(ridx + (plan.streams ? (size_t)per * split_ridx_stride(kmax) : 0));
+    int* flist = rlist + per + 1;  // and the flagged slots
     const int W = g_lekf_tune.gram_waves;
     const int kr = eig_kr(kmax);
     const size_t elds = eig_lds_doubles(kmax, nvmax) * sizeof(double);
@@ -3311,13 +3303,13 @@ static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int km
         hipError_t e = hipSuccess;
         if (plan.streams)
             e = launch_streams(kr, nb, elds, st, djobs, njobs, g0, (double*)ws, gs, nvmax, kmax,
-                               rot, ridx, pass, thr, rlist, per, plan.all);
+                               rot, ridx, pass, thr, rlist, per, flist, plan.all);
         if (e == hipSuccess && plan.plain)
             e = lekf_trf_launch(nb, st, djobs, njobs, g0, (double*)ws, gs, nvmax, kmax, pass,
-                                pass ? 0 : MODE, thr, rlist, per);
+                                pass ? 0 : MODE, thr, rlist, per, flist);
         if (e == hipSuccess && (plan.streams || plan.plain))
-            e = launch_fix(kr, nb, elds, st, djobs, njobs, g0, (double*)ws, gs, nvmax, kmax, pass,
-                           plan.streams, rlist);
+            e = launch_fix(kr, nb, elds, st, djobs, njobs, g0, (double*)ws, gs, nvmax, pass, rlist,
+                           flist);
         if (e == hipSuccess && plan.fused)
             e = launch_eig(plan.all ? kr : 0, nb, elds, st, djobs, njobs, g0, (double*)ws, gs,
                            nvmax, plan.all);
@@ -3326,7 +3318,7 @@ static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int km
     for (long g0 = 0; g0 < npt; g0 += per) {
         const long nb = per < npt - g0 ? per : npt - g0;
         hipError_t e = lekf_gram_launch(MODE, W, kmax, outs, nb, st, djobs, njobs, g0, (double*)ws,
-                                        gs, nullptr, g0 == 0 ? rlist : nullptr);
+                                        gs, nullptr, g0 == 0 ? rlist : nullptr, flist);
         if (e == hipSuccess) e = solve(g0, nb, 0, kthr);
         if (e != hipSuccess) return e;
     }
@@ -3334,7 +3326,7 @@ static hipError_t launch_split(const LekfJob* djobs, int njobs, long npt, int km
         // grids of one sub-batch; the slots past the list's length return at once
         const long nl = per < npt ? per : npt;
         hipError_t e = lekf_gram_launch(0, W, kmax, outs, nl, st, djobs, njobs, 0, (double*)ws, gs,
-                                        rlist, nullptr);
+                                        rlist, nullptr, flist);
         if (e == hipSuccess) e = solve(0, nl, 1, 0.0);
         if (e != hipSuccess) return e;
     }

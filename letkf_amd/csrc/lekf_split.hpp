@@ -34,8 +34,10 @@ __host__ __device__ inline long gram_stride(int kmax)
 constexpr int kSplitRedo = 16;
 
 // split-record flag: the point is left to lekf_eig_fix_kernel (its rotation stream
-// overflowed, or its condition number is past the rational form's tables)
+// overflowed, or its condition number is past the rational form's tables), which finds
+// its slot in flist (flist[0] entries from flist[1])
 constexpr int kSplitOverflow = 8;
+__device__ inline void split_flag_slot(int* flist, long slot) { flist[1 + atomicAdd(flist, 1)] = (int)slot; }
 
 // Flat point of slot `slot` of a split kernel: pass 0 the sub-batch's own
 // (gp0 + slot, nb slots), pass 1 the redo list's (rlist[0] entries from
@@ -81,4 +83,4 @@ __host__ __device__ inline long trf_stride(int kmax)
 // the plain solve of a sub-batch of nb slots (lekf_trf.hip)
 hipError_t lekf_trf_launch(long nb, hipStream_t st, const LekfJob* djobs, int njobs, long g0,
                            double* ws, long gs, int nvmax, int kmax, int pass, int mode,
-                           double kthr, int* rlist, long lcap);
+                           double kthr, int* rlist, long lcap, int* flist);

@@ -5,7 +5,7 @@
 // C + (k-1)/alpha I to its tridiagonal T and carries the state rows and b through
 // Q; lekf_trf_kernel evaluates the functions of T, carries the rows back and
 // writes the analysis.  A point whose bounds put its condition number past the
-// rational form's tables (or are not finite) is flagged and left to
+// rational form's tables (or are not finite) is flagged, listed and left to
 // lekf_eig_fix_kernel, whose Gram is still at the start of the record.
 //
 // Both are bound by VALU issue at two to four waves per SIMD (about 170 FP64
@@ -98,7 +98,8 @@ template <int NB, int NE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(trd_waves_per_simd(NB))))
 void lekf_trd_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
                      double* __restrict__ ws, long gstride, int nvmax, int kmax, int pass,
-                     int mode, double kthr, int* __restrict__ rlist, long lcap)
+                     int mode, double kthr, int* __restrict__ rlist, long lcap,
+                     int* __restrict__ flist)
 {
 #pragma clang fp contract(off)
     extern __shared__ double smem[];
@@ -210,6 +211,7 @@ void lekf_trd_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
         rec[S.sc] = m;
         rec[S.sc + 1] = (double)lev;
         rec[S.sc + 2] = tr;
+        if (hard && ((redo & kSplitRedo) != 0) == (pass != 0)) split_flag_slot(flist, blockIdx.x);
     }
     if (hard) return;
     for (int i = lane; i < k; i += 64) {
@@ -398,14 +400,14 @@ void lekf_trf_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
 template <int NB, int NE>
 static hipError_t launch_trf(long nb, hipStream_t st, const LekfJob* djobs, int njobs, long g0,
                              double* ws, long gs, int nvmax, int kmax, int pass, int mode,
-                             double kthr, int* rlist, long lcap)
+                             double kthr, int* rlist, long lcap, int* flist)
 {
     const size_t dlds = trd_lds_doubles(NB, nvmax, kmax) * sizeof(double);
     const size_t flds = trf_lds_doubles(NB, NE, kmax) * sizeof(double);
     {
         KTime kt(pass ? "redo_tri" : "eig_tri", st);
         hipLaunchKernelGGL((lekf_trd_kernel<NB, NE>), dim3((unsigned)nb), dim3(LEKF_WAVE), dlds, st,
-                           djobs, njobs, g0, ws, gs, nvmax, kmax, pass, mode, kthr, rlist, lcap);
+                           djobs, njobs, g0, ws, gs, nvmax, kmax, pass, mode, kthr, rlist, lcap, flist);
     }
     KTime kt(pass ? "redo_apply" : "eig_apply", st);
     hipLaunchKernelGGL((lekf_trf_kernel<NB, NE>), dim3((unsigned)nb), dim3(LEKF_WAVE), flds, st,
@@ -417,16 +419,16 @@ static hipError_t launch_trf(long nb, hipStream_t st, const LekfJob* djobs, int 
 
 hipError_t lekf_trf_launch(long nb, hipStream_t st, const LekfJob* djobs, int njobs, long g0,
                            double* ws, long gs, int nvmax, int kmax, int pass, int mode,
-                           double kthr, int* rlist, long lcap)
+                           double kthr, int* rlist, long lcap, int* flist)
 {
     const bool one = nvmax + 1 <= 8;
     switch (trf_slots(kmax)) {
 #define LEKF_TRF_CASE(NB)                                                                       \
     case NB:                                                                                    \
         return one ? launch_trf<NB, 1>(nb, st, djobs, njobs, g0, ws, gs, nvmax, kmax, pass,     \
-                                       mode, kthr, rlist, lcap)                                 \
+                                       mode, kthr, rlist, lcap, flist)                          \
                    : launch_trf<NB, 3>(nb, st, djobs, njobs, g0, ws, gs, nvmax, kmax, pass,     \
-                                       mode, kthr, rlist, lcap);
+                                       mode, kthr, rlist, lcap, flist);
         LEKF_TRF_CASE(5)
         LEKF_TRF_CASE(6)
         LEKF_TRF_CASE(7)

@@ -1,0 +1,117 @@
+"""Badly conditioned points of the solve without eigenvalues (32 < k <= 95, no trans, no
+pao): those past the rational form's tables are listed and solved by the fused eigen
+kernel, all at once, and agree with it in every precision.
+
+Timings compare batches within one process and only with wide margins: 256 listed points
+run on 256 CUs in about the time of one (one after another they took 64 times it).
+"""
+import time
+
+import numpy as np
+import pytest
+
+import oracle
+from letkf_amd import _lib, core, tune
+from letkf_amd.device import DeviceArray, sync
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(np.float64).eps
+
+
+@pytest.fixture
+def knobs():
+    before = tune.current()
+    yield
+    for name, v in before.items():
+        tune.set(name, v)
+
+
+def _problem(k, spreads, p, seed, nv=4):
+    rng = np.random.default_rng(seed)
+    npt = len(spreads)
+    n = npt * p
+    hd = rng.standard_normal((n, k)) * np.repeat(spreads, p)[:, None]
+    hd -= hd.mean(axis=1, keepdims=True)
+    return dict(k=k, npt=npt, nv=nv, hd=hd, rd=rng.uniform(0.5, 2.0, n), dep=rng.standard_normal(n),
+                rho=rng.uniform(0.1, 1.0, n), off=np.arange(npt + 1, dtype=np.int64) * p,
+                xb=rng.standard_normal((npt, nv, k)))
+
+
+def _job(q, prec="f64"):
+    t = DeviceArray.from_numpy
+    k, npt, nv = q["k"], q["npt"], q["nv"]
+    out = dict(xa=DeviceArray.zeros((npt, nv, k)), transm=DeviceArray.zeros((npt, k)),
+               status=DeviceArray.zeros((npt,), np.int32), infl=DeviceArray.zeros(npt))
+    kw = {"hdxf32": t(q["hd"].astype(np.float32))} if prec != "f64" else {}
+    job = core.make_job(k=k, npt=npt, hdxf=t(q["hd"]), rdiag=t(q["rd"]), dep=t(q["dep"]),
+                        loc_off=t(q["off"]), loc_idx=t(np.arange(q["hd"].shape[0], dtype=np.int32)),
+                        loc_rho=t(q["rho"]), infl_in=t(np.full(npt, 1.05)), infl_out=out["infl"],
+                        status=out["status"], transm=out["transm"],
+                        apply=dict(nij=npt, nv3d=nv, nv2d=0, x3b=t(q["xb"]), x3a=out["xa"]), **kw)
+    return job, out
+
+
+def _kappa(q, b):
+    sl = slice(q["off"][b], q["off"][b + 1])
+    c = (q["hd"][sl].T * (q["rho"][sl] / q["rd"][sl])) @ q["hd"][sl]
+    lam = np.linalg.eigvalsh(c + (q["k"] - 1) / 1.05 * np.eye(q["k"]))
+    return lam[-1] / lam[0]
+
+
+def _ms(job, prec="f64"):
+    ts = []
+    for i in range(6):
+        sync()
+        t0 = time.perf_counter()
+        core.letkf_core_batch([job], prec)
+        sync()
+        ts.append(time.perf_counter() - t0)
+    return 1e3 * min(ts[1:])
+
+
+@pytest.mark.parametrize("k", [40, 64, 80])
+def test_listed_points_run_side_by_side(gpu, k):
+    """Past the truncation threshold every point is listed: 256 of them against one."""
+    one, _ = _job(_problem(k, [1e5], 2 * k, 1))
+    many, out = _job(_problem(k, [1e5] * 256, 2 * k, 1))
+    t1, tn = _ms(one), _ms(many)
+    print(f"k={k}: 1 point {t1:.3f} ms, 256 points {tn:.3f} ms", flush=True)
+    assert (out["status"].numpy() & _lib.LEKF_PT_RANKDEF).all()
+    assert tn < 8 * t1
+
+
+@pytest.mark.parametrize("k", [36, 40, 57, 64])
+def test_mixed_forms_past_their_tables(gpu, knobs, k):
+    """FP32 and split-BF16x3 without the FP64 redo: condition numbers below and above the
+    mixed forms' last table (4 * 8^4), against the fused kernel on the same Gram.  Both are
+    backward stable: a small multiple of k eps cond(A)."""
+    _mixed(k)
+
+
+@pytest.mark.parametrize("k", [65, 72, 80, 95])
+def test_mixed_forms_past_their_tables_lds(gpu, knobs, k):
+    _mixed(k)
+
+
+def _mixed(k):
+    tune.set("mixed_kappa", 0)
+    q = _problem(k, [0.2, 1.0, 4.0, 12.0, 25.0, 40.0, 80.0], 2 * k, k)
+    kap = np.array([_kappa(q, b) for b in range(q["npt"])])
+    assert kap.min() < 32 and (kap < 16384).sum() >= 4 and (kap > 16384).sum() >= 1
+    for prec in ("f32", "bf16x3"):
+        res = []
+        for split in (1, 0):
+            tune.set("eig_split", split)
+            job, out = _job(q, prec)
+            core.letkf_core_batch([job], prec)
+            sync()
+            res.append({n: a.numpy() for n, a in out.items()})
+        a, f = res
+        np.testing.assert_array_equal(a["status"], f["status"])
+        for b in range(q["npt"]):
+            tol = 8 * k * EPS * kap[b]
+            for n in ("xa", "transm"):
+                d = np.abs(a[n][b] - f[n][b]).max()
+                assert d <= tol * np.abs(f[n][b]).max(), (prec, b, kap[b], n, d)
+            assert abs(a["infl"][b] - f["infl"][b]) <= 1e-12 * abs(f["infl"][b]), (prec, b)

@@ -8,15 +8,15 @@
 //   om_j = (2/pi) (K'/N) sc'(u_j),       u_j = (j - 1/2) K' / N.
 // Every term is positive, so the sum loses nothing to cancellation.  sc is taken
 // from its theta functions at an imaginary argument, whose nome is tiny here.
-// The tables hold N = 8, 12, .., 32 nodes for kappa = 4 * 8^i: the largest relative
-// error over [1, kappa] is below 4e-16 in each.  Evaluated at compile time.
+// The tables hold N = 8, 12, .., 40 nodes for kappa = 4 * 8^i, up to 2^26, where an
+// eigenvalue is small enough to be truncated: the largest relative error over [1, kappa]
+// is below 4e-16 in each.  Evaluated at compile time.
 #pragma once
 
 namespace lekf_invsqrt {
 
-constexpr int kLevels = 7;
+constexpr int kLevels = 9;
 constexpr int kMaxNodes = 8 + 4 * (kLevels - 1);
-constexpr double kKappaMax = 4.0 * 262144.0;  // 4 * 8^6
 
 struct Table {
     double sg[kLevels][kMaxNodes];
@@ -44,8 +44,9 @@ constexpr double c_exp(double x)
         t *= f / i;
         s += t;
     }
-    for (; n > 0; --n) s *= 2.0;
+    for (; n <= -32; n += 32) s *= 1.0 / 4294967296.0;
     for (; n < 0; ++n) s *= 0.5;
+    for (; n > 0; --n) s *= 2.0;
     return s;
 }
 

@@ -2203,7 +2203,7 @@ __device__ __forceinline__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec
 
 // The analysis' functions applied in T's basis, for both forms: L.B = Q^T b and the rows
 // of V = Q^T rows are replaced by f(T)'s, L.Cw by the rows' products with (T + g0)^-1 b.
-// The rational form where its tables reach the condition number (they do up to 4 8^6 in
+// The rational form where its tables reach the condition number (they do up to 2^26 in
 // FP64; 4 8^4 in the mixed forms, whose C is only positive semidefinite to 1e-6 of its
 // norm), else QL by wave 0 with its rotations kept in wsp.  shift = (k-1)/alpha bounds
 // the spectrum from below; gam > 0: the dual form (g0 = gam = shift).  Returns the status

@@ -390,7 +390,7 @@ void lekf_trf_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
                                 : adaptive_alpha(alpha, rec[(long)k * k + k],
                                                  rec[S.sc + 2] / (double)(k - 1),
                                                  rec[(long)k * k + k + 1]);
-        // the condition number is below the tables' 2^20, so no eigenvalue is truncated
+        // the condition number is below the tables' 2^26, so no eigenvalue is truncated
         if (J.status) J.status[b] = pass ? LEKF_PT_FP64 : 0;
     }
 }

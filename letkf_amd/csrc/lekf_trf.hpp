@@ -4,7 +4,7 @@
 // definite): A^-1 b and, for each state row x, x A^-1/2 and x A^-1 b.  With the
 // Householder form A = Q T Q^T they are (x Q) f(T) Q^T, and f(T) z is a sum of
 // tridiagonal solves, T^-1/2 z ~ sum_j om_j (T + sg_j I)^-1 z (lekf_invsqrt.hpp):
-// all terms positive, 16 to 24 of them for the condition numbers of local lists,
+// all terms positive, 16 to 24 of them for the condition numbers of most local lists,
 // to rounding.  Against tridiagonalisation + QL + rotation replay this drops Q
 // (4k^3/3 flops and 2 k^2 values out and in), the scalar QL recurrence (one lane
 // per point) and the rotation streams (46 KB written and read twice per point at

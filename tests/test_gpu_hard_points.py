@@ -81,6 +81,37 @@ def test_listed_points_run_side_by_side(gpu, k):
     assert tn < 8 * t1
 
 
+@pytest.mark.parametrize("k,nv", [(40, 5), (64, 9), (80, 3), (120, 2), (200, 6)])
+def test_tables_reach_the_truncation_threshold(gpu, k, nv):
+    """Condition numbers from 2^20 to the truncation threshold 2^26 (common_mtx.f90:66-74):
+    the rational form's, without eigenvalues, as fast as well conditioned points, against
+    oracle.letkf_core.  Both sides are backward stable: a small multiple of k eps cond(A)."""
+    q = _problem(k, [700.0, 1500.0, 2500.0, 3000.0], 2 * k, k, nv)
+    job, out = _job(q)
+    core.letkf_core_batch([job])
+    sync()
+    a = {n: x.numpy() for n, x in out.items()}
+    kaps = []
+    for b in range(q["npt"]):
+        sl = slice(q["off"][b], q["off"][b + 1])
+        ref = oracle.letkf_core(q["hd"][sl], q["rd"][sl], q["rho"][sl], q["dep"][sl], 1.05,
+                                transm=True)
+        kap = _kappa(q, b)
+        kaps.append(kap)
+        tol = 8 * k * EPS * kap
+        xm = q["xb"][b].mean(axis=1, keepdims=True)
+        want = xm + (q["xb"][b] - xm) @ (ref["trans"] + ref["transm"][:, None])
+        assert a["status"][b] == 0
+        assert np.abs(a["xa"][b] - want).max() <= tol * np.abs(want - xm).max() + 1e-13
+        assert np.abs(a["transm"][b] - ref["transm"]).max() <= tol * np.abs(ref["transm"]).max()
+    assert 2 ** 20 < min(kaps) and max(kaps) < 2 ** 26, kaps
+    hard, easy = (_job(_problem(k, [s] * 256, 2 * k, 3, nv))[0] for s in (1500.0, 0.5))
+    th, te = _ms(hard), _ms(easy)
+    print(f"k={k}: condition {min(kaps):.2g} .. {max(kaps):.2g}, {th:.3f} ms, {te:.3f} ms well conditioned",
+          flush=True)
+    assert th < 3 * te
+
+
 @pytest.mark.parametrize("k", [36, 40, 57, 64])
 def test_mixed_forms_past_their_tables(gpu, knobs, k):
     """FP32 and split-BF16x3 without the FP64 redo: condition numbers below and above the

@@ -1502,6 +1502,14 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// The order of one wave's LDS accesses alone (the hardware runs them in order; global
+// stores are not waited for)
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // a[u] summed over the wave for all u at once: lane l gets the sum of u = l % 8
 __device__ __forceinline__ double wave_sum8(const double (&a)[8], int lane)
 {
@@ -2082,23 +2090,32 @@ __device__ __forceinline__ int big_level(const EigLds& L, int n, double g0, doub
     return trf_level(hi, m);
 }
 
-// eig_ql on (d, e) without eigenvectors: each sweep's rotations are applied
-// to the nvec vectors (lane q owns vector q; the same update as a row of Z,
-// so u = Z^T y is maintained) and appended to rbuf.  Returns nonzero if an
-// eigenvalue needed more than kQlMaxIter sweeps; ovf is set if rbuf filled.
-__device__ __forceinline__ int eig_ql_vec(EigLds& L, int n, int lane, const VecSet& V, int nvec, double* rbuf,
-                          long rcap, long& rpos, bool& ovf)
+// eig_ql on (d, e) without eigenvectors: each rotation is applied to the nvec vectors as
+// it is formed (lane q owns vector q; the same update as a row of Z, so u = Z^T y is
+// maintained, in the shadow of the recurrence) and appended to rbuf.  Returns nonzero if
+// an eigenvalue needed more than kQlMaxIter sweeps; ovf is set if rbuf filled.
+__device__ __forceinline__ int eig_ql_vec(EigLds& L, int n, int lane, const VecSet& V, int nvec,
+                                          double* rbuf, long rcap, long& rpos, bool& ovf)
 {
     double* d = L.d;
     double* e = L.e;
+    double* z = V.at(lane < nvec ? lane : 0);
     double tst = 0.0;
     for (int l = 0; l < n; ++l) {
         tst = fmax(tst, fabs(d[l]) + fabs(e[l]));
         int iter = 0;
         for (;;) {
+            // the first negligible sub-diagonal element, 64 looked at at once
             int m = l;
-            for (; m < n - 1; ++m)
-                if (tst + fabs(e[m]) == tst) break;
+            for (;; m += 64) {
+                const int t = m + lane;
+                const unsigned long long small =
+                    __ballot(t >= n - 1 || tst + fabs(e[t]) == tst);
+                if (small) {
+                    m += __builtin_ctzll(small);
+                    break;
+                }
+            }
             if (m == l) break;
             if (iter++ == kQlMaxIter) return 1;
             const double dl = d[l], el = e[l];
@@ -2108,37 +2125,43 @@ __device__ __forceinline__ int eig_ql_vec(EigLds& L, int n, int lane, const VecS
             double s = 1.0, c = 1.0, p = 0.0;
             int i = m - 1;
             bool split = false;
-            double ei = e[i], di1 = d[i + 1];
+            double ei = e[i], di1 = d[i + 1], z1 = z[m], z0 = z[i];
             for (; i >= l; --i) {
-                const double di = d[i];
-                const double eprev = i > l ? e[i - 1] : 0.0;
+                // the next step's e and z, loaded before this one's stores
+                const int in = i > l ? i - 1 : l;
+                const double di = d[i], en = e[in], zn = z[in];
                 const double f = s * ei, bb = c * ei;
-                r = sqrt(fma(f, f, g * g));
-                e[i + 1] = r;
-                if (r == 0.0) {
+                const double x = fma(f, f, g * g);
+                if (x == 0.0) {
+                    e[i + 1] = 0.0;
                     d[i + 1] = di1 - p;
                     e[m] = 0.0;
                     split = true;
                     break;
                 }
-                const double ri = rcp_nr(r);
-                s = f * ri;
-                c = g * ri;
+                const double y = rsq_nr(x);
+                e[i + 1] = x * y;  // hypot(f, g)
+                s = f * y;
+                c = g * y;
                 g = di1 - p;
                 r = fma(di - g, s, 2.0 * c * bb);
                 p = s * r;
                 d[i + 1] = g + p;
                 g = fma(c, r, -bb);
+                if (lane < nvec) z[i + 1] = fma(s, z0, c * z1);
+                z1 = fma(c, z0, -s * z1);
                 if (lane == 0) {
                     L.rot[2 * i] = c;
                     L.rot[2 * i + 1] = s;
                 }
-                ei = eprev;
+                ei = en;
                 di1 = di;
+                z0 = zn;
             }
-            wave_sync();
             const int ilo = split ? i + 1 : l;
             const int cnt = m - ilo;
+            if (lane < nvec) z[ilo] = z1;
+            wave_order();
             if (!ovf && rpos + 2L * cnt + 2 <= rcap) {
                 for (int q = lane; q < 2 * cnt; q += 64)
                     rbuf[rpos + q] = L.rot[2 * (m - 1 - (q >> 1)) + (q & 1)];
@@ -2150,53 +2173,62 @@ __device__ __forceinline__ int eig_ql_vec(EigLds& L, int n, int lane, const VecS
             } else {
                 ovf = true;
             }
-            if (lane < nvec) {
-                double* z = V.at(lane);
-                double z1 = z[m];
-                for (int ii = m - 1; ii >= ilo; --ii) {
-                    const double cc = L.rot[2 * ii], ss = L.rot[2 * ii + 1];
-                    const double z0 = z[ii];
-                    z[ii + 1] = fma(ss, z0, cc * z1);
-                    z1 = fma(cc, z0, -ss * z1);
-                }
-                z[ilo] = z1;
-            }
             if (!split) {
                 d[l] = d[l] - p;
                 e[l] = g;
                 e[m] = 0.0;
             }
-            wave_sync();
+            wave_order();
         }
     }
     return 0;
 }
 
+// Rotations whose (c, s) and vector elements are loaded at once: the vector's stores would
+// otherwise hold back the next step's loads.
+constexpr int kRotBatch = 8;
+
 // y <- S y: the recorded sweeps in reverse order, each sweep's rotations in
 // increasing index (the inverse of the forward update)
-__device__ __forceinline__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec, const double* rbuf, long rpos,
-                            int lane)
+__device__ __forceinline__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec,
+                                            const double* rbuf, long rpos, int lane)
 {
+    if (rpos <= 0) return;
+    double* z = V.at(lane < nvec ? lane : 0);
     long pos = rpos;
+    double hilo = rbuf[pos - 2], hm = rbuf[pos - 1];
     while (pos > 0) {
-        const int ilo = (int)rbuf[pos - 2], m = (int)rbuf[pos - 1];
+        const int ilo = (int)hilo, m = (int)hm;
         const int cnt = m - ilo;
         const long base = pos - 2 - 2L * cnt;
+        if (base > 0) {  // the next sweep's trailer, while this one is applied
+            hilo = rbuf[base - 2];
+            hm = rbuf[base - 1];
+        }
         for (int q = lane; q < 2 * cnt; q += 64)
             L.rot[2 * (m - 1 - (q >> 1)) + (q & 1)] = rbuf[base + q];
-        wave_sync();
+        wave_order();
         if (lane < nvec) {
-            double* z = V.at(lane);
             double zl = z[ilo];
-            for (int ii = ilo; ii < m; ++ii) {
-                const double cc = L.rot[2 * ii], ss = L.rot[2 * ii + 1];
-                const double zi1 = z[ii + 1];
-                z[ii] = fma(cc, zl, ss * zi1);
-                zl = fma(-ss, zl, cc * zi1);
+            for (int i0 = ilo; i0 < m; i0 += kRotBatch) {
+                double cc[kRotBatch], ss[kRotBatch], z1[kRotBatch];
+#pragma unroll
+                for (int u = 0; u < kRotBatch; ++u) {
+                    const int ii = i0 + u < m ? i0 + u : m - 1;
+                    cc[u] = L.rot[2 * ii];
+                    ss[u] = L.rot[2 * ii + 1];
+                    z1[u] = z[ii + 1];
+                }
+#pragma unroll
+                for (int u = 0; u < kRotBatch; ++u)
+                    if (i0 + u < m) {
+                        z[i0 + u] = fma(cc[u], zl, ss[u] * z1[u]);
+                        zl = fma(-ss[u], zl, cc[u] * z1[u]);
+                    }
             }
             z[m] = zl;
         }
-        wave_sync();
+        wave_order();
         pos = base;
     }
 }
@@ -2205,9 +2237,10 @@ __device__ __forceinline__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec
 // of V = Q^T rows are replaced by f(T)'s, L.Cw by the rows' products with (T + g0)^-1 b.
 // The rational form where its tables reach the condition number (they do up to 2^26 in
 // FP64; 4 8^4 in the mixed forms, whose C is only positive semidefinite to 1e-6 of its
-// norm), else QL by wave 0 with its rotations kept in wsp.  shift = (k-1)/alpha bounds
-// the spectrum from below; gam > 0: the dual form (g0 = gam = shift).  Returns the status
-// bits.
+// norm), else QL by wave 0 with its rotations kept in wsp (2000 points, k = 200 / 256: 69 /
+// 106 ms against 18 / 27 with the tables; one wave per point took 69 / 163).  shift =
+// (k-1)/alpha bounds the spectrum from below; gam > 0: the dual form (g0 = gam = shift).
+// Returns the status bits.
 template <int MODE>
 __device__ __forceinline__ int big_spectral(EigLds& L, int n, int k, double shift, double gam, const VecSet& V,
                             double* wsp, long wcap, int tid)

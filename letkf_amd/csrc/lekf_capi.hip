@@ -939,6 +939,7 @@ RegionalArgs make_reg_args(const lekf_handle* h)
     R.nlev = h->nlev;
     R.nbkt = h->nbkt;
     R.nobs_max = h->r.nobs_max;
+    R.nbinned = h->nbinned;
     R.dx = h->r.dx;
     R.dy = h->r.dy;
     R.sigma_h = h->r.sigma_h;

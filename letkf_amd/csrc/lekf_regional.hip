@@ -32,6 +32,7 @@
 // union, and a candidate evicted within its own block passes its slot on
 // (pointer jumping).
 #include <algorithm>
+#include <cmath>
 
 #include "lekf_dev.hpp"
 #include "lekf_regional.hpp"
@@ -938,6 +939,177 @@ __device__ __forceinline__ unsigned long long wc_block(WaveCap& L, int* so, cons
     return L.key[cap - 1];
 }
 
+// The same block of at most 64 candidates, one per lane, for small caps and short streams,
+// where the counts over LEKF_CAP_LDS places and the scans over them would cost more than
+// the candidates: they are sorted across the lanes by (key, lane), and the entries of S move
+// up 64 at a time, one entrant after the other counted.
+__device__ __forceinline__ void wc_sort64(unsigned long long& k, int& id, int lane)
+{
+#pragma unroll
+    for (int sz = 2; sz <= 64; sz <<= 1) {
+#pragma unroll
+        for (int j = sz >> 1; j > 0; j >>= 1) {
+            const unsigned lo = (unsigned)lane_xor((int)(unsigned)k, j, lane);
+            const unsigned hi = (unsigned)lane_xor((int)(unsigned)(k >> 32), j, lane);
+            const unsigned long long ok = ((unsigned long long)hi << 32) | lo;
+            const int oid = lane_xor(id, j, lane);
+            const bool up = (lane & sz) == 0;
+            const bool lower = (lane & j) == 0;
+            const bool oless = ok < k || (ok == k && oid < id);
+            if (lower == up ? oless : !oless) {
+                k = ok;
+                id = oid;
+            }
+        }
+    }
+}
+
+// Entries 0 .. n-1 of S move up by the entrants placed before them (lanes with ent, at
+// count c1 of the old entries, ascending: before entry i iff c1 <= i); an entry that lands
+// at lim or above goes to ev (its slot).  Windows of 64 go top down, so a window's writes
+// only reach entries that have moved.
+__device__ __forceinline__ void wc_shift64(WaveCap& L, int* ev, int n, int lim, bool ent, int c1,
+                                           int lane)
+{
+    const unsigned long long em = __ballot(ent);
+    if (!em || n <= 0) return;
+    const int c1min = __builtin_amdgcn_readlane(c1, __builtin_ctzll(em));
+    for (int lo = ((n - 1) >> 6) << 6; lo >= 0 && lo + 64 > c1min; lo -= 64) {
+        const int i = lo + lane;
+        unsigned long long k = 0;
+        int s = 0;
+        if (i < n) {
+            k = L.key[i];
+            s = L.slot[i];
+        }
+        int up = __popcll(__ballot(ent && c1 < lo));
+        for (unsigned long long w = __ballot(ent && c1 >= lo && c1 < lo + 64); w; w &= w - 1)
+            up += lane >= __builtin_amdgcn_readlane(c1, __builtin_ctzll(w)) - lo ? 1 : 0;
+        if (i < n && up > 0) {
+            if (i + up < lim) {
+                L.key[i + up] = k;
+                L.slot[i + up] = (unsigned short)s;
+            } else {
+                ev[i + up - lim] = s;
+            }
+        }
+    }
+}
+
+template <class Eval>
+__device__ __forceinline__ unsigned long long wc_block64(WaveCap& L, int* so, const int* src,
+                                                         int np, int fill, int cap, int lane,
+                                                         unsigned long long tau, Eval eval)
+{
+    const bool full = fill < 0;
+    const int n = full ? cap : fill;         // entries of S
+    const int lim = full ? cap : fill + np;  // and after the block
+    int* ev = (int*)L.cnt;  // entries that left, ascending: slot, or -(entrant + 1)
+    int* slotn = ev + 64;
+    int* link = ev + 128;
+    const int p = lane < np ? src[lane] : -1;
+    wave_sync();
+    bool ok = false;
+    unsigned long long y = ~0ull;
+    if (p >= 0) y = eval(p, ok);
+    const bool live = p >= 0 && (full ? ok && y < tau : true);
+    const int nlive = __popcll(__ballot(live));
+    if (nlive == 0) return tau;
+    // sorted by (key, lane), the live candidates first
+    unsigned long long sk = live ? y : ~0ull;
+    int sid = live ? lane : lane + 64;
+    wc_sort64(sk, sid, lane);
+    sid &= 63;
+    const bool slive = lane < nlive;
+    const int ps = __shfl(p, sid, 64);
+    int c1 = 0;  // entries of S before it
+    {
+        int lo = 0, hi = slive ? n : 0;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (L.key[mid] <= sk)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        c1 = lo;
+    }
+    wave_sync();
+    if (!full) {
+        wc_shift64(L, ev, n, lim, slive, c1, lane);
+        wave_sync();
+        if (slive) {
+            L.key[c1 + lane] = sk;
+            L.slot[c1 + lane] = (unsigned short)(fill + sid);
+            so[fill + sid] = ps;
+        }
+        wave_sync();
+        return L.key[lim - 1];
+    }
+    // earlier (in scan order) live candidates sorted before this one
+    const unsigned long long own = slive ? 1ull << sid : 0ull;
+    unsigned long long pm = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned long long o = __shfl_up(pm, d, 64);
+        if (lane >= d) pm |= o;
+    }
+    const int c2 = __popcll(pm & ~own & lane_lt(sid));
+    const bool ent = slive && c1 + c2 < cap;
+    const unsigned long long em = __ballot(ent);
+    const int e = __popcll(em);
+    if (e == 0) return tau;
+    const int at = c1 + __popcll(em & lane_lt(lane));  // position in S and the entrants
+    // scan-order index of each entrant: its flag back to the candidate's lane
+    const unsigned long long eo =
+        __ballot(__builtin_amdgcn_ds_permute(sid << 2, ent ? 1 : 0) != 0);
+    const int t = __popcll(eo & lane_lt(sid));
+    wc_shift64(L, ev, cap, cap, ent, c1, lane);
+    wave_sync();
+    if (ent) {
+        if (at < cap)
+            L.key[at] = sk;
+        else
+            ev[at - cap] = -(t + 1);
+    }
+    wave_sync();
+    int sl = -1, ln = -1;
+    if (ent) {
+        const int v = ev[e - 1 - t];
+        if (v >= 0)
+            sl = v;
+        else
+            ln = -v - 1;
+        slotn[t] = sl;
+        link[t] = ln;
+    }
+    wave_sync();
+    // chains of at most 64 entrants: 6 doublings
+    for (int round = 0; round < 6 && __ballot(ent && sl < 0); ++round) {
+        int s2 = -1, l2 = -1;
+        if (ent && sl < 0) {
+            s2 = slotn[ln];
+            l2 = link[ln];
+        }
+        wave_sync();
+        if (ent && sl < 0) {
+            if (s2 >= 0)
+                sl = s2;
+            else
+                ln = l2;
+            slotn[t] = sl;
+            link[t] = ln;
+        }
+        wave_sync();
+    }
+    if (ent && at < cap && sl >= 0) {
+        L.slot[at] = (unsigned short)sl;
+        so[sl] = ps;
+    }
+    wave_sync();
+    return L.key[cap - 1];
+}
+
 // A chunk of the stream: lane l's candidate p enters the fill or the queue iff in
 // (while S fills every stream candidate; then at least those with a key below tau).
 __device__ __forceinline__ void wc_push(WaveCap& L, WcState& S, bool in, int p, int cap, int lane)
@@ -958,26 +1130,31 @@ __device__ __forceinline__ void wc_push(WaveCap& L, WcState& S, bool in, int p, 
     wave_sync();
 }
 
-// Blocks that are due: the fill's once S has cap entries, the queue's when kWcB
-// candidates wait, or any with last.
-template <class Eval>
+// Blocks that are due: the fill's once S has cap entries, the queue's when a block's
+// candidates wait (kWcB, SMALL: 64), or any with last.
+template <bool SMALL, class Eval>
 __device__ __forceinline__ void wc_service(WaveCap& L, int* so, WcState& S, int cap, int lane,
                                            bool last, Eval eval)
 {
+    constexpr int B = SMALL ? 64 : kWcB;
     while (S.n >= cap) {
         const bool filling = S.m < cap;
-        if (!filling && S.q < kWcB && !(last && S.q > 0)) break;
+        if (!filling && S.q < B && !(last && S.q > 0)) break;
         const int have = filling ? cap - S.m : S.q;
-        const int np = have < kWcB ? have : kWcB;
-        S.tau = wc_block(L, so, filling ? wc_fill_pos(L) + S.m : L.qp, np, filling ? S.m : -1, cap,
-                         lane, S.tau, eval);
+        const int np = have < B ? have : B;
+        const int* src = filling ? wc_fill_pos(L) + S.m : L.qp;
+        const int fill = filling ? S.m : -1;
+        if constexpr (SMALL)
+            S.tau = wc_block64(L, so, src, np, fill, cap, lane, S.tau, eval);
+        else
+            S.tau = wc_block(L, so, src, np, fill, cap, lane, S.tau, eval);
         if (filling) {
             S.m += np;
         } else {
             // the rest of the queue (fewer than 64) moves to its front
             S.q -= np;
             int o = 0;
-            if (lane < S.q) o = L.qp[kWcB + lane];
+            if (lane < S.q) o = L.qp[B + lane];
             wave_sync();
             if (lane < S.q) L.qp[lane] = o;
             wave_sync();
@@ -1140,7 +1317,12 @@ __global__ __launch_bounds__(kSelT) void reg_select(RegionalArgs A, long npt)
 // bucket by bucket in slot order, rho recomputed from the kept obs.
 constexpr int kTileX = 16, kTileY = 8;  // columns of a selection tile
 
-template <int NW>
+//
+// Forms.  kDense: each row's candidates in chunks of their own.  kFewRows: rows of a few
+// candidates, several in a chunk.  kSmallCap: the same, and blocks of 64.
+constexpr int kDense = 0, kFewRows = 1, kSmallCap = 2;
+
+template <int NW, int FORM>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3)))
 void reg_select_wave(RegionalArgs A, long npt)
 {
@@ -1244,67 +1426,92 @@ void reg_select_wave(RegionalArgs A, long npt)
                 }
             }
             // the rows that hold candidates, 64 of one row at a time; the next chunk's
-            // loads are on their way while one is tested
-            unsigned long long rows = __ballot(len > 0);
-            int r = 0, rbeg = 0, rlen = 0, at = 0, np = -1;
-            float4 nrec = make_float4(0.f, 0.f, 0.f, 0.f);
-            auto row = [&]() {
-                r = __builtin_ctzll(rows);
-                rbeg = __builtin_amdgcn_readlane(beg, r);
-                rlen = __builtin_amdgcn_readlane(len, r);
-                at = 0;
-            };
-            auto fetch = [&]() {
-                np = at + lane < rlen ? rbeg + at + lane : -1;
-                if (np >= 0) nrec = A.brf[np];
-            };
-            if (rows) {
-                row();
-                fetch();
+            // loads are on their way while one is tested.  Where that would leave the chunks
+            // less than half full (not kDense), all rows as one sequence, 64 of it at a time,
+            // each lane looking up its candidate's row among the sums of the lengths.
+            int ntot = 0;
+            bool packed = false;
+            if constexpr (FORM != kDense) {
+                ntot = __builtin_amdgcn_readlane(wave_scan(len), 63);
+                const int nch = __builtin_amdgcn_readlane(wave_scan((len + 63) >> 6), 63);
+                packed = 2 * ((ntot + 63) >> 6) <= nch;
             }
-            do {
-                if (rows) {
-                    if (at == 0 && S.m >= cap && (double)(j0 + r) - rj > 0.5) {
-                        // rows from this one on lie beyond the point: an obs of
-                        // row j has |rj_o - rj| > j - rj - 0.5, so
-                        // nd > ((j - rj - 0.5) dy / sigma_h)^2 and its key
-                        // err^2 / rho exceeds err2_min exp(nd / 2); once that
-                        // bound (less a 1e-9 margin for rounding) reaches tau,
-                        // which only falls, no later candidate can enter
-                        const double g = ((double)(j0 + r) - rj - 0.5) * A.dy / A.sigma_h;
-                        const double lb = e2min * exp(0.5 * g * g) * (1.0 - 1e-9);
-                        if (lb >= __longlong_as_double((long long)S.tau)) {
-                            fin = true;
-                            rows = 0;
+            for (int q0 = 0;; q0 += 64) {
+                unsigned long long rows = __ballot(len > 0);
+                int r = 0, rbeg = 0, rlen = 0, at = 0, np = -1;
+                float4 nrec = make_float4(0.f, 0.f, 0.f, 0.f);
+                auto row = [&]() {
+                    r = __builtin_ctzll(rows);
+                    rbeg = __builtin_amdgcn_readlane(beg, r);
+                    rlen = __builtin_amdgcn_readlane(len, r);
+                    at = 0;
+                };
+                auto fetch = [&]() {
+                    np = at + lane < rlen ? rbeg + at + lane : -1;
+                    if (np >= 0) nrec = A.brf[np];
+                };
+                if (FORM != kDense && packed && rows) {
+                    const int pre = wave_scan(len), q = q0 + lane;
+                    int k = 0;  // rows whose candidates all come before q
+#pragma unroll
+                    for (int d = 32; d > 0; d >>= 1)
+                        if (__shfl(pre, k + d - 1, 64) <= q) k += d;
+                    const int p0 = __shfl(beg - (pre - len), k, 64);
+                    np = q < ntot ? p0 + q : -1;
+                    if (np >= 0) nrec = A.brf[np];
+                    r = __builtin_amdgcn_readfirstlane(k);
+                    rows = 1;  // one chunk
+                } else if (rows) {
+                    row();
+                    fetch();
+                }
+                do {
+                    if (rows) {
+                        if (at == 0 && S.m >= cap && (double)(j0 + r) - rj > 0.5) {
+                            // rows from this one on lie beyond the point: an obs of
+                            // row j has |rj_o - rj| > j - rj - 0.5, so
+                            // nd > ((j - rj - 0.5) dy / sigma_h)^2 and its key
+                            // err^2 / rho exceeds err2_min exp(nd / 2); once that
+                            // bound (less a 1e-9 margin for rounding) reaches tau,
+                            // which only falls, no later candidate can enter
+                            const double g = ((double)(j0 + r) - rj - 0.5) * A.dy / A.sigma_h;
+                            const double lb = e2min * exp(0.5 * g * g) * (1.0 - 1e-9);
+                            if (lb >= __longlong_as_double((long long)S.tau)) {
+                                fin = true;
+                                rows = 0;
+                            }
                         }
                     }
-                }
-                if (rows) {
-                    const float4 cur = nrec;
-                    const int p = np;
-                    at += 64;
-                    if (at >= rlen) {
-                        rows &= rows - 1;
-                        if (rows) row();
+                    if (rows) {
+                        const float4 cur = nrec;
+                        const int p = np;
+                        at += 64;
+                        if (at >= rlen) {
+                            rows &= rows - 1;
+                            if (rows) row();
+                        }
+                        if (rows) fetch();
+                        const float fx = fri - cur.x, fy = frj - cur.y, fz = cur.z - frz;
+                        const float nd = __builtin_fmaf(fx * fx, cx,
+                                                        __builtin_fmaf(fy * fy, cy, fz * fz * cv));
+                        bool in = p >= 0 && !(nd > nd_out);
+                        if (S.n < cap) {
+                            if (in && !(nd < nd_in))
+                                in = eval_rec(A, load_rec(p), p, ri, rj, rz).ok;
+                        } else if (S.m >= cap) {
+                            in = in && !(__builtin_fmaf(0.72134752f, nd, cur.w) > l2tau);
+                        }
+                        wc_push(W, S, in, p, cap, lane);
                     }
-                    if (rows) fetch();
-                    const float fx = fri - cur.x, fy = frj - cur.y, fz = cur.z - frz;
-                    const float nd = __builtin_fmaf(fx * fx, cx,
-                                                    __builtin_fmaf(fy * fy, cy, fz * fz * cv));
-                    bool in = p >= 0 && !(nd > nd_out);
-                    if (S.n < cap) {
-                        if (in && !(nd < nd_in)) in = eval_rec(A, load_rec(p), p, ri, rj, rz).ok;
-                    } else if (S.m >= cap) {
-                        in = in && !(__builtin_fmaf(0.72134752f, nd, cur.w) > l2tau);
-                    }
-                    wc_push(W, S, in, p, cap, lane);
-                }
-                const unsigned long long tau0 = S.tau;
-                wc_service(W, so, S, cap, lane, fin, eval);
-                if (S.tau != tau0)
-                    // 0.73 em for nd's error, 1e-3 for the logarithms'
-                    l2tau = (float)log2(__longlong_as_double((long long)S.tau)) + 0.73f * em + 1.0e-3f;
-            } while (rows);
+                    const unsigned long long tau0 = S.tau;
+                    wc_service<FORM == kSmallCap>(W, so, S, cap, lane, fin, eval);
+                    if (S.tau != tau0)
+                        // 0.73 em for nd's error, 1e-3 for the logarithms'
+                        l2tau = (float)log2(__longlong_as_double((long long)S.tau)) + 0.73f * em +
+                                1.0e-3f;
+                } while (rows);
+                if (FORM == kDense || !packed || fin || q0 + 64 >= ntot) break;
+            }
             if (fin) break;
         }
         const int kept = S.n < cap ? S.n : cap;
@@ -1396,6 +1603,7 @@ __device__ __forceinline__ unsigned long long rho_key(double rho)
     return 0x7fffffffffffffffull - (unsigned long long)__double_as_longlong(rho);
 }
 
+template <bool SMALL>
 __global__ __launch_bounds__(64) void list_cap_wave(ListCapArgs A)
 {
     __shared__ WaveCap L;
@@ -1423,7 +1631,7 @@ __global__ __launch_bounds__(64) void list_cap_wave(ListCapArgs A)
                 const int i = i0 + lane;
                 rn = i + 64 < n ? ir[i + 64] : 0.0;
                 wc_push(L, S, i < n && rho_key(rc) < S.tau, i, A.cap, lane);
-                wc_service(L, so, S, A.cap, lane, i0 + 64 >= n, [&](int p, bool& ok) {
+                wc_service<SMALL>(L, so, S, A.cap, lane, i0 + 64 >= n, [&](int p, bool& ok) {
                     ok = true;
                     return rho_key(ir[p]);
                 });
@@ -1653,6 +1861,11 @@ long lekf_reg_wave_slots_max()
 // one to end, which nearly doubles the launch)
 static constexpr int lds_fit(size_t lds) { return (int)(128 / ((lds + 1279) / 1280)); }
 
+// Largest cap merged in blocks of 64.  96 x 48 x 7 points, 4000 stations, list_cap_wave at
+// caps 10 / 40 / 64 / 100: 1.08 / 1.41 / 1.62 / 1.91 ms so, 1.34 / 1.53 / 1.63 / 1.75 in
+// blocks of 224.
+constexpr int kSmallCapMax = 64;
+
 hipError_t lekf_list_cap_launch(const ListCapArgs& A, int nslots, hipStream_t st)
 {
     const long npt = (long)A.ncols * A.nlev;
@@ -1663,11 +1876,12 @@ hipError_t lekf_list_cap_launch(const ListCapArgs& A, int nslots, hipStream_t st
         int dev = 0, ncu = 256, per_cu = 1;
         if (hipGetDevice(&dev) == hipSuccess)
             (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, list_cap_wave, 64, 0);
+        const auto fn = A.cap <= kSmallCapMax ? list_cap_wave<true> : list_cap_wave<false>;
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64, 0);
         per_cu = std::min(per_cu, lds_fit(sizeof(WaveCap) + sizeof(int) * LEKF_CAP_LDS));
         long g = (long)(per_cu > 0 ? per_cu : 1) * (ncu > 0 ? ncu : 256);
         if (g > npt) g = npt;
-        hipLaunchKernelGGL(list_cap_wave, dim3((unsigned)g), dim3(64), 0, st, A);
+        hipLaunchKernelGGL(fn, dim3((unsigned)g), dim3(64), 0, st, A);
         return hipGetLastError();
     }
     const long g = npt < nslots ? npt : nslots;
@@ -1675,21 +1889,41 @@ hipError_t lekf_list_cap_launch(const ListCapArgs& A, int nslots, hipStream_t st
     return hipGetLastError();
 }
 
-template <int NW>
+template <int NW, int FORM>
 static hipError_t launch_select_wave(const RegionalArgs& A, long npt, hipStream_t st)
 {
     // as many workgroups as the LDS lets the CUs hold
     int dev = 0, ncu = 256, per_cu = 1;
     if (hipGetDevice(&dev) == hipSuccess)
         (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reg_select_wave<NW>, 64 * NW, 0);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (reg_select_wave<NW, FORM>), 64 * NW,
+                                                       0);
     per_cu = std::min(per_cu, lds_fit(NW * sizeof(WaveCap)));
     long g = (long)(per_cu > 0 ? per_cu : 1) * (ncu > 0 ? ncu : 256);
     if (g * NW > A.wc_so_waves) g = A.wc_so_waves / NW;  // one slot map per wave
     if (g > npt) g = npt;
     if (g < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(reg_select_wave<NW>, dim3((unsigned)g), dim3(64 * NW), 0, st, A, npt);
+    hipLaunchKernelGGL((reg_select_wave<NW, FORM>), dim3((unsigned)g), dim3(64 * NW), 0, st, A,
+                       npt);
     return hipGetLastError();
+}
+
+// Rows of fewer candidates than this, on average over the grid and per bucket, share chunks
+constexpr double kFewRow = 32.0;
+
+// Which form of reg_select_wave: 64 x 64 x 10 points, two buckets, ms with kSmallCap /
+// kFewRows / kDense at cap 10: 0.42 / 0.57 / 1.16 (3 candidates a row), 0.79 / 0.92 / 1.33 (15),
+// 1.93 / 2.36 / 2.37 (150); at cap 100: 0.18 / 0.20 / 0.59, 1.05 / 0.97 / 1.40, 3.31 / 3.08 /
+// 3.09; at cap 500: 0.18 / 0.20 / 0.59, 0.40 / 0.45 / 0.72, 6.60 / 4.73 / 4.67.  At 30
+// candidates a row, cap 500, kFewRows 1.63 and kDense 1.79; at 60 they are alike.
+template <int NW>
+static hipError_t launch_select_form(const RegionalArgs& A, long npt, hipStream_t st)
+{
+    if (A.nobs_max <= kSmallCapMax) return launch_select_wave<NW, kSmallCap>(A, npt, st);
+    const double row = (2.0 * std::sqrt(kNdMax) * A.sigma_h / A.dx + 1.0) * A.nbinned /
+                       ((double)A.nbkt * A.nx * A.ny);
+    return row < kFewRow ? launch_select_wave<NW, kFewRows>(A, npt, st)
+                         : launch_select_wave<NW, kDense>(A, npt, st);
 }
 
 hipError_t lekf_reg_select_launch(const RegionalArgs& A, long npt, int nslots, hipStream_t st)
@@ -1698,10 +1932,10 @@ hipError_t lekf_reg_select_launch(const RegionalArgs& A, long npt, int nslots, h
     KTime kt("select", st);
     if (lekf_reg_select_fused(A.nobs_max) && A.bcc) {
         switch (A.nbkt) {
-        case 1: return launch_select_wave<1>(A, npt, st);
-        case 2: return launch_select_wave<2>(A, npt, st);
-        case 3: return launch_select_wave<3>(A, npt, st);
-        case 4: return launch_select_wave<4>(A, npt, st);
+        case 1: return launch_select_form<1>(A, npt, st);
+        case 2: return launch_select_form<2>(A, npt, st);
+        case 3: return launch_select_form<3>(A, npt, st);
+        case 4: return launch_select_form<4>(A, npt, st);
         default: return hipErrorInvalidValue;
         }
     }

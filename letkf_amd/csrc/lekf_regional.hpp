@@ -26,7 +26,7 @@ struct RegObsArgs {
 };
 
 struct RegionalArgs {
-    int nx, ny, nlev, nbkt, nobs_max;
+    int nx, ny, nlev, nbkt, nobs_max, nbinned;
     double dx, dy, sigma_h, sigma_v, dlon_zero, dlat_zero;
     const double* zlev;                     // nlev level heights (m)
     const int* cellcum;                     // nx * ny inclusive cumulative obs counts, (j, i) order

@@ -12,10 +12,10 @@ selection (obs_local), the local solve (letkf_core) and the apply.
 Prints ONE JSON line.  value = plain-FP64 local analyses/s (inputs resident in
 HBM).  Beside it: the FP32 and split-BF16x3 forms, p50/p99 cycle latency of
 every form (with and without the host-to-device obs upload), every form's
-error against the reference Fortran letkf_core on a seeded sample of points,
-the roofline of the dominant kernel (HIP events around its launches on the
-handle's stream), the reference Fortran timed on this host's cores, and the
-other configurations (SPEEDY-sized, GFS-sized, k=256, a served stream).
+error against the reference letkf_core on a seeded sample of points (the
+Fortran; without its build the oracle's C restatement of it), the roofline of
+the dominant kernel (HIP events around its launches on the handle's stream),
+the same letkf_core timed on this host's cores, and the other configurations (SPEEDY-sized, GFS-sized, k=256, a served stream).
 """
 from __future__ import annotations
 
@@ -86,8 +86,8 @@ def radar_scan_records(p):
     """Obs records the regional selection scans per cycle: at every point, the obs
     of the cells of its search rectangle's rows that can hold an obs within the
     cutoff (rows trimmed as the selection trims them; the same horizontal set at
-    each of the nlev levels of a column).  Each record is 36 B (ri, rj, z, err and
-    the obs index)."""
+    each of the nlev levels of a column).  Each record is 16 B (ri, rj, z and
+    log2 err^2 in FP32)."""
     nx, ny, nlev = p["nx"], p["ny"], p["nlev"]
     dx, dy, sh = p["dx"], p["dy"], p["sigma_h"]
     ci = np.clip(np.ceil(np.asarray(p["ri"]) - 0.5).astype(np.int64), 1, nx)
@@ -141,10 +141,11 @@ def roofline(kt, nobsl, k, nv, steps, profile_name, scan_records=None):
         achieved = fl / tot_s / 1e12
         work = {"flops_per_cycle": float(fl), "kernels": names}
     else:
-        # selection, a scan: the obs records read (36 B per candidate and point)
-        # and the lists written (index + rho, 12 B per kept entry)
+        # selection, a scan: the FP32 records read (16 B per candidate and point;
+        # the candidates evaluated exactly, 32 B more, are not counted) and the
+        # lists written (index + rho, 12 B per kept entry)
         lb = 12.0 * float(nobsl.sum())
-        sb = 36.0 * float(scan_records) if scan_records else 0.0
+        sb = 16.0 * float(scan_records) if scan_records else 0.0
         by = sb + lb
         bound, unit, peak = "hbm", "GB/s", HBM_PEAK_GBS
         achieved = by / per_cycle_s / 1e9
@@ -228,10 +229,13 @@ def radar_headline(args):
     k, nv = p["ne"], p["nv3d"]
     log(f"generated radar 256x256x60 inputs ({p['ri'].size} obs) in {gen_s:.1f}s")
 
-    # seeded sample of points for the reference Fortran (the FP64 oracle at this size)
+    # seeded sample of points for the reference Fortran (the FP64 oracle at this size);
+    # a quarter of them for its C restatement, which takes four times as long
+    import oracle
     rng = np.random.default_rng(11)
     nij = p["nx"] * p["ny"]
-    sample = np.sort(rng.choice(npt, args.cpu_points, replace=False))  # b = lev * nij + ij
+    ncpu = args.cpu_points if oracle.ref_available() else max(1, args.cpu_points // 4)
+    sample = np.sort(rng.choice(npt, ncpu, replace=False))  # b = lev * nij + ij
     s_ij, s_lev = sample % nij, sample // nij
     xb_s = np.ascontiguousarray(p["gues3d"][s_ij, s_lev].transpose(0, 2, 1))  # (pt, var, member)
     spread_s = np.maximum(xb_s.std(axis=2, ddof=1), 1e-300)
@@ -274,8 +278,8 @@ def radar_headline(args):
         log(f"radar {prec}: {ms:.0f} ms/cycle (p99 {f['latency_ms']['p99']:.0f} ms), "
             f"set_obs {r['obs_ms']:.0f} ms")
 
-    # reference Fortran letkf_core + apply on the sample: the FP64 oracle and the CPU baseline
-    import oracle
+    # reference letkf_core + apply on the sample: the FP64 oracle and the CPU baseline (the
+    # Fortran, or where its build is absent the C restatement, equal bit for bit)
     perm, _ = oracle.obs_bins_regional(p["ri"], p["rj"], p["nx"], p["ny"])
     off = np.cumsum([0] + [l[0].size for l in lists])
     hd = np.ascontiguousarray(np.asarray(p["hdxf"])[perm])
@@ -297,14 +301,18 @@ def radar_headline(args):
             f["err_within_budget"] = bool(f["err_vs_oracle"]["max_over_bg_spread"] <= MIXED_BUDGET)
             f["speedup_vs_f64"] = f["local_analyses_per_s"] / forms["f64"]["local_analyses_per_s"]
     cores = host_cores()
+    fortran = oracle.ref_available()
+    how = ("reference Fortran letkf_core + EISPACK + reference DGEMM + apply to 6 variables, "
+           "OpenMP over points" if fortran else
+           "C restatement of letkf_core + EISPACK's eigensolver + apply to 6 variables (numpy), "
+           "a thread per point")
     cpu = {"value": sample.size / t_ref, "unit": "local analyses/s",
-           "cores": oracle.ref_threads(), "kind": "reference",
+           "cores": oracle.ref_threads(), "kind": "reference" if fortran else "restatement",
            "sample": (f"{sample.size} seeded points of the radar 256x256x60 k=50 grid on their "
-                      f"capped local lists (mean {np.mean(np.diff(off)):.0f} obs): reference "
-                      f"Fortran letkf_core + EISPACK + reference DGEMM + apply to 6 variables, "
-                      f"OpenMP over points, {t_ref:.2f} s; selection not timed"),
+                      f"capped local lists (mean {np.mean(np.diff(off)):.0f} obs): {how}, "
+                      f"{t_ref:.2f} s; selection not timed"),
            "host": cores}
-    log(f"reference Fortran on {sample.size} radar points: {t_ref:.1f}s "
+    log(f"{cpu['kind']} on {sample.size} radar points: {t_ref:.1f}s "
         f"({oracle.ref_threads()} threads, nproc {cores['nproc']})")
 
     f64 = forms["f64"]

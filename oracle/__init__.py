@@ -16,6 +16,7 @@ Two legs:
 """
 from __future__ import annotations
 
+import concurrent.futures
 import ctypes
 import os
 from ctypes import POINTER, c_double, c_int, c_long
@@ -504,10 +505,13 @@ def ref_obsope1(elm, rlon, rlat, rlev, odat, v3d, v2d):
 
 
 def ref_solve_apply(loc_off, loc_idx, loc_rho, hdxf, rdiag, dep, xb, infl, fixed_infl=0.0):
-    """Reference letkf_core + apply over packed local problems (OpenMP over points).
+    """Reference letkf_core + apply over packed local problems (OpenMP over points); where
+    the reference build is absent, the C restatement's (solve_apply).
 
     hdxf: (nobs, ne) row = obs; xb: (npt, nv, ne).  Returns (xa, infl_out).
     """
+    if not ref_available():
+        return solve_apply(loc_off, loc_idx, loc_rho, hdxf, rdiag, dep, xb, infl, fixed_infl)
     lib = _lib_ref()
     npt = loc_off.size - 1
     nobs, ne = hdxf.shape
@@ -526,8 +530,35 @@ def ref_solve_apply(loc_off, loc_idx, loc_rho, hdxf, rdiag, dep, xb, infl, fixed
     return xa, inf
 
 
+def solve_apply(loc_off, loc_idx, loc_rho, hdxf, rdiag, dep, xb, infl, fixed_infl=0.0):
+    """ref_solve_apply with letkf_core by the C restatement, which equals the reference's
+    bit for bit (tests/test_oracle_core.py), and Xa = xmean + Xb' T by numpy."""
+    off, idx, rho = (np.asarray(a) for a in (loc_off, loc_idx, loc_rho))
+    hdxf, rdiag, dep, xb, infl = (np.asarray(a, dtype=np.float64)
+                                  for a in (hdxf, rdiag, dep, xb, infl))
+    _lib_c()
+    xa, out = np.empty_like(xb), np.empty(off.size - 1)
+
+    def point(b):
+        o = idx[off[b]:off[b + 1]]
+        r = letkf_core(hdxf[o], rdiag[o], rho[off[b]:off[b + 1]], dep[o], float(infl[b]))
+        xm = xb[b].mean(axis=1, keepdims=True)
+        xa[b] = xm + (xb[b] - xm) @ r["trans"]
+        out[b] = fixed_infl if fixed_infl > 0.0 else r["parm_infl"]
+
+    with concurrent.futures.ThreadPoolExecutor(solve_threads()) as ex:
+        list(ex.map(point, range(off.size - 1)))
+    return xa, out
+
+
+def solve_threads() -> int:
+    """Threads of solve_apply (letkf_core runs outside the interpreter's lock)."""
+    return min(16, len(os.sched_getaffinity(0)))
+
+
 def ref_threads() -> int:
-    return int(_lib_ref().ref_max_threads())
+    """Threads of ref_solve_apply."""
+    return int(_lib_ref().ref_max_threads()) if ref_available() else solve_threads()
 
 
 # ---------------------------------------------------------------------------

@@ -9,7 +9,8 @@ tests/test_oracle_regional.py).  The kept set is also checked against an
 independent sort by (-rho, list position).  The GPU lists must equal the
 oracle's in content and order, and the capped lists must hold u, v, T and q
 obs (a key by err^2/rho would keep only the q obs, whose error is 1e-4).
-Analysis: the reference letkf_core + apply (oracle/_ref) on the capped lists,
+Analysis: the reference letkf_core + apply (oracle/_ref, or the C restatement that
+equals it bit for bit where that build is absent) on the capped lists,
 for the 3-D u, v, T and q rows and, with the level-1 transform, ps, within
 1e-10 of the analysis perturbation scale; q above level 4 is the background
 rebuilt from its mean and perturbations, bit for bit (the SPEEDY rules,

@@ -450,10 +450,11 @@ int lekf_ktime_read(const char *name, double *total_ms, long *launches);
 int lekf_device_count(void);
 /* free and total device memory of the current GPU, bytes */
 int lekf_mem_info(size_t *free_bytes, size_t *total_bytes);
-/* device bytes of the local-solve workspace a grid of npt points at ensemble
- * size k takes under the current tuning (0 for k <= 32), for callers that
- * budget device memory (no counterpart in the reference, which has no device
- * workspace) */
+/* device bytes of the local-solve workspace that npt points at ensemble size k
+ * take at most under the current tuning (0 for k <= 32), for callers that
+ * budget device memory: with jobs that output trans or pao among them; without,
+ * 32 < k <= 64 take about a third (no counterpart in the reference, which has no
+ * device workspace) */
 long lekf_solve_workspace_bytes(long npt, int k);
 const char *lekf_version(void);
 const char *lekf_last_error(void);

@@ -557,7 +557,7 @@ int lekf_mem_info(size_t* free_bytes, size_t* total_bytes)
 long lekf_solve_workspace_bytes(long npt, int k)
 {
     if (npt <= 0 || k < 2 || k > LEKF_KMAX) return 0;
-    return (long)lekf_solve_ws_bytes(npt, k, LEKF_OUT_PLAIN);
+    return (long)lekf_solve_ws_bytes(npt, k, LEKF_OUT_PLAIN | LEKF_OUT_TRANS);
 }
 
 int lekf_core_f64(int ne, int nobs, int nobsl, const double* hdxb, const double* rdiag,

@@ -50,9 +50,9 @@ def test_large_plain_matches_oracle(gpu, k, nv):
               infl_out=inf2, status=st, transm=wm)
     # the second job of the launch outputs trans: the two kernels share the launch
     tr = DeviceArray.zeros((1, k, k), np.float64)
-    sel = npt - 1
+    sel = pts.index((k + 70, 30.0), npt - len(spreads))
     one = {m: DeviceArray.from_numpy(v) for m, v in
-           dict(off=off[sel:sel + 2].copy(), infl=infl[sel:].copy(),
+           dict(off=off[sel:sel + 2].copy(), infl=infl[sel:sel + 1].copy(),
                 inf2=np.zeros(1)).items()}
     core.letkf_core_batch([
         core.make_job(apply=dict(nij=npt, nv3d=nv, nv2d=0, x3b=d["xb"], x3a=xa), **kw),
@@ -81,6 +81,10 @@ def test_large_plain_matches_oracle(gpu, k, nv):
         scale = np.abs(want - xm).max()
         assert np.abs(a[b] - want).max() <= tol * scale + 2 * k * EPS * np.abs(xm).max(), (p, s, kap)
         assert np.abs(w2[b] - ref["transm"]).max() <= tol * np.abs(ref["transm"]).max(), (p, s, kap)
+        if b == sel:  # the second job: trans (column-major) with w-bar in it
+            full = ref["trans"] + ref["transm"][:, None]
+            assert np.abs(tr.numpy()[0].T - full).max() <= tol * np.abs(full).max(), kap
+            assert abs(one["inf2"].numpy()[0] - ref["parm_infl"]) <= tol * abs(ref["parm_infl"])
         if p:
             assert abs(i2[b] - ref["parm_infl"]) <= 1e-12 * abs(ref["parm_infl"]) + tol
         else:

@@ -6,7 +6,7 @@
 // instructions, and the vector instructions that fetch and scale the rows, which do not
 // run beside them (each adds ~4.4 cycles).  128 x 128 x 60 points, k = 50: 203 ms with
 // the columns rounded up to whole 16-column tiles, 147 ms with tiles and strips;
-// half-degree global grid, k = 40: 37 -> 33 ms.  Memory does not show: with every row
+// 192 x 94 x 64 global grid, k = 40: 37 -> 33 ms.  Memory does not show: with every row
 // read from a few hot lines it takes 141 ms, and ordering the workgroups so that an XCD's
 // points share their rows in L2 (misses 54% -> 4%) left it at 147 ms.
 #include "lekf_ktime.hpp"
@@ -46,7 +46,10 @@ __device__ __forceinline__ bool gram_point(const LekfJob* jobs, int njobs, long 
 
 // LDS of a workgroup: C (k x k, leading dimension k + 1), b, then [0] sum w d^2,
 // [4 + w] P3 of wave w
-constexpr size_t gram_lds_doubles(int kmax, int W) { return (size_t)kmax * (kmax + 1) + kmax + 4 + W; }
+constexpr size_t gram_lds_doubles(int kmax, int W)
+{
+    return (size_t)kmax * (kmax + 1) + kmax + 4 + W;
+}
 
 // C, b and the sums of the workgroup's LDS to the point's record
 template <int W>
@@ -121,7 +124,8 @@ constexpr int gram_waves_per_simd(int nt, int mode)
 }
 
 template <int NT, int MODE, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(gram_waves_per_simd(NT, MODE))))
+__global__ __launch_bounds__(64 * W)
+__attribute__((amdgpu_waves_per_eu(gram_waves_per_simd(NT, MODE))))
 void lekf_gram_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
                       double* __restrict__ ws, long gstride, const int* __restrict__ rlist,
                       int* __restrict__ zlist, int* __restrict__ flist)

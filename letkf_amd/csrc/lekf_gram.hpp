@@ -67,9 +67,10 @@ template <int NT>
 __device__ __forceinline__ void gram_f64(const GramIn& I, int lane,
                                          lekf_d4* acc, double& p3, int wv, int nw)
 {
-    // 4-obs steps whose rows are gathered at once (bounded by the registers
+    // k <= 32.  4-obs steps whose rows are gathered at once (bounded by the registers
     // the rows and the NT (NT + 1) / 2 accumulator tiles take)
-    constexpr int SUB = NT == 1 ? 16 : NT == 2 ? 8 : NT == 3 ? 4 : NT == 4 ? 2 : 1;
+    static_assert(NT <= 3, "whole tiles up to k = 32");
+    constexpr int SUB = NT == 1 ? 16 : NT == 2 ? 8 : 4;
     const int lr = lane & 15, kq = lane >> 4, p = I.p, k = I.k;
     for (int q0 = 64 * wv; q0 < p; q0 += 64 * nw) {
         const ObsChunk ch = stage_chunk(I, q0, lane, p3);

@@ -36,9 +36,11 @@ constexpr double c_sqrt(double x)
 
 constexpr double c_exp(double x)
 {
-    // x = n ln 2 + f, |f| <= ln 2 / 2, with ln 2 in two parts
-    int n = (int)(x * 1.4426950408889634 + (x >= 0 ? 0.5 : -0.5));
-    const double f = (x - n * 0.693147180369123816490) - n * 1.90821492927058770002e-10;
+    // x = n ln 2 + f, |f| <= ln 2 / 2; ln 2 in two parts, the first of 16 bits so that
+    // n times it is exact
+    const double hi = 45426.0 / 65536.0, lo = 1.4286068203094172321e-6;
+    int n = (int)(x / (hi + lo) + (x >= 0 ? 0.5 : -0.5));
+    const double f = (x - n * hi) - n * lo;
     double s = 1.0, t = 1.0;
     for (int i = 1; i < 24; ++i) {
         t *= f / i;

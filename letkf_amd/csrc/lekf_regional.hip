@@ -503,7 +503,6 @@ __device__ int cap_stream(SelLds& S, const CapGlobal& G, KeyAt keyat, Emit emit,
 // and merged at once:
 // * a candidate enters iff fewer than cap of S and of the earlier queued
 //   candidates precede it.  All of S precedes it in scan order, so its count there
-//   candidates precede it.  All of S precedes it in scan order, so its count there
 //   is c1, the number of keys <= its key; the block's candidates are ranked by key
 //   (a counting sort over the leading bits of the keys' range), and where c1 and the
 //   rank together reach cap the earlier ones among those ranked before are counted

@@ -15,7 +15,7 @@
 //   6. optionally the fused apply Xa = xmean + Xb' T over the point's state
 //      rows (speedy/letkf/letkf_tools.f90:94-112,164-177,192-197).
 //
-// Two kernel families, chosen by the ensemble size k:
+// Three kernel families, chosen by the ensemble size k:
 //   * k <= 32: one fused kernel, one wave per point; the eigendecomposition is
 //     a one-sided Jacobi with the matrix in registers.
 //   * 32 < k <= LEKF_KSPLIT: a Gram kernel (2-8 waves per point, MFMA) writes
@@ -566,8 +566,8 @@ __device__ __forceinline__ bool big_dual(const LekfJob& J, int p, int k)
 
 // One upper 64 x 64 block of G (p x p, row-major at out) over the k members.
 template <int MODE>
-__device__ __forceinline__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk, double* out,
-                              int lane)
+__device__ __forceinline__ void gram_dual_blk(const LekfJob& J, long off, int p, int k, int tblk,
+                                              double* out, int lane)
 {
     constexpr int NB = kBlkNB;
     const int nbp = (p + 16 * NB - 1) / (16 * NB);
@@ -735,7 +735,8 @@ __device__ __forceinline__ void gram_dual_blk(const LekfJob& J, long off, int p,
 // record out: [C | b | sum w d^2 | P3] (64 x 64 blocks of the augmented
 // (k+1)^2 product), or a block of G in the dual form.
 template <int MODE>
-__device__ __forceinline__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out, int lane)
+__device__ __forceinline__ void gram_blk_point(const LekfJob& J, int b, int tblk, double* out,
+                                               int lane)
 {
     constexpr int NB = kBlkNB;
     const int k = J.k;
@@ -1315,7 +1316,7 @@ __device__ void eig_tridiag64(EigLds& L, int n, int lda, int lane)
 // lane-per-row QL sweeps read contiguously.
 constexpr int kRowBatch = 8;  // rows in flight per lane in the global-memory reduction
 
-template <int NR, bool FORMQ = true>
+template <int NR>
 __device__ void big_tridiag(double* A, int n, int lda, double* d, double* e, double* tauv, int lane)
 {
     for (int j = 0; j + 2 < n; ++j) {
@@ -1424,7 +1425,6 @@ __device__ void big_tridiag(double* A, int n, int lda, double* d, double* e, dou
         e[n - 1] = 0.0;
     }
     __syncthreads();
-    if (!FORMQ) return;
     // Q = H_0 ... H_{n-3} from the right end, as in eig_tridiag; the reflector
     // of step j is in row j, columns j+1..
     for (int r = lane; r < 4; r += 64) {
@@ -1542,8 +1542,8 @@ __device__ __forceinline__ double wave_sum8(const double (&a)[8], int lane)
 // columns s+1..) are as big_tridiag leaves them, the elementwise update being rounded
 // identically.
 template <int NR>
-__device__ __forceinline__ void big_tridiag_sym(double* A, int n, int lda, double* d, double* e, double* tauv,
-                                double* red, int lane, int wv)
+__device__ __forceinline__ void big_tridiag_sym(double* A, int n, int lda, double* d, double* e,
+                                                double* tauv, double* red, int lane, int wv)
 {
     double vp[NR], wp[NR], v[NR];
 #pragma unroll
@@ -1927,16 +1927,12 @@ __device__ int eig_reg(EigLds& L, int n, int lda, int lane)
 __host__ __device__ inline long big_rot_cap(int kmax) { return 2 * (2L * kmax * kmax + 4L * kmax); }
 __host__ __device__ inline long big_stride(int kmax) { return gram_stride(kmax) + big_rot_cap(kmax); }
 
-// the vectors carried along: nrow rows of R (k apart), then v1, then v2
+// the vectors carried along: nrow rows of R (k apart), then v1
 struct VecSet {
     double* R;
     int nrow, k;
     double* v1;
-    double* v2;
-    __device__ double* at(int q) const
-    {
-        return q < nrow ? R + (size_t)q * k : (q == nrow ? v1 : v2);
-    }
+    __device__ double* at(int q) const { return q < nrow ? R + (size_t)q * k : v1; }
 };
 
 // y <- Q^T y (transpose: H_0 first) or y <- Q y (H_{n-3} first) for nvec
@@ -1944,8 +1940,9 @@ struct VecSet {
 // The waves take the vectors in turns of two, held in registers (lane l: elements
 // l, l + 64, ..); the next reflector is loaded while one is applied.
 template <int NR>
-__device__ __forceinline__ void big_refl_vecs(const double* A, int n, int lda, const double* tauv, const VecSet& V,
-                              int nvec, bool transpose, int lane, int wv)
+__device__ __forceinline__ void big_refl_vecs(const double* A, int n, int lda, const double* tauv,
+                                              const VecSet& V, int nvec, bool transpose, int lane,
+                                              int wv)
 {
     auto load = [&](int s, double (&v)[NR]) {
         const int j = transpose ? s : n - 3 - s;
@@ -2242,8 +2239,8 @@ __device__ __forceinline__ void ql_back_vec(EigLds& L, const VecSet& V, int nvec
 // (k-1)/alpha bounds the spectrum from below; gam > 0: the dual form (g0 = gam = shift).
 // Returns the status bits.
 template <int MODE>
-__device__ __forceinline__ int big_spectral(EigLds& L, int n, int k, double shift, double gam, const VecSet& V,
-                            double* wsp, long wcap, int tid)
+__device__ __forceinline__ int big_spectral(EigLds& L, int n, int k, double shift, double gam,
+                                            const VecSet& V, double* wsp, long wcap, int tid)
 {
     const int lane = tid & 63, wv = tid >> 6;
     const double g0 = gam;  // T + g0 has the spectrum of C + (k-1)/alpha
@@ -2312,8 +2309,8 @@ __device__ __forceinline__ int big_spectral(EigLds& L, int n, int k, double shif
 //   w-bar = B^T U diag(1/(gamma + s)) U^T (sqrt(w) d).
 // G's tridiagonalisation runs exactly as C's, carrying sqrt(w) d and B x'_r.
 template <int MODE>
-__device__ __forceinline__ void big_vec_point(const LekfJob& J, int b, double* rec, double* wsp, long wcap,
-                              EigLds& L, int tid)
+__device__ __forceinline__ void big_vec_point(const LekfJob& J, int b, double* rec, double* wsp,
+                                              long wcap, EigLds& L, int tid)
 {
     constexpr int NT = 64 * kBigW;
     const int lane = tid & 63, wv = tid >> 6;
@@ -2408,7 +2405,7 @@ __device__ __forceinline__ void big_vec_point(const LekfJob& J, int b, double* r
         }
         __syncthreads();
         big_tridiag_sym<4>(rec, n, n, L.d, L.e, L.tau, L.rot, lane, wv);
-        const VecSet V{L.R, nrow, ks, L.B, nullptr};
+        const VecSet V{L.R, nrow, ks, L.B};
         big_refl_vecs<4>(rec, n, n, L.tau, V, nrow + 1, true, lane, wv);
         __syncthreads();
         status |= big_spectral<MODE>(L, n, k, gam, dual ? gam : 0.0, V, wsp, wcap, tid);
@@ -2489,12 +2486,13 @@ __device__ __forceinline__ void big_vec_point(const LekfJob& J, int b, double* r
 // the optional trans/transm/pao outputs and the fused apply
 // Xa = x-mean + X' T evaluated as x-mean + (X' V) diag(sqrt((k-1)/L)) V^T
 // + (X' w-bar) 1^T.
+//
 // The solve with recorded rotations (32 < k <= 64, three kernels per sub-batch,
-// for the jobs that output trans or pao): the point's record carries, after the Gram, the Householder Q (transposed: Q_rt
-// at qoff + t k + r), the tridiagonal d and e, then the eigenvalues, the
-// rotation-stream length and the QL status written by the QL kernel.  The
-// rotation stream of a point holds, per QL sweep, a header (m, count) and the
-// sweep's (c, s) pairs for i = m-1 down to m-count.
+// for the jobs that output trans or pao): the point's record carries, after the
+// Gram, the Householder Q (transposed: Q_rt at qoff + t k + r), the tridiagonal
+// d and e, then the eigenvalues, the rotation-stream length and the QL status
+// written by the QL kernel.  The rotation stream of a point holds, per QL sweep,
+// a header (m, count) and the sweep's (c, s) pairs for i = m-1 down to m-count.
 struct SplitRec {
     long qoff, doff, eoff, lamoff, cntoff, flagoff;
     const double* rot;  // this point's rotation stream
@@ -2983,7 +2981,8 @@ __global__ __launch_bounds__(64) void lekf_ql_kernel(const LekfJob* __restrict__
 
 // Kernel 3 for jobs that output trans or pao (one wave per point): the
 // eigenvectors by replaying the rotations on Q, then the W assembly,
-// inflation, outputs and the fused apply of eig_point.  A point whose stream overflowed is left to lekf_eig_fix_kernel.
+// inflation, outputs and the fused apply of eig_point.  A point whose stream
+// overflowed is left to lekf_eig_fix_kernel.
 template <int KR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(eig_waves_per_simd(KR))))
 void lekf_eig3_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
@@ -3071,10 +3070,8 @@ __global__ __launch_bounds__(64) void lekf_big_kernel(const LekfJob* __restrict_
 // read and written per point) and its 2 barriers per step.
 template <int MODE>
 __global__ __launch_bounds__(64 * kBigW) __attribute__((amdgpu_waves_per_eu(2)))
-void lekf_bigvec_kernel(const LekfJob* __restrict__ jobs,
-                                                                 int njobs, long npt,
-                                                                 double* __restrict__ ws,
-                                                                 long gstride, int nvmax, int kmax)
+void lekf_bigvec_kernel(const LekfJob* __restrict__ jobs, int njobs, long npt,
+                        double* __restrict__ ws, long gstride, int nvmax, int kmax)
 {
     extern __shared__ double smem[];
     const int tid = threadIdx.x, nblk = gram_nblk(kmax);
@@ -3433,7 +3430,6 @@ hipError_t lekf_solve_launch(const LekfJob* djobs, int njobs, long npt, int kmax
     if (npt <= 0) return hipSuccess;
     if (nvmax > LEKF_NVMAX) return hipErrorInvalidValue;
     const int cls = lekf_solve_class(kmax);
-    if (mode == 0) return launch_mode<0>(cls, djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
-    if (mode == 1) return launch_mode<1>(cls, djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
-    return launch_mode<2>(cls, djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
+    const auto fn = mode == 0 ? launch_mode<0> : mode == 1 ? launch_mode<1> : launch_mode<2>;
+    return fn(cls, djobs, njobs, npt, kmax, nvmax, outs, ws, ws_bytes, st);
 }

@@ -37,7 +37,10 @@ constexpr int kSplitRedo = 16;
 // overflowed, or its condition number is past the rational form's tables), which finds
 // its slot in flist (flist[0] entries from flist[1])
 constexpr int kSplitOverflow = 8;
-__device__ inline void split_flag_slot(int* flist, long slot) { flist[1 + atomicAdd(flist, 1)] = (int)slot; }
+__device__ inline void split_flag_slot(int* flist, long slot)
+{
+    flist[1 + atomicAdd(flist, 1)] = (int)slot;
+}
 
 // Flat point of slot `slot` of a split kernel: pass 0 the sub-batch's own
 // (gp0 + slot, nb slots), pass 1 the redo list's (rlist[0] entries from

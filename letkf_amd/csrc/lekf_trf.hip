@@ -26,12 +26,12 @@ __host__ __device__ constexpr int trf_slots(int k) { return (k + 7) / 8; }
 __host__ __device__ constexpr int trf_ldz(int kmax) { return kmax | 1; }
 __host__ __device__ constexpr int trd_lds_doubles(int NB, int nvmax, int kmax)
 {
-    return 16 * trf_ld(8, NB) + 24 * NB + LEKF_NVMAX + 1 + nvmax * trf_ldz(kmax);
+    return 16 * trf_ld(NB) + 24 * NB + LEKF_NVMAX + 1 + nvmax * trf_ldz(kmax);
 }
 __host__ __device__ constexpr int trf_lds_doubles(int NB, int NE, int kmax)
 {
     // (d, e), tau, the row of b's solution, then rows and factors or a stage's reflectors
-    const int a = (8 * NE + 9) * trf_ldz(8 * NB), b = 64 * trf_ld(8, NB);
+    const int a = (8 * NE + 9) * trf_ldz(8 * NB), b = 64 * trf_ld(NB);
     return 16 * NB + 8 * NB + 8 * NB + LEKF_NVMAX + 1 + 1 + (a > b ? a : b);
 }
 
@@ -103,7 +103,7 @@ void lekf_trd_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
 {
 #pragma clang fp contract(off)
     extern __shared__ double smem[];
-    constexpr int P = 8, LD = trf_ld(P, NB);
+    constexpr int LD = trf_ld(NB);
     long gp;
     if (!split_slot_point(blockIdx.x, gp0, (long)gridDim.x, pass, rlist, gp)) return;
     const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
@@ -168,8 +168,8 @@ void lekf_trd_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
             X[e][q] = x;
         }
     bool bad = false;
-    trf_reduce<0, P, NB, NE>(M, X, k, k, r, c, lane, vx, vw, es, ts, bad);
-    trf_diagonal<P, NB>(M, k, r, c, ds, es);
+    trf_reduce<0, NB, NE>(M, X, k, r, c, lane, vx, vw, es, ts, bad);
+    trf_diagonal<NB>(M, k, r, c, ds, es);
     __syncthreads();
     tr = wave_sum(tr);
     // bounds of the spectrum: C is positive semidefinite, so A >= shift up to the
@@ -243,7 +243,7 @@ template <int T, int NB, int NE>
 __device__ __forceinline__ void trf_back(double (&out)[NE][NB], double (&st)[NB], int k, int r,
                                          int c, const double* V, double* vst, const double* ts)
 {
-    constexpr int P = 8, LD = trf_ld(P, NB);
+    constexpr int LD = trf_ld(NB);
     __syncthreads();
 #pragma unroll
     for (int q = T; q < NB; ++q) vst[(r * P + c) * LD + q] = st[q];
@@ -256,7 +256,7 @@ __device__ __forceinline__ void trf_back(double (&out)[NE][NB], double (&st)[NB]
             st[q] = (j < k && i < j) ? V[(long)i * k + j] : 0.0;
         }
     }
-    trf_back_stage<T, P, NB, NE>(out, k, k, c, vst, ts);
+    trf_back_stage<T, NB, NE>(out, k, c, vst, ts);
     if constexpr (T > 0) trf_back<T - 1, NB, NE>(out, st, k, r, c, V, vst, ts);
 }
 
@@ -268,7 +268,7 @@ void lekf_trf_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
 {
 #pragma clang fp contract(off)
     extern __shared__ __align__(16) double smem[];
-    constexpr int P = 8, KP = P * NB, ldz = trf_ldz(KP);
+    constexpr int KP = P * NB, ldz = trf_ldz(KP);
     long gp;
     if (!split_slot_point(blockIdx.x, gp0, (long)gridDim.x, pass, rlist, gp)) return;
     const LekfJob& J = jobs[lekf_job_of(jobs, njobs, gp)];
@@ -335,7 +335,7 @@ void lekf_trf_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
         const int rb = nvmax - P * e;  // grid row of b in this group
-        trf_function<P, NB>(zl + (P * e + r) * ldz, de, k, lev, 8 + 4 * lev, m, scale,
+        trf_function<NB>(zl + (P * e + r) * ldz, de, k, lev, m, scale,
                             rb >= 0 && rb < P ? rb : -1, r, c, tl, ldz, out[e]);
         if (r == rb) {
 #pragma unroll
@@ -350,7 +350,7 @@ void lekf_trf_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
         double s = 0.0;
 #pragma unroll
         for (int q = 0; q < NB; ++q) s = fma(zl[(P * e + r) * ldz + c + P * q], yb[c + P * q], s);
-        cw[e] = grid_sum_c<P>(s);
+        cw[e] = grid_sum_c(s);
     }
     double st[NB];
 #pragma unroll
@@ -407,7 +407,8 @@ static hipError_t launch_trf(long nb, hipStream_t st, const LekfJob* djobs, int 
     {
         KTime kt(pass ? "redo_tri" : "eig_tri", st);
         hipLaunchKernelGGL((lekf_trd_kernel<NB, NE>), dim3((unsigned)nb), dim3(LEKF_WAVE), dlds, st,
-                           djobs, njobs, g0, ws, gs, nvmax, kmax, pass, mode, kthr, rlist, lcap, flist);
+                           djobs, njobs, g0, ws, gs, nvmax, kmax, pass, mode, kthr, rlist, lcap,
+                           flist);
     }
     KTime kt(pass ? "redo_apply" : "eig_apply", st);
     hipLaunchKernelGGL((lekf_trf_kernel<NB, NE>), dim3((unsigned)nb), dim3(LEKF_WAVE), flds, st,

@@ -1,4 +1,4 @@
-// lekf_trf.hpp -- the local solve without eigenvalues, on a P x P grid of lanes.
+// lekf_trf.hpp -- the local solve without eigenvalues, on a P x P grid of lanes (P = 8).
 //
 // The analysis needs three functions of A = C + (k-1)/alpha I (k x k, positive
 // definite): A^-1 b and, for each state row x, x A^-1/2 and x A^-1 b.  With the
@@ -29,12 +29,11 @@ namespace {
 
 __device__ constexpr lekf_invsqrt::Table g_invsqrt = lekf_invsqrt::make_table();
 
+constexpr int P = 8;  // the wave's grid of lanes
+
 // LDS stride of a vector stored [coordinate][slot]: even (16-byte reads) and such
 // that the P coordinates' reads fall on distinct banks
-__host__ __device__ constexpr int trf_ld(int P, int NB)
-{
-    return P == 8 ? (NB <= 10 ? 10 : 14) : ((NB + 1) & ~1) + 2;
-}
+__host__ __device__ constexpr int trf_ld(int NB) { return NB <= 10 ? 10 : 14; }
 
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double x)
@@ -53,38 +52,30 @@ __device__ __forceinline__ double xor_f64(double x, int j, int lane)
 }
 
 // sum over the P lanes of a grid row (c), in every lane
-template <int P>
 __device__ __forceinline__ double grid_sum_c(double x)
 {
-    x += dpp_f64<0xB1>(x);                // quad_perm [1,0,3,2]
-    x += dpp_f64<0x4E>(x);                // quad_perm [2,3,0,1]
-    if (P == 8) x += dpp_f64<0x141>(x);   // row_half_mirror: the other quad
+    x += dpp_f64<0xB1>(x);   // quad_perm [1,0,3,2]
+    x += dpp_f64<0x4E>(x);   // quad_perm [2,3,0,1]
+    x += dpp_f64<0x141>(x);  // row_half_mirror: the other quad
     return x;
 }
 
 // sum over the grid rows (r) of a value that is the same in every lane of a row
-template <int P>
 __device__ __forceinline__ double grid_sum_r(double x, int lane)
 {
-    if (P == 4) x += dpp_f64<0x141>(x);   // row_half_mirror: r ^ 1
-    x += dpp_f64<0x128>(x);               // row_ror:8
-    if (P == 8) {
-        x += xor_f64(x, 16, lane);
-        x += xor_f64(x, 32, lane);
-    }
+    x += dpp_f64<0x128>(x);  // row_ror:8
+    x += xor_f64(x, 16, lane);
+    x += xor_f64(x, 32, lane);
     return x;
 }
 
 // v[0..P-1] summed over the P lanes of a grid row, element c to lane c
-template <int P>
 __device__ __forceinline__ double grid_scatter_c(double (&v)[P], int c)
 {
-    if (P == 8) {
 #pragma unroll
-        for (int u = 0; u < P / 2; ++u) {
-            const double keep = (c & 4) ? v[u + P / 2] : v[u], send = (c & 4) ? v[u] : v[u + P / 2];
-            v[u] = keep + dpp_f64<0x141>(send);
-        }
+    for (int u = 0; u < P / 2; ++u) {
+        const double keep = (c & 4) ? v[u + P / 2] : v[u], send = (c & 4) ? v[u] : v[u + P / 2];
+        v[u] = keep + dpp_f64<0x141>(send);
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -98,22 +89,20 @@ __device__ __forceinline__ double grid_scatter_c(double (&v)[P], int c)
 // Householder steps s = P T .. P T + P - 1 of the point's matrix (those below
 // k - 2), each applied to M from both sides and to the rows X from the right:
 // H = I - tau v v^T, v zero up to s, v[s+1] = v0.  On exit row s of M holds v
-// (columns above s), es[s] the off-diagonal and ts[s] tau.  kw: the largest k in
-// the wave (a point past its own last step gets tau = 0).  vx, vw: P * trf_ld
-// doubles of LDS each, es and ts P * NB, all of this point.  bad: an entry of the
-// reduction was not finite.
-template <int T, int P, int NB, int NE>
-__device__ __forceinline__ void trf_stage(double (&M)[NB][NB], double (&X)[NE][NB], int k, int kw,
-                                          int r, int c, int lane, double* vx, double* vw,
+// (columns above s), es[s] the off-diagonal and ts[s] tau.  vx, vw: P * trf_ld doubles of
+// LDS each, es and ts P * NB.  bad: an entry of the reduction was not finite.
+template <int T, int NB, int NE>
+__device__ __forceinline__ void trf_stage(double (&M)[NB][NB], double (&X)[NE][NB], int k, int r,
+                                          int c, int lane, double* vx, double* vw,
                                           double* es, double* ts, bool& bad)
 {
 #pragma clang fp contract(off)
-    constexpr int LD = trf_ld(P, NB);
+    constexpr int LD = trf_ld(NB);
     constexpr int T1 = T + 1 < NB ? T + 1 : T;
 #pragma unroll 1
     for (int u = 0; u < P; ++u) {
         const int s = P * T + u;
-        if (s >= kw - 2) break;
+        if (s >= k - 2) break;
         if (r == u) {
 #pragma unroll
             for (int b = T; b < NB; ++b) vx[c * LD + b] = M[T][b];
@@ -131,16 +120,15 @@ __device__ __forceinline__ void trf_stage(double (&M)[NB][NB], double (&X)[NE][N
         double n2 = 0.0;
 #pragma unroll
         for (int b = T; b < NB; ++b) n2 = fma(xc[b], xc[b], n2);
-        n2 = grid_sum_c<P>(n2);
-        const bool mine = s < k - 2;
-        bad |= mine && !(n2 <= 1.0e300);
-        const bool live = mine && n2 > 1.0e-280;
+        n2 = grid_sum_c(n2);
+        bad |= !(n2 <= 1.0e300);
+        const bool live = n2 > 1.0e-280;
         const double n2s = live ? n2 : 1.0;
         const double nrm = n2s * rsq_nr(n2s);
         const double al = x0 >= 0.0 ? -nrm : nrm;
         const double v0 = x0 - al;
         const double tau = live ? rcp_nr(nrm * (nrm + fabs(x0))) : 0.0;
-        if (r == 0 && c == 0 && mine) {
+        if (r == 0 && c == 0) {
             es[s] = live ? al : x0;
             ts[s] = tau;
         }
@@ -161,19 +149,19 @@ __device__ __forceinline__ void trf_stage(double (&M)[NB][NB], double (&X)[NE][N
             double t = M[a][T] * xc[T];
 #pragma unroll
             for (int b = T + 1; b < NB; ++b) t = fma(M[a][b], xc[b], t);
-            p[a] = grid_sum_c<P>(t);
+            p[a] = grid_sum_c(t);
         }
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
             double t = X[e][T] * xc[T];
 #pragma unroll
             for (int b = T + 1; b < NB; ++b) t = fma(X[e][b], xc[b], t);
-            px[e] = tau * grid_sum_c<P>(t);
+            px[e] = tau * grid_sum_c(t);
         }
         double pv = p[T] * xr[T];
 #pragma unroll
         for (int a = T + 1; a < NB; ++a) pv = fma(p[a], xr[a], pv);
-        pv = grid_sum_r<P>(pv, lane);
+        pv = grid_sum_r(pv, lane);
         const double g = 0.5 * tau * tau * pv;
         // w = tau p - g v, zero up to s
 #pragma unroll
@@ -199,18 +187,18 @@ __device__ __forceinline__ void trf_stage(double (&M)[NB][NB], double (&X)[NE][N
     }
 }
 
-template <int T, int P, int NB, int NE>
-__device__ __forceinline__ void trf_reduce(double (&M)[NB][NB], double (&X)[NE][NB], int k, int kw,
-                                           int r, int c, int lane, double* vx, double* vw,
+template <int T, int NB, int NE>
+__device__ __forceinline__ void trf_reduce(double (&M)[NB][NB], double (&X)[NE][NB], int k, int r,
+                                           int c, int lane, double* vx, double* vw,
                                            double* es, double* ts, bool& bad)
 {
-    trf_stage<T, P, NB, NE>(M, X, k, kw, r, c, lane, vx, vw, es, ts, bad);
+    trf_stage<T, NB, NE>(M, X, k, r, c, lane, vx, vw, es, ts, bad);
     if constexpr (T + 1 < NB)
-        trf_reduce<T + 1, P, NB, NE>(M, X, k, kw, r, c, lane, vx, vw, es, ts, bad);
+        trf_reduce<T + 1, NB, NE>(M, X, k, r, c, lane, vx, vw, es, ts, bad);
 }
 
 // The diagonal to ds and the last off-diagonal to es (es[k-1] = 0).
-template <int P, int NB>
+template <int NB>
 __device__ __forceinline__ void trf_diagonal(const double (&M)[NB][NB], int k, int r, int c,
                                              double* ds, double* es)
 {
@@ -246,11 +234,11 @@ __device__ __forceinline__ int trf_level(double hi, double m)
 // summed on the way back and element i = c + P b of the result lands in out[b] of
 // lane c.  zrow: this lane's row in LDS; de: (d_i, e_i) pairs with (1, 0) from k on;
 // tl: (P + 1) * ldt doubles for the factors e_i / delta_i of the P shifts (b's own
-// shift 0 in the last).  nmax: the most shifts of a point in the wave.  The y of the forward pass stay in registers.
-template <int P, int NB>
-__device__ __forceinline__ void trf_function(const double* zrow, const double2* de, int kw, int lev,
-                                             int nmax, double m, double scale, int rb, int r, int c,
-                                             double* tl, int ldt, double (&out)[NB])
+// shift 0 in the last).  The y of the forward pass stay in registers.
+template <int NB>
+__device__ __forceinline__ void trf_function(const double* zrow, const double2* de, int k, int lev,
+                                             double m, double scale, int rb, int r, int c, double* tl,
+                                             int ldt, double (&out)[NB])
 {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -260,7 +248,7 @@ __device__ __forceinline__ void trf_function(const double* zrow, const double2* 
     // one grid row writes the factors of the shifts; b's lane of shift 0 its own
     const bool shared = r == (rb == 0 ? 1 : 0), own = isb && c == 0;
     double* tw = tl + (own ? P : c) * ldt;
-    for (int pass = 0; pass * P < nmax; ++pass) {
+    for (int pass = 0; pass * P < N; ++pass) {
         const int j = pass * P + c;
         double sh = m, wt = 0.0;
         if (own) {
@@ -274,7 +262,7 @@ __device__ __forceinline__ void trf_function(const double* zrow, const double2* 
         double t = 0.0, yp = 0.0, ep = 0.0;
 #pragma unroll
         for (int i = 0; i < P * NB; ++i)
-            if (i < kw) {
+            if (i < k) {
                 const double2 q = de[i];
                 const double rr = rcp_nr(fma(-ep, t, q.x + sh));
                 yp = fma(-t, yp, wt * zrow[i]);
@@ -287,18 +275,18 @@ __device__ __forceinline__ void trf_function(const double* zrow, const double2* 
         double x = 0.0;
 #pragma unroll
         for (int b = NB - 1; b >= 0; --b)
-            if (P * b < kw) {
+            if (P * b < k) {
                 double v[P];
 #pragma unroll
                 for (int u = P - 1; u >= 0; --u) {
                     const int i = P * b + u;
                     v[u] = 0.0;
-                    if (i < kw) {
+                    if (i < k) {
                         x = fma(-tw[i], x, y[i]);
                         v[u] = x;
                     }
                 }
-                out[b] += grid_scatter_c<P>(v, c);
+                out[b] += grid_scatter_c(v, c);
             }
         __syncthreads();
     }
@@ -306,17 +294,17 @@ __device__ __forceinline__ void trf_function(const double* zrow, const double2* 
 
 // rows <- rows H_s for s = P T + P - 1 down to P T (those below k - 2); vst: the
 // stage's P reflectors in LDS, [u][coordinate][slot]; ts: tau
-template <int T, int P, int NB, int NE>
-__device__ __forceinline__ void trf_back_stage(double (&out)[NE][NB], int k, int kw, int c,
-                                               const double* vst, const double* ts)
+template <int T, int NB, int NE>
+__device__ __forceinline__ void trf_back_stage(double (&out)[NE][NB], int k, int c, const double* vst,
+                                               const double* ts)
 {
 #pragma clang fp contract(off)
-    constexpr int LD = trf_ld(P, NB);
+    constexpr int LD = trf_ld(NB);
 #pragma unroll 1
     for (int u = P - 1; u >= 0; --u) {
         const int s = P * T + u;
-        if (s >= kw - 2) continue;
-        const double tau = s < k - 2 ? ts[s] : 0.0;
+        if (s >= k - 2) continue;
+        const double tau = ts[s];
         double v[NB];
 #pragma unroll
         for (int b = T; b < NB; ++b) v[b] = vst[(u * P + c) * LD + b];
@@ -326,7 +314,7 @@ __device__ __forceinline__ void trf_back_stage(double (&out)[NE][NB], int k, int
             double t = out[e][T] * v[T];
 #pragma unroll
             for (int b = T + 1; b < NB; ++b) t = fma(out[e][b], v[b], t);
-            t = tau * grid_sum_c<P>(t);
+            t = tau * grid_sum_c(t);
 #pragma unroll
             for (int b = T; b < NB; ++b) out[e][b] = fma(-t, v[b], out[e][b]);
         }

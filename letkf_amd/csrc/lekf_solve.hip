@@ -2247,7 +2247,9 @@ __device__ __forceinline__ int big_spectral(EigLds& L, int n, int k, double shif
     const double m = shift * (MODE == 0 ? 0.999 : 0.75);
     const int lev = big_level(L, n, g0, m, lane);
     int status = 0;
-    if (lev < (MODE == 0 ? lekf_invsqrt::kLevels : 5)) {
+    // (said to the compiler, since QL's code beside it otherwise costs these points 1%)
+    if (__builtin_expect_with_probability(lev < (MODE == 0 ? lekf_invsqrt::kLevels : 5), 1,
+                                          0.9999)) {
         const long w = wcap / (2 * n);
         big_function(L, n, g0, m, sqrt((double)(k - 1) * m), gam, lev, V, wsp,
                      w < 64 * kBigW ? (int)w : 64 * kBigW, tid);

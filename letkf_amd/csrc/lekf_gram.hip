@@ -3,12 +3,12 @@
 // W waves per point; wave w takes every W-th chunk of 64 local obs, and the partial
 // Grams are summed in LDS in wave order (deterministic for a given W), then written to
 // the point's workspace record.  The FP64 form is bound by issue: its matrix
-// instructions, and the vector instructions that fetch and scale the rows, which do not
-// run beside them (each adds ~4.4 cycles).  128 x 128 x 60 points, k = 50: 203 ms with
-// the columns rounded up to whole 16-column tiles, 147 ms with tiles and strips;
-// 192 x 94 x 64 global grid, k = 40: 37 -> 33 ms.  Memory does not show: with every row
-// read from a few hot lines it takes 141 ms, and ordering the workgroups so that an XCD's
-// points share their rows in L2 (misses 54% -> 4%) left it at 147 ms.
+// instructions (busy 70% of the time at 256 x 256 x 60, k = 50), and the vector
+// instructions that fetch and scale the rows, which do not run beside them.  128 x 128 x
+// 60 points, k = 50: 203 ms with the columns rounded up to whole 16-column tiles, 147 ms
+// with tiles and strips; 192 x 94 x 64 global grid, k = 40: 37 -> 33 ms.  Memory does not
+// show: with every row read from a few hot lines it takes 141 ms, and ordering the
+// workgroups so that an XCD's points share their rows in L2 left it at 147 ms.
 #include "lekf_ktime.hpp"
 #include "lekf_gram.hpp"
 #include "lekf_split.hpp"

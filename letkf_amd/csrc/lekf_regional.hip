@@ -513,11 +513,11 @@ __device__ int cap_stream(SelLds& S, const CapGlobal& G, KeyAt keyat, Emit emit,
 //   slot of the i-th largest entry that left: the reference evicts the current last
 //   entry each time, and the last key only falls; an entrant that leaves in its own
 //   block hands its slot on (pointer jumping).
-// Bound by VALU issue, 62% of it at three waves per SIMD.  Against blocks of 64 sorted
-// across the lanes with every candidate evaluated exactly as it was scanned, a stream
-// takes 46 k vector and 17 k scalar instructions instead of 69 k and 42 k, and the
-// radar 128 x 128 x 60 selection (two streams of 12.5 k candidates per point) 251
-// instead of 401 ms per cycle; the GFS-sized grid's list_cap_wave 22 instead of 33 ms.
+// Bound by VALU issue: 67% busy at three waves per SIMD, 52 k vector and 18 k scalar
+// instructions a stream (radar 256 x 256 x 60, two streams of 12.6 k candidates per point).
+// Against blocks of 64 sorted across the lanes with every candidate evaluated exactly as
+// it was scanned, the radar 128 x 128 x 60 selection takes 251 instead of 401 ms per cycle,
+// the GFS-sized grid's list_cap_wave 22 instead of 33 ms.
 // ---------------------------------------------------------------------------
 
 // order of the lanes' LDS traffic within the wave (no cross-wave sharing)

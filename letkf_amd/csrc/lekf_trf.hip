@@ -8,8 +8,8 @@
 // rational form's tables (or are not finite) is flagged, listed and left to
 // lekf_eig_fix_kernel, whose Gram is still at the start of the record.
 //
-// Both are bound by VALU issue at two to four waves per SIMD (about 170 FP64
-// operations per Householder step at k = 50, half of them the rank-2 update; a step's
+// Both are bound by VALU issue at two to four waves per SIMD (75% and 60% busy at k = 50;
+// about 170 FP64 operations per Householder step, half of them the rank-2 update; a step's
 // chain of reductions, rsq and rcp is what the second and third wave cover).
 // Against the recorded-rotation solve it replaced for these jobs (Householder with Q,
 // QL one lane per point, rotation replay), per cycle: radar 128 x 128 x 60, k = 50:
@@ -88,7 +88,12 @@ __device__ void trf_extremes(const double* ds, const double* es, int k, int lane
     lmin = 0.5 * (a[1] + b[1]);
 }
 
-// Registers per lane: the matrix takes 2 NB^2 of them until its slots are finished.
+// Registers per lane: the matrix takes 2 NB^2 of them until its slots are finished.  Held to
+// these waves lekf_trd_kernel spills at NB = 5, 8 and 9 (72, 64 and 244 bytes a lane with one
+// row group, 164, 212 and 404 with three).  20,000 points, ms with one wave per SIMD fewer:
+// one group k = 40 0.36 (0.34 so), k = 64 1.44 (0.91), k = 72 1.76 (1.50); three groups k = 40
+// 0.42 (0.56), k = 64 1.53 (1.22), k = 72 1.92 (2.67): the two slower ones are the price of one
+// rule for both.
 constexpr int trd_waves_per_simd(int nb) { return nb <= 5 ? 4 : nb <= 6 ? 3 : nb <= 9 ? 2 : 1; }
 constexpr int trf_waves_per_simd(int nb) { return nb <= 5 ? 4 : nb <= 7 ? 3 : nb <= 8 ? 2 : 1; }
 
@@ -396,7 +401,9 @@ void lekf_trf_kernel(const LekfJob* __restrict__ jobs, int njobs, long gp0,
 }
 
 // the plain solve of a sub-batch: nvmax + 1 rows hang below the matrix, in one
-// group of eight or three
+// group of eight or three (up to 7 state rows, the models' 3-D fields; 8 to 16 pay for
+// 24: 20,000 points at k = 50, reduction and functions 0.68 + 0.24 ms with 7 rows in
+// all, 0.73 + 0.62 with 10, 0.76 + 0.66 with 16)
 template <int NB, int NE>
 static hipError_t launch_trf(long nb, hipStream_t st, const LekfJob* djobs, int njobs, long g0,
                              double* ws, long gs, int nvmax, int kmax, int pass, int mode,

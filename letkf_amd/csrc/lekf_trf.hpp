@@ -237,8 +237,8 @@ __device__ __forceinline__ int trf_level(double hi, double m)
 // shift 0 in the last).  The y of the forward pass stay in registers.
 template <int NB>
 __device__ __forceinline__ void trf_function(const double* zrow, const double2* de, int k, int lev,
-                                             double m, double scale, int rb, int r, int c, double* tl,
-                                             int ldt, double (&out)[NB])
+                                             double m, double scale, int rb, int r, int c,
+                                             double* tl, int ldt, double (&out)[NB])
 {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -295,8 +295,8 @@ __device__ __forceinline__ void trf_function(const double* zrow, const double2* 
 // rows <- rows H_s for s = P T + P - 1 down to P T (those below k - 2); vst: the
 // stage's P reflectors in LDS, [u][coordinate][slot]; ts: tau
 template <int T, int NB, int NE>
-__device__ __forceinline__ void trf_back_stage(double (&out)[NE][NB], int k, int c, const double* vst,
-                                               const double* ts)
+__device__ __forceinline__ void trf_back_stage(double (&out)[NE][NB], int k, int c,
+                                               const double* vst, const double* ts)
 {
 #pragma clang fp contract(off)
     constexpr int LD = trf_ld(NB);

@@ -2,10 +2,10 @@
 
 The FP32 and split-BF16x3 Grams perturb the analysis roughly in proportion to
 the square of the condition number of C + (k-1)/alpha I
-(tests/test_mixed_emulation.py).  On the three-kernel eigensolver
-(32 < k <= 64) the QL kernel flags a point whose condition number exceeds the
-mixed_kappa tuning value (16 times it for FP32, whose Gram rounds finer) and
-lists it; after the launch's last sub-batch one FP64 pass solves the listed
+(tests/test_mixed_emulation.py).  On the split solve (32 < k <= 64) the
+tridiagonal kernel (with trans or pao, or a stream cap, the QL kernel) flags a
+point whose condition number exceeds the mixed_kappa tuning value (16 times it
+for FP32, whose Gram rounds finer) and lists it; after the launch's last sub-batch one FP64 pass solves the listed
 points again from an FP64 Gram, and their status gets LEKF_PT_FP64.  The redo runs the FP64
 form's own kernels, so a redone point equals the FP64 form bit for bit and
 every other point the plain mixed form bit for bit (the reference has one
@@ -125,7 +125,7 @@ def _radar_run(p, prec):
 @pytest.mark.parametrize("rcap", [0, 8])
 def test_radar_redo_is_the_fp64_analysis(gpu, knobs, radar40, rcap):
     """Threshold 1 redoes every point with local obs: the BF16x3 handle's analysis
-    is then the FP64 handle's, bit for bit, on the eigenvector-free apply and
+    is then the FP64 handle's, bit for bit, on the rational apply and
     (rotation streams capped at 8) on the overflow fallback."""
     tune.set("split_rcap", rcap)
     tune.set("mixed_kappa", 0)

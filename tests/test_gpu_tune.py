@@ -3,8 +3,9 @@
 The Gram workspace size and the selection slot count only re-partition the
 same per-point work, so the analysis must be bit-identical for every value;
 the Gram wave count re-orders the waves' partial-sum reduction and the
-three-kernel eigensolver applies the eigenvectors without forming them, so
-those agree to rounding (1e-12 of the analysis perturbation scale).
+split solve forms no eigenvectors (a rational form of the functions of the
+tridiagonal matrix), so those agree to rounding (1e-12 of the analysis
+perturbation scale).
 A graph captured before a change is retaken after it, and the autotuner's
 choice is one of the candidates, is applied, and lands in its cache.
 """
@@ -83,10 +84,10 @@ def test_slots_and_workspace_bit_identical(gpu, mk):
 
 @pytest.mark.parametrize("mk", [_radar, _global_capped])
 def test_eig_split_agrees(gpu, mk):
-    """k = 50 and k = 40: the three-kernel eigensolver (Householder, QL with one
-    lane per point recording its rotations, then the apply through Q and the
-    rotations without forming the eigenvectors) agrees with the fused kernel's
-    explicit eigenvectors to rounding; its sub-batching leaves it bit-identical."""
+    """k = 50 and k = 40: the split solve (Householder, then the apply through Q
+    and the rational form of the functions of the tridiagonal matrix, without
+    the eigenvectors) agrees with the fused kernel's explicit eigenvectors to
+    rounding; its sub-batching leaves it bit-identical."""
     job = mk()
     tune.set("eig_split", 1)
     a1 = _analysis(job)
@@ -99,8 +100,9 @@ def test_eig_split_agrees(gpu, mk):
 
 @pytest.mark.parametrize("mk", [_radar, _global_capped])
 def test_split_overflow_fallback(gpu, mk):
-    """A point whose QL rotation stream outgrows its cap is solved by the fused
-    kernel's steps (lekf_eig_fix_kernel) from the Gram still in its record:
+    """A stream cap above 0 has every job take the solve with recorded
+    rotations.  There a point whose QL rotation stream outgrows its cap is solved
+    by the fused kernel's steps (lekf_eig_fix_kernel) from the Gram still in its record:
     with a cap of one rotation every point with obs takes that path (then the
     analysis is the fused kernel's, bit for bit), with 900 some do; both agree
     with the default cap to rounding."""

@@ -157,3 +157,44 @@ def _mixed(k):
                 d = np.abs(a[n][b] - f[n][b]).max()
                 assert d <= tol * np.abs(f[n][b]).max(), (prec, b, kap[b], n, d)
             assert abs(a["infl"][b] - f["infl"][b]) <= 1e-12 * abs(f["infl"][b]), (prec, b)
+
+
+@pytest.mark.parametrize("k", [33, 40, 64])
+@pytest.mark.parametrize("prec,thr", [("f32", 125), ("bf16x3", 2000)])
+def test_redo_list_at_its_edge(gpu, knobs, k, prec, thr):
+    """The FP64 redo of a plain job first bounds the condition number by lambda_max over
+    0.75 (k-1)/infl and takes the extreme eigenvalues only where that passes.  Points of
+    one mode (lambda_min is (k-1)/infl itself) around that bound and around the threshold
+    (2000; FP32 takes 16 times the value set), and points far past the bound whose smallest
+    eigenvalue is large too: the ones above the threshold get the FP64 solve's bits, the
+    others the plain mixed solve's.  2% off the threshold is 20 times what the mixed
+    Gram (5e-7 of lambda_max) moves lambda_min there."""
+    eff, rng = 2000.0, np.random.default_rng(k)
+    goal = eff * np.array([0.5, 0.74, 0.76, 0.98, 1.02, 1.3, 1.36, 6.0, 0.0, 0.0, 0.0])
+    p = 4 * k
+    q = _problem(k, [1.0] * goal.size, p, k)
+    for b in range(goal.size):
+        sl = slice(b * p, (b + 1) * p)
+        if not goal[b]:  # of full rank: the members' mean is left in
+            q["hd"][sl] = 30.0 * rng.standard_normal((p, k))
+            continue
+        v = rng.standard_normal(k)
+        q["hd"][sl] = np.outer(rng.standard_normal(p), v - v.mean())
+        q["hd"][sl] *= np.sqrt((goal[b] - 1.0) / (_kappa(q, b) - 1.0))
+    kap = np.array([_kappa(q, b) for b in range(q["npt"])])
+    above = kap > eff
+    np.testing.assert_allclose(kap[goal > 0], goal[goal > 0], rtol=1e-6)
+    assert above.sum() == 4 and kap[goal == 0].max() < 0.1 * eff
+
+    def run(prec, value):
+        tune.set("mixed_kappa", value)
+        job, out = _job(q, prec)
+        core.letkf_core_batch([job], prec)
+        sync()
+        return {n: a.numpy() for n, a in out.items()}
+
+    ref, mix, got = run("f64", thr), run(prec, 0), run(prec, thr)
+    np.testing.assert_array_equal((got["status"] & _lib.LEKF_PT_FP64) != 0, above)
+    for n in ("xa", "transm", "infl"):
+        np.testing.assert_array_equal(got[n][above], ref[n][above])
+        np.testing.assert_array_equal(got[n][~above], mix[n][~above])
